@@ -217,6 +217,21 @@ FftArgs fft_args(const dbec_ctx *c, int axis, const Solves &v) {
     return a;
 }
 
+// The x convolution's arguments: where the plane kernels carry the step, the
+// spectrum rows are in their digit order along y.
+FftArgs xconv_args(const dbec_ctx *c, const Solves &v) {
+    FftArgs a = fft_args(c, 0, v);
+    a.yq = c->planes ? (int)(c->Ny / 8) : 0;
+    return a;
+}
+
+int run_xconv(dbec_ctx *c, const Solves &v) {
+    const double spec_b = (double)c->Nkz * c->Nx * c->Ny * (double)(2 * real_elem(c));
+    const double pq = (double)c->Nkz * (c->Nx / 2 + 1) * (c->Ny / 2 + 1) * real_elem(c);
+    HIPCHK(c, timed(c, "xconv", v.nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, xconv_args(c, v)); }), "xconv");
+    return DBEC_OK;
+}
+
 // calcpsidd2 of the context's own psi (no pending scale): |psi|^2 -> half
 // spectrum -> * potdd -> phi, then the face copies.
 int run_calcpsidd2(dbec_ctx *c) {
@@ -224,10 +239,16 @@ int run_calcpsidd2(dbec_ctx *c) {
     const double ce = (double)(2 * real_elem(c));
     const double spec_b = (double)c->Nkz * c->Nx * c->Ny * ce;
     const double nre = (double)c->N * real_elem(c);
+    if (c->planes) {
+        HIPCHK(c, timed(c, "plane_zfwd", (double)c->N * psi_elem(c) + spec_b, [&] { return launch_plane_fwd(c, v, false, true); }), "plane_zfwd");
+        CHK(run_xconv(c, v));
+        HIPCHK(c, timed(c, "plane_phi", spec_b + nre, [&] { return launch_plane_inv(c, v, true); }), "plane_phi");
+        c->phi_valid = true;
+        return DBEC_OK;
+    }
     HIPCHK(c, timed(c, "zfwd", (double)c->N * psi_elem(c) + spec_b, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }), "zfwd");
     HIPCHK(c, timed(c, "ypass_fwd", 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }), "ypass");
-    const double pq = (double)c->Nkz * (c->Nx / 2 + 1) * (c->Ny / 2 + 1) * real_elem(c);
-    HIPCHK(c, timed(c, "xconv", 2 * spec_b + pq, [&] { return launch_xconv(c->Nx, fft_args(c, 0, v)); }), "xconv");
+    CHK(run_xconv(c, v));
     HIPCHK(c, timed(c, "ypass_inv", 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, fft_args(c, 1, v)); }), "ypass");
     HIPCHK(c, timed(c, "zinv", spec_b + nre, [&] { return launch_zinv(c->Nz, fft_args(c, 2, v)); }), "zinv");
     const double fb = 2.0 * (double)(c->Ny * c->Nz + c->Nx * c->Nz + c->Nx * c->Ny) * real_elem(c);
@@ -248,8 +269,7 @@ int run_conv_nu(dbec_ctx *c, const Solves &v, bool z_done) {
     if (!z_done)
         HIPCHK(c, timed(c, "zfwd", nb * ((double)c->N * psi_elem(c) + spec_b), [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }), "zfwd");
     HIPCHK(c, timed(c, "ypass_fwd", nb * 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }), "ypass");
-    const double pq = (double)c->Nkz * (c->Nx / 2 + 1) * (c->Ny / 2 + 1) * real_elem(c);
-    HIPCHK(c, timed(c, "xconv", nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, fft_args(c, 0, v)); }), "xconv");
+    CHK(run_xconv(c, v));
     HIPCHK(c, timed(c, "ypass_inv", nb * 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, fft_args(c, 1, v)); }), "ypass");
     const double nf = (double)(c->Nx + c->Ny - 1);
     HIPCHK(c, timed(c, "zinv_nu", nb * (spec_b + 2.0 * c->N * psi_elem(c) + nf * c->Nkz * 2 * ce),
@@ -276,6 +296,34 @@ bool fuse_z(const dbec_ctx *c) {
     return on && sweepz_zfwd_fusable(c->Nz, c->prec == DBEC_MIXED, c->mode == DBEC_REAL, sweep_z_rows(c));
 }
 
+// Whether a step's end runs fused with the start of the next step.
+bool fuse_steps(const dbec_ctx *c) { return c->planes || fuse_z(c); }
+
+// v.fold of a step whose predecessor ran with fuse_next == fuse_steps(c).
+int fold_next(const dbec_ctx *c) {
+    if (c->mode != DBEC_IMAG) return 0;
+    return c->planes ? 3 : (fuse_z(c) ? 2 : 1);
+}
+
+// Column partials per x that a step leaves (one where the planes carry it).
+int norm_tiles(const dbec_ctx *c) { return c->planes ? 1 : (int)sweep_z_tiles(c); }
+
+// run_step with the plane kernels: the y sweep runs with the z sweep at the
+// end of the step, and both forward passes of the next one with them.
+int run_step_planes(dbec_ctx *c, const Solves &v, bool z_done, bool fuse_next) {
+    const double spec_b = (double)c->Nkz * c->Nx * c->Ny * (double)(2 * real_elem(c));
+    const double psi_b = (double)c->N * psi_elem(c);
+    if (!z_done)
+        HIPCHK(c, timed(c, "plane_zfwd", v.nb * (psi_b + spec_b), [&] { return launch_plane_fwd(c, v, false, true); }), "plane_zfwd");
+    CHK(run_xconv(c, v));
+    HIPCHK(c, timed(c, "plane_nu", v.nb * (spec_b + 2 * psi_b), [&] { return launch_plane_inv(c, v, false); }), "plane_nu");
+    c->phi_valid = false;
+    CHK(run_sweep(c, 0, v, false));
+    HIPCHK(c, timed(c, fuse_next ? "plane_sweep_zfwd" : "plane_sweep", v.nb * (2 * psi_b + (fuse_next ? spec_b : 0.)),
+                    [&] { return launch_plane_fwd(c, v, true, fuse_next); }), "plane_sweep");
+    return DBEC_OK;
+}
+
 // One split step (calcpsidd2, calcnu, calclux/y/z) of the solves v.  In
 // imaginary time the z sweep leaves the Simpson column partials of the new
 // psi: the next step folds the norm in (v.fold), or run_norm computes it.
@@ -285,6 +333,7 @@ bool fuse_z(const dbec_ctx *c) {
 // then has v.fold == 2).
 int run_step(dbec_ctx *c, const Solves &v, bool z_done, bool fuse_next) {
     const bool imag = c->mode == DBEC_IMAG;
+    if (c->planes) return run_step_planes(c, v, z_done, fuse_next);
     CHK(run_conv_nu(c, v, z_done));
     CHK(run_sweep(c, 0, v, false));
     CHK(run_sweep(c, 1, v, false));
@@ -301,8 +350,9 @@ int run_step(dbec_ctx *c, const Solves &v, bool z_done, bool fuse_next) {
 
 // calcnorm from the column partials: scal[NORM], scal[SCALE] = 1/norm.
 int run_norm(dbec_ctx *c, const Solves &v) {
-    HIPCHK(c, timed(c, "norm", v.nb * (double)c->Nx * sweep_z_tiles(c) * 8.0,
-                    [&] { return launch_norm_from_cols(c->stream, c, v); }), "norm");
+    const int tiles = norm_tiles(c);
+    HIPCHK(c, timed(c, "norm", v.nb * (double)c->Nx * tiles * 8.0,
+                    [&] { return launch_norm_from_cols(c->stream, c, v, tiles); }), "norm");
     return DBEC_OK;
 }
 
@@ -483,10 +533,12 @@ int setup(dbec_ctx *c) {
             }
     pq[0] = 0.;
     // device layout [kz][|ky|][|kx|]: rows contiguous in kx for the x convolution
-    std::vector<double> pqd(pq.size());
+    const int yq = c->planes ? (int)(Ny / 8) : 0;
+    const long rows = pot_rows((int)Ny, yq);
+    std::vector<double> pqd(qz * rows * qx, 0.0);
     for (long k = 0; k < qz; k++)
-        for (long i = 0; i < qx; i++)
-            for (long j = 0; j < qy; j++) pqd[(k * qy + j) * qx + i] = pq[(k * qx + i) * qy + j];
+        for (long j = 0; j < qy; j++)
+            for (long i = 0; i < qx; i++) pqd[(k * rows + pot_row((int)j, yq)) * qx + i] = pq[(k * qx + i) * qy + j];
     // host copy of the half table [kx][ky][kz<=Nz/2] for dbec_get_table
     c->h_potdd_half.resize(Nx * Ny * qz);
     for (long i = 0; i < Nx; i++)
@@ -515,7 +567,7 @@ int setup(dbec_ctx *c) {
     CHK(dev_alloc(c, &b.psi, (size_t)c->N * psi_elem(c), "psi"));
     CHK(dev_alloc(c, &b.spec, (size_t)c->Nkz * Nx * Ny * 2 * re, "spectrum"));
     CHK(dev_alloc(c, &b.phi, (size_t)c->N * re, "psidd2"));
-    CHK(dev_alloc(c, &b.potddq, pq.size() * re, "potdd"));
+    CHK(dev_alloc(c, &b.potddq, pqd.size() * re, "potdd"));
     CHK(dev_alloc(c, (void **)&b.rows, (size_t)2 * Nx * Ny * sizeof(double), "row sums"));
     CHK(dev_alloc(c, (void **)&b.scal, SC_COUNT * sizeof(double), "scalars"));
     CHK(dev_alloc(c, (void **)&b.coef, coef.size() * sizeof(double), "CN coefficients"));
@@ -568,9 +620,9 @@ int setup(dbec_ctx *c) {
 // dbec_tuning() returns them as text.
 struct TuneKey {
     long nx, ny, nz;
-    int mode, prec, dev;
+    int mode, prec, dev, planes;
     bool operator<(const TuneKey &o) const {
-        return std::tie(nx, ny, nz, mode, prec, dev) < std::tie(o.nx, o.ny, o.nz, o.mode, o.prec, o.dev);
+        return std::tie(nx, ny, nz, mode, prec, dev, planes) < std::tie(o.nx, o.ny, o.nz, o.mode, o.prec, o.dev, o.planes);
     }
 };
 std::mutex g_tune_mu;
@@ -639,7 +691,7 @@ void describe_tuning(const dbec_ctx *c, char *buf, size_t len) {
 int autotune(dbec_ctx *c) {
     const char *env = getenv("DBEC_AUTOTUNE");
     if (env && std::strcmp(env, "0") == 0) return DBEC_OK;
-    const TuneKey key{c->Nx, c->Ny, c->Nz, (int)c->mode, (int)c->prec, c->device};
+    const TuneKey key{c->Nx, c->Ny, c->Nz, (int)c->mode, (int)c->prec, c->device, (int)c->planes};
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune.find(key);
@@ -657,10 +709,15 @@ int autotune(dbec_ctx *c) {
         return DBEC_OK;
     };
     Tuning &t = c->tune;
-    CHK(choose(&t.lm[0], {0, 1, 2}, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }));
-    CHK(choose(&t.lm[1], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }));
-    CHK(choose(&t.lm[2], {0, 1, 2}, [&] { return launch_xconv(c->Nx, fft_args(c, 0, v)); }));
-    if (c->prec != DBEC_MIXED) {
+    const bool planes = c->planes;  // the plane kernels take the z and y passes' place
+    if (!planes) {
+        CHK(choose(&t.lm[0], {0, 1, 2}, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }));
+        CHK(choose(&t.lm[1], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }));
+    }
+    CHK(choose(&t.lm[2], {0, 1, 2}, [&] { return launch_xconv(c->Nx, xconv_args(c, v)); }));
+    if (planes) {
+        // no fused inverse z pass
+    } else if (c->prec != DBEC_MIXED) {
         // the FP64 fused inverse pass has two buffer layouts: its tile
         // multiplier and layout are chosen together
         const int lms[5] = {0, 1, 2, 1, 2}, sws[5] = {-1, 0, 0, 1, 1};
@@ -708,6 +765,13 @@ const char *dbec_last_error(const dbec_ctx *ctx) {
 }
 
 int dbec_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stream, dbec_ctx **out) {
+    return core_create(p, mode, prec, stream, false, out);
+}
+
+}  // extern "C"
+
+namespace dbec {
+int core_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stream, bool shared, dbec_ctx **out) {
     if (!p || !out) return fail(nullptr, DBEC_EINVAL, "null argument");
     *out = nullptr;
     if (mode != DBEC_IMAG && mode != DBEC_REAL) return fail(nullptr, DBEC_EINVAL, "bad mode");
@@ -742,6 +806,7 @@ int dbec_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stre
     c->N = c->Nx * c->Ny * c->Nz;
     c->Nkz = c->Nz / 2 + 1;
     c->pi = (p->pi != 0.) ? p->pi : 3.14159265358979;
+    c->planes = plane_ok(c, shared);
     if (stream) {
         c->stream = static_cast<hipStream_t>(stream);
     } else {
@@ -765,6 +830,9 @@ int dbec_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stre
     *out = c;
     return DBEC_OK;
 }
+}  // namespace dbec
+
+extern "C" {
 
 int dbec_destroy(dbec_ctx *c) {
     if (!c) return DBEC_OK;
@@ -933,7 +1001,7 @@ int dbec_step(dbec_ctx *c, long nsteps, double g_stp, double gd_stp, double *nor
     if (!c || nsteps < 0) return fail(c, DBEC_EINVAL, "bad argument");
     (void)hipSetDevice(c->device);
     const bool imag = c->mode == DBEC_IMAG;
-    const bool fuse = fuse_z(c);
+    const bool fuse = fuse_steps(c);
     bool z_done = false;
     for (long s = 0; s < nsteps; s++) {
         if (g_stp != 0. || gd_stp != 0.) {
@@ -942,7 +1010,7 @@ int dbec_step(dbec_ctx *c, long nsteps, double g_stp, double gd_stp, double *nor
         }
         // after the first step the previous norm is folded into this one
         Solves v = solve_ref(c, imag && (c->scale_pending || s > 0));
-        v.fold = (imag && s > 0) ? (z_done ? 2 : 1) : 0;
+        v.fold = s > 0 ? fold_next(c) : 0;
         const bool fuse_next = fuse && s + 1 < nsteps;
         CHK(run_step(c, v, z_done, fuse_next));
         z_done = fuse_next;
@@ -1253,7 +1321,8 @@ Solves core_solves(const dbec_ctx *c, bool use_scale) { return solve_ref(c, use_
 int core_step(dbec_ctx *c, const Solves &v, bool z_done, bool fuse_next) {
     return run_step(c, v, z_done, fuse_next);
 }
-bool core_fuse_z(const dbec_ctx *c) { return fuse_z(c); }
+bool core_fuse(const dbec_ctx *c) { return fuse_steps(c); }
+int core_fold(const dbec_ctx *c) { return fold_next(c); }
 
 int core_norm(dbec_ctx *c, const Solves &v) { return run_norm(c, v); }
 

@@ -444,9 +444,13 @@ k_ypass(Solves v, long nlines, const cpx<R> *__restrict__ twg, const double *__r
 }
 
 // ---------------------------------------------------------------------------
-template <int N, typename R, int LM>
+// PL: the spectrum's rows come from the plane kernels (digit order along y,
+// yq = Ny / 8; the norm from one partial per x with v.fold == 3); a template
+// parameter, so the other grids' kernel stays as lean as without it.
+template <int N, typename R, int LM, bool PL>
 __global__ void __launch_bounds__((FftTile<N, LM>::WG))
-k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict__ twg) {
+k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict__ twg, const double *__restrict__ wx,
+        int yq) {
     constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
     constexpr int T = FftPlan<N>::T, K = N / T;  // x values per thread
     static_assert(L * T == WG, "xconv tile");
@@ -456,7 +460,7 @@ k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict
     const SolveAt sr = solve_at(v);
     cpx<R> *__restrict__ spec = reinterpret_cast<cpx<R> *>(sr.spec);
     // folded norm: |psi|^2 was transformed unscaled, so potdd takes 1/norm^2
-    const R s2 = v.fold ? (R)(sr.scal[SC_SCALE] * sr.scal[SC_SCALE]) : R(1);
+    R s2 = (!PL && v.fold) ? (R)(sr.scal[SC_SCALE] * sr.scal[SC_SCALE]) : R(1);
     const int tid = threadIdx.x;
     const int ytiles = (Ny + L - 1) / L;
     const int kz = blockIdx.x / ytiles;
@@ -480,13 +484,21 @@ k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict
 #pragma unroll
     for (int k = 0; k < K; ++k) r[k] = g[(unsigned)((t + k * T) * Ny)];
     // potdd(|kx|, |ky|, kz): the table rows [kz][|ky|] are contiguous in |kx|
-    const int Ny2 = Ny / 2, Nyh = Ny2 + 1;
-    const R *pk = potddq + ((long)kz * Nyh + (y <= Ny2 ? y : Ny - y)) * NXH;
+    const int Ny2 = Ny / 2;
+    const int ky = PL ? y / yq + 8 * (y % yq) : y, ka = ky <= Ny2 ? ky : Ny - ky;
+    const R *pk = potddq + ((long)kz * pot_rows(Ny, PL ? yq : 0) + pot_row(ka, PL ? yq : 0)) * NXH;
     R pw[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int e = t + k * T;
         pw[k] = pk[e <= N / 2 ? e : N - e];
+    }
+    if (PL && v.fold) {  // one partial per x: every workgroup forms the norm, the first one stores it
+        static_assert(sizeof(buf) >= WG * sizeof(double), "norm scratch");
+        const double sc = norm_from_cols<WG>(sr.rows, 1, wx, N, sr.scal, v.shift, reinterpret_cast<double *>(buf),
+                                             blockIdx.x == 0);
+        s2 = (R)(sc * sc);
+        __syncthreads();  // the scratch becomes the transform buffer
     }
     FftPlan<N>::template run_reg<-1, L>(buf, l, t, tw, r);
 #pragma unroll
@@ -863,12 +875,17 @@ struct FftLaunchImpl {
         using Tl = FftTile<N, LM>;
         const int ytiles = (int)((a.Ny + Tl::L - 1) / Tl::L);
         dim3 grid((unsigned)(a.Nkz * ytiles), (unsigned)a.v.nb), block(Tl::WG);
-        if (!a.fp32)
-            k_xconv<N, double, LM><<<grid, block, 0, a.stream>>>(a.v, static_cast<const double *>(a.potddq),
-                                                                 (int)a.Ny, static_cast<const cpx<double> *>(a.tw));
-        else
-            k_xconv<N, float, LM><<<grid, block, 0, a.stream>>>(a.v, static_cast<const float *>(a.potddq),
-                                                                (int)a.Ny, static_cast<const cpx<float> *>(a.tw));
+        const auto launch = [&](auto planes) {
+            constexpr bool PL = decltype(planes)::value;
+            if (!a.fp32)
+                k_xconv<N, double, LM, PL><<<grid, block, 0, a.stream>>>(
+                    a.v, static_cast<const double *>(a.potddq), (int)a.Ny, static_cast<const cpx<double> *>(a.tw), a.wx, a.yq);
+            else
+                k_xconv<N, float, LM, PL><<<grid, block, 0, a.stream>>>(
+                    a.v, static_cast<const float *>(a.potddq), (int)a.Ny, static_cast<const cpx<float> *>(a.tw), a.wx, a.yq);
+        };
+        if (a.yq) launch(std::true_type{});
+        else launch(std::false_type{});
         return hipGetLastError();
     }
     static hipError_t xconv(const FftArgs &a) {

@@ -22,7 +22,8 @@ namespace dbec {
 //   phi    [x][y][z]        real: unnormalised dipolar potential (psidd2)
 //   potddq [kz][ky][kx]     real, kz <= Nz/2, kx <= Nx/2, ky <= Ny/2: the
 //                           dipolar kernel is even in every k component, so a
-//                           quarter table indexed by |k| holds it exactly
+//                           quarter table indexed by |k| holds it exactly;
+//                           rows ky in the order of pot_row
 //   rows   [2][Ny][Nx]      double: per-row z integrals for the reductions
 struct Buffers {
     void *psi = nullptr;
@@ -78,6 +79,7 @@ struct dbec_ctx {
     std::vector<double> h_potdd_half;              // [kx][ky][kz<=Nz/2], for dbec_get_table
     bool scale_pending = false;  // psi must be multiplied by scal[SC_SCALE]
     bool view = false;           // buffers belong to another owner (request-loop slot)
+    bool planes = false;         // the plane kernels carry the step (plane_ok at creation)
     bool phi_valid = false;
     dbec::Buffers b;
     dbec::Tuning tune;
@@ -86,6 +88,14 @@ struct dbec_ctx {
 };
 
 namespace dbec {
+
+// The rows |ky| of one kz in potddq: in order, or (yq = Ny / 8 > 0, the plane
+// kernels' digit order) row (|ky| & 7) (yq/2 + 1) + |ky| / 8, so that the lanes
+// of the x convolution, which hold y frequencies 8 apart there, read adjacent
+// rows; rows 8 apart (2080 bytes at 128 FP32) crowd two L2 channels: xconv of 16
+// solves at 128^3 mixed 69 us against 46.
+__host__ __device__ inline int pot_rows(int Ny, int yq) { return yq ? 8 * (yq / 2 + 1) : Ny / 2 + 1; }
+__host__ __device__ inline int pot_row(int ka, int yq) { return yq ? (ka & 7) * (yq / 2 + 1) + (ka >> 3) : ka; }
 
 // ---- The solves of a launch ----------------------------------------------
 // The step kernels advance nb solves of one grid at once: gridDim.y = nb and
@@ -113,7 +123,8 @@ struct Solves {
     int shift;                // calcnu multiplies by exp(scal[SC_SHIFT]) too (mixed imaginary time)
     int fold;                 // the last step's norm is still in the column partials: the forward z
                               // pass computes it (workgroup 0 of each solve), reads psi unscaled, and
-                              // the x convolution applies 1/norm^2 (the transform is linear)
+                              // the x convolution applies 1/norm^2 (the transform is linear); 3: the
+                              // partials are one per x plane and the x convolution forms the norm itself
 };
 
 struct SolveAt {
@@ -156,6 +167,9 @@ struct FftArgs {
     double zk[3][2];
     const double *wz, *wy;
     int zrows;
+    // x convolution: > 0 where slot s of a spectrum row holds the y frequency
+    // s / yq + 8 (s % yq) (the plane kernels' digit order), 0: s itself
+    int yq = 0;
 };
 // Each returns hipSuccess or an error; `n` is the transformed length.
 hipError_t launch_zfwd(long n, const FftArgs &a);    // |psi|^2 -> spec (R2C along z)

@@ -14,10 +14,12 @@ namespace dbec {
 // c of the mixed form, scal[SHIFT] = c - log(norm): psi carried an extra
 // factor exp(c), so the reference's norm is norm * exp(-c), and the new shift
 // brings the next step's norm to about 1 (c follows dt * mu).
+// Returns 1/norm in every thread; `write` false: scal is left alone (every
+// workgroup of a launch may form the norm, one of them stores it).
 template <int NT>
-__device__ __forceinline__ void norm_from_cols(const double *__restrict__ rows, int tiles,
-                                               const double *__restrict__ wx, int Nx, double *__restrict__ scal,
-                                               int shift, double *sh) {
+__device__ __forceinline__ double norm_from_cols(const double *__restrict__ rows, int tiles,
+                                                 const double *__restrict__ wx, int Nx, double *__restrict__ scal,
+                                                 int shift, double *sh, bool write = true) {
     const int tid = threadIdx.x;
     double p = 0.0;
     for (int x = tid; x < Nx; x += NT) {
@@ -32,8 +34,8 @@ __device__ __forceinline__ void norm_from_cols(const double *__restrict__ rows, 
         if (tid < o && tid + o < NT) sh[tid] += sh[tid + o];
         __syncthreads();
     }
-    if (tid == 0) {
-        const double norm = sqrt(sh[0]);
+    const double norm = sqrt(sh[0]);
+    if (write && tid == 0) {
         if (shift) {
             const double c = scal[SC_SHIFT];
             scal[SC_NORM] = norm * exp(-c);
@@ -44,6 +46,7 @@ __device__ __forceinline__ void norm_from_cols(const double *__restrict__ rows, 
         scal[SC_SCALE] = 1.0 / norm;
         scal[SC_LASTNORM] = scal[SC_NORM];
     }
+    return 1.0 / norm;
 }
 
 }  // namespace dbec

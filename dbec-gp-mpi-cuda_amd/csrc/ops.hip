@@ -395,20 +395,29 @@ int sweep_z_rows(const dbec_ctx *c) {
     return f32 ? z_rows<cpx<float>>(c->Nz) : z_rows<cpx<double>>(c->Nz);
 }
 
-void sweep_z_args(const dbec_ctx *c, FftArgs &a) {
+AxisArgs sweep_axis_args(const dbec_ctx *c, int axis) {
     const CoefLayout lay(c->Nx, c->Ny, c->Nz);
     const bool cplx = c->mode == DBEC_REAL;
     const size_t el = sizeof(double) * (cplx ? 2 : 1);  // FP64 tables in every precision
     const char *base = reinterpret_cast<const char *>(c->b.coef);
-    a.ztab[0] = base + el * lay.ca(2);
-    a.ztab[1] = base + el * lay.cg(2);
-    a.ztab[2] = base + el * lay.gb(2, 0);
-    a.ztab[3] = base + el * lay.fa(2, 0);
+    AxisArgs a;
+    a.tab[0] = base + el * lay.ca(axis);
+    a.tab[1] = base + el * lay.cg(axis);
+    a.tab[2] = base + el * lay.gb(axis, 0);
+    a.tab[3] = base + el * lay.fa(axis, 0);
     for (int q = 0; q < 2; q++) {
-        a.zk[0][q] = c->A0r[2][q];
-        a.zk[1][q] = c->A[2][q];
-        a.zk[2][q] = c->mA[2][q];
+        a.k[0][q] = c->A0r[axis][q];
+        a.k[1][q] = c->A[axis][q];
+        a.k[2][q] = c->mA[axis][q];
     }
+    return a;
+}
+
+void sweep_z_args(const dbec_ctx *c, FftArgs &a) {
+    const AxisArgs z = sweep_axis_args(c, 2);
+    for (int i = 0; i < 4; i++) a.ztab[i] = z.tab[i];
+    for (int i = 0; i < 3; i++)
+        for (int q = 0; q < 2; q++) a.zk[i][q] = z.k[i][q];
     a.wz = c->b.wgt + c->Nx + c->Ny;
     a.wy = c->b.wgt + c->Nx;
     a.zrows = sweep_z_rows(c);
@@ -594,8 +603,8 @@ k_norm_cols(Solves v, int tiles, const double *__restrict__ wx, int Nx) {
     norm_from_cols<256>(sr.rows, tiles, wx, Nx, sr.scal, v.shift, sh);
 }
 
-hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves &v) {
-    k_norm_cols<<<dim3(1, (unsigned)v.nb), 256, 0, s>>>(v, (int)sweep_z_tiles(c), c->b.wgt, (int)c->Nx);
+hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves &v, int tiles) {
+    k_norm_cols<<<dim3(1, (unsigned)v.nb), 256, 0, s>>>(v, tiles, c->b.wgt, (int)c->Nx);
     return hipGetLastError();
 }
 

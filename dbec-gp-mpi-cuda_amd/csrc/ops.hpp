@@ -49,8 +49,23 @@ int sweep_z_rows(const dbec_ctx *c);
 // The z sweep's tables, constants, weights and rows per workgroup for the
 // z sweep fused with the forward z pass.
 void sweep_z_args(const dbec_ctx *c, FftArgs &a);
-// norm of each solve from its column partials: scal[NORM], scal[SCALE]
-hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves &v);
+// One axis' sweep tables (calpha, cgamma, gb, fa for segments of 16; FP64 in
+// every precision) and constants A0r, A, mA (re, im).
+struct AxisArgs {
+    const void *tab[4];
+    double k[3][2];
+};
+AxisArgs sweep_axis_args(const dbec_ctx *c, int axis);
+// The plane kernels (plane.hip): whether they are to carry the context's step
+// (dbec_ctx::planes), the y and z sweeps and the next step's forward z and y passes (either or both),
+// and the inverse y and z passes with calcnu (or writing phi).
+// shared: the context's launches advance several solves and run beside other
+// contexts' (the request loop).
+bool plane_ok(const dbec_ctx *c, bool shared);
+hipError_t launch_plane_fwd(const dbec_ctx *c, const Solves &v, bool sweeps, bool fft);
+hipError_t launch_plane_inv(const dbec_ctx *c, const Solves &v, bool phi);
+// norm of each solve from its column partials (`tiles` per x): scal[NORM], scal[SCALE]
+hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves &v, int tiles);
 TrapConst trap_const(const dbec_ctx *c);
 NuConst nu_const(const dbec_ctx *c);
 hipError_t launch_rows_mod2(hipStream_t s, const dbec_ctx *c, double *rows0, double *rowsz);

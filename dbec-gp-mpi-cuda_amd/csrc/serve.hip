@@ -210,7 +210,7 @@ struct dbec_server {
         b->key = r;
         b->cap = cfg.max_batch;
         const dbec_params p = params_of(r, device);
-        int rc = dbec_create(&p, (dbec_mode)r.mode, (dbec_prec)r.prec, nullptr, &b->tab);
+        int rc = core_create(&p, (dbec_mode)r.mode, (dbec_prec)r.prec, nullptr, true, &b->tab);
         if (rc != DBEC_OK) {
             err = dbec_last_error(nullptr);
             return rc;
@@ -261,6 +261,7 @@ struct dbec_server {
             std::memcpy(v->A, t->A, sizeof v->A);
             std::memcpy(v->mA, t->mA, sizeof v->mA);
             v->tune = t->tune;
+            v->planes = t->planes;
             v->b = t->b;  // tables, phi and reduction scratch of the bucket
             v->b.psi = b->psi + (size_t)s * b->psi_st;
             v->b.spec = b->spec + (size_t)s * b->spec_st;
@@ -422,11 +423,10 @@ struct dbec_server {
         v.use_scale = imag ? 1 : 0;
         v.shift = (imag && t->prec == DBEC_MIXED) ? 1 : 0;
         v.fold = 0;
-        // steps after the first fold the previous norm in; with the z sweep
-        // fused into the next forward z pass, the y pass forms that norm
-        const bool fuse = core_fuse_z(t);
+        // steps after the first fold the previous norm in
+        const bool fuse = core_fuse(t);
         Solves vf = v;
-        vf.fold = imag ? (fuse ? 2 : 1) : 0;
+        vf.fold = core_fold(t);
         static const bool use_graphs = [] {
             const char *e = getenv("DBEC_SERVE_GRAPHS");
             return !e || atoi(e) != 0;
