@@ -217,18 +217,24 @@ FftArgs fft_args(const dbec_ctx *c, int axis, const Solves &v) {
     return a;
 }
 
-// The x convolution's arguments: where the plane kernels carry the step, the
-// spectrum rows are in their digit order along y.
-FftArgs xconv_args(const dbec_ctx *c, const Solves &v) {
+// The x convolution's arguments; planes: the spectrum rows are in the plane
+// kernels' digit order along y.
+FftArgs xconv_args(const dbec_ctx *c, const Solves &v, bool planes) {
     FftArgs a = fft_args(c, 0, v);
-    a.yq = c->planes ? (int)(c->Ny / 8) : 0;
+    a.yq = planes ? (int)(c->Ny / 8) : 0;
     return a;
 }
 
-int run_xconv(dbec_ctx *c, const Solves &v) {
+// Whether the standalone calcpsidd2 runs on the plane kernels too: in FP64.
+// The mixed form keeps the passes of the larger grids for it, so that phi of a
+// given FP32 psi, and with it mu and E, keep their rounding (planes in FP32 move
+// mu of a 48^3 state by 6e-10 of its value).
+bool phi_planes(const dbec_ctx *c) { return c->planes && c->prec == DBEC_FP64; }
+
+int run_xconv(dbec_ctx *c, const Solves &v, bool planes) {
     const double spec_b = (double)c->Nkz * c->Nx * c->Ny * (double)(2 * real_elem(c));
     const double pq = (double)c->Nkz * (c->Nx / 2 + 1) * (c->Ny / 2 + 1) * real_elem(c);
-    HIPCHK(c, timed(c, "xconv", v.nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, xconv_args(c, v)); }), "xconv");
+    HIPCHK(c, timed(c, "xconv", v.nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, xconv_args(c, v, planes)); }), "xconv");
     return DBEC_OK;
 }
 
@@ -239,16 +245,16 @@ int run_calcpsidd2(dbec_ctx *c) {
     const double ce = (double)(2 * real_elem(c));
     const double spec_b = (double)c->Nkz * c->Nx * c->Ny * ce;
     const double nre = (double)c->N * real_elem(c);
-    if (c->planes) {
+    if (phi_planes(c)) {
         HIPCHK(c, timed(c, "plane_zfwd", (double)c->N * psi_elem(c) + spec_b, [&] { return launch_plane_fwd(c, v, false, true); }), "plane_zfwd");
-        CHK(run_xconv(c, v));
+        CHK(run_xconv(c, v, true));
         HIPCHK(c, timed(c, "plane_phi", spec_b + nre, [&] { return launch_plane_inv(c, v, true); }), "plane_phi");
         c->phi_valid = true;
         return DBEC_OK;
     }
     HIPCHK(c, timed(c, "zfwd", (double)c->N * psi_elem(c) + spec_b, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }), "zfwd");
     HIPCHK(c, timed(c, "ypass_fwd", 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }), "ypass");
-    CHK(run_xconv(c, v));
+    CHK(run_xconv(c, v, false));
     HIPCHK(c, timed(c, "ypass_inv", 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, fft_args(c, 1, v)); }), "ypass");
     HIPCHK(c, timed(c, "zinv", spec_b + nre, [&] { return launch_zinv(c->Nz, fft_args(c, 2, v)); }), "zinv");
     const double fb = 2.0 * (double)(c->Ny * c->Nz + c->Nx * c->Nz + c->Nx * c->Ny) * real_elem(c);
@@ -269,7 +275,7 @@ int run_conv_nu(dbec_ctx *c, const Solves &v, bool z_done) {
     if (!z_done)
         HIPCHK(c, timed(c, "zfwd", nb * ((double)c->N * psi_elem(c) + spec_b), [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }), "zfwd");
     HIPCHK(c, timed(c, "ypass_fwd", nb * 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }), "ypass");
-    CHK(run_xconv(c, v));
+    CHK(run_xconv(c, v, false));
     HIPCHK(c, timed(c, "ypass_inv", nb * 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, fft_args(c, 1, v)); }), "ypass");
     const double nf = (double)(c->Nx + c->Ny - 1);
     HIPCHK(c, timed(c, "zinv_nu", nb * (spec_b + 2.0 * c->N * psi_elem(c) + nf * c->Nkz * 2 * ce),
@@ -315,7 +321,7 @@ int run_step_planes(dbec_ctx *c, const Solves &v, bool z_done, bool fuse_next) {
     const double psi_b = (double)c->N * psi_elem(c);
     if (!z_done)
         HIPCHK(c, timed(c, "plane_zfwd", v.nb * (psi_b + spec_b), [&] { return launch_plane_fwd(c, v, false, true); }), "plane_zfwd");
-    CHK(run_xconv(c, v));
+    CHK(run_xconv(c, v, true));
     HIPCHK(c, timed(c, "plane_nu", v.nb * (spec_b + 2 * psi_b), [&] { return launch_plane_inv(c, v, false); }), "plane_nu");
     c->phi_valid = false;
     CHK(run_sweep(c, 0, v, false));
@@ -362,9 +368,11 @@ int run_calcnu(dbec_ctx *c, const double *scale) {
     return DBEC_OK;
 }
 
+// Waits for the stream and reads scalars from the pinned host copy, which the
+// last launch wrote.
 int read_scalars(dbec_ctx *c, double *dst, int first, int count) {
-    HIPCHK(c, hipMemcpyAsync(dst, c->b.scal + first, sizeof(double) * count, hipMemcpyDeviceToHost, c->stream), "copy scalars");
     HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
+    for (int i = 0; i < count; i++) dst[i] = c->h_scal[first + i];
     return DBEC_OK;
 }
 
@@ -415,6 +423,8 @@ void free_buffers(dbec_ctx *c) {
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     b = Buffers();
+    if (c->h_scal) (void)hipHostFree(c->h_scal);
+    c->h_scal = nullptr;
 }
 
 int dev_alloc(dbec_ctx *c, void **p, size_t bytes, const char *what) {
@@ -533,7 +543,7 @@ int setup(dbec_ctx *c) {
             }
     pq[0] = 0.;
     // device layout [kz][|ky|][|kx|]: rows contiguous in kx for the x convolution
-    const int yq = c->planes ? (int)(Ny / 8) : 0;
+    const int yq = c->planes && (f32 ? pot_digit_rows<float>() : pot_digit_rows<double>()) ? (int)(Ny / 8) : 0;
     const long rows = pot_rows((int)Ny, yq);
     std::vector<double> pqd(qz * rows * qx, 0.0);
     for (long k = 0; k < qz; k++)
@@ -710,11 +720,11 @@ int autotune(dbec_ctx *c) {
     };
     Tuning &t = c->tune;
     const bool planes = c->planes;  // the plane kernels take the z and y passes' place
-    if (!planes) {
+    if (!phi_planes(c)) {
         CHK(choose(&t.lm[0], {0, 1, 2}, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }));
         CHK(choose(&t.lm[1], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }));
     }
-    CHK(choose(&t.lm[2], {0, 1, 2}, [&] { return launch_xconv(c->Nx, xconv_args(c, v)); }));
+    CHK(choose(&t.lm[2], {0, 1, 2}, [&] { return launch_xconv(c->Nx, xconv_args(c, v, planes)); }));
     if (planes) {
         // no fused inverse z pass
     } else if (c->prec != DBEC_MIXED) {
@@ -818,6 +828,13 @@ int core_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stre
         c->own_stream = true;
     }
     int rc = setup(c);
+    if (rc == DBEC_OK && !shared) {
+        e = hipHostMalloc((void **)&c->h_scal, (SC_COUNT + 2) * sizeof(double), 0);
+        if (e != hipSuccess) {
+            c->h_scal = nullptr;
+            rc = fail(c, DBEC_ENOMEM, std::string("pinned host scalars: ") + hipGetErrorString(e));
+        }
+    }
     if (rc == DBEC_OK) rc = autotune(c);
     if (rc != DBEC_OK) {
         std::string m = c->err;
@@ -935,8 +952,7 @@ int dbec_calcnorm(dbec_ctx *c, double *norm, int rescale) {
     if (!c) return fail(c, DBEC_EINVAL, "null context");
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
-    HIPCHK(c, launch_rows_mod2(c->stream, c, c->b.rows, nullptr), "rows");
-    HIPCHK(c, launch_finalize(c->stream, c, 0, c->b.rows, nullptr), "finalize");
+    HIPCHK(c, launch_obs_norm(c->stream, c, false), "norm");
     if (rescale) HIPCHK(c, launch_scale(c->stream, c, c->b.scal + SC_SCALE), "scale");
     double v;
     CHK(read_scalars(c, &v, SC_NORM, 1));
@@ -949,9 +965,7 @@ static int calcmuen_api(dbec_ctx *c, double *mu, double *en, bool phase) {
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
     CHK(run_calcpsidd2(c));
-    double *rmu = c->b.rows, *ren = c->b.rows + c->Nx * c->Ny;
-    HIPCHK(c, launch_rows_muen(c->stream, c, rmu, ren, phase), "muen rows");
-    HIPCHK(c, launch_finalize(c->stream, c, 2, rmu, ren), "finalize");
+    HIPCHK(c, launch_obs_muen(c->stream, c, phase), "muen");
     double v[2];
     CHK(read_scalars(c, v, SC_MU, 2));
     *mu = v[0];
@@ -966,9 +980,7 @@ int dbec_calcrms(dbec_ctx *c, double rms[4]) {
     if (!c || !rms) return fail(c, DBEC_EINVAL, "null argument");
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
-    double *r0 = c->b.rows, *rz = c->b.rows + c->Nx * c->Ny;
-    HIPCHK(c, launch_rows_mod2(c->stream, c, r0, rz), "rms rows");
-    HIPCHK(c, launch_finalize(c->stream, c, 1, r0, rz), "finalize");
+    HIPCHK(c, launch_obs_norm(c->stream, c, true), "rms");
     double v[4];
     CHK(read_scalars(c, v, SC_R0, 4));
     for (int i = 0; i < 4; i++) rms[i] = v[i];
@@ -980,20 +992,8 @@ int dbec_psi_center(dbec_ctx *c, double out[2]) {
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
     const long n = ((c->Nx / 2) * c->Ny + c->Ny / 2) * c->Nz + c->Nz / 2;
-    const size_t el = psi_elem(c);
-    unsigned char buf[16];
-    HIPCHK(c, hipMemcpyAsync(buf, static_cast<char *>(c->b.psi) + n * el, el, hipMemcpyDeviceToHost, c->stream), "copy");
-    HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
-    double v[2] = {0., 0.};
-    if (c->prec == DBEC_FP64) std::memcpy(v, buf, el);
-    else {
-        float f[2] = {0.f, 0.f};
-        std::memcpy(f, buf, el);
-        v[0] = f[0];
-        v[1] = f[1];
-    }
-    out[0] = v[0];
-    out[1] = (c->mode == DBEC_REAL) ? v[1] : 0.;
+    HIPCHK(c, launch_export_point(c->stream, c, n), "psi centre");
+    CHK(read_scalars(c, out, SC_COUNT, 2));
     return DBEC_OK;
 }
 
@@ -1021,6 +1021,7 @@ int dbec_step(dbec_ctx *c, long nsteps, double g_stp, double gd_stp, double *nor
     }
     if (imag && nsteps > 0 && norm) {
         CHK(materialize_scale(c));
+        HIPCHK(c, launch_export_scalars(c->stream, c), "scalars");
         CHK(read_scalars(c, norm, SC_NORM, 1));
     }
     return DBEC_OK;
@@ -1331,16 +1332,11 @@ int core_observe_async(dbec_ctx *c, int what) {
         HIPCHK(c, launch_scale(c->stream, c, c->b.scal + SC_SCALE), "scale");
         HIPCHK(c, launch_set_scalar(c->stream, c->b.scal + SC_SCALE, 1.0), "scalar");
     }
-    double *r0 = c->b.rows, *r1 = c->b.rows + c->Nx * c->Ny;
     if (what & OBS_MUEN) {
         CHK(run_calcpsidd2(c));
-        HIPCHK(c, launch_rows_muen(c->stream, c, r0, r1), "muen rows");
-        HIPCHK(c, launch_finalize(c->stream, c, 2, r0, r1), "finalize");
+        HIPCHK(c, launch_obs_muen(c->stream, c, false), "muen");
     }
-    if (what & OBS_RMS) {
-        HIPCHK(c, launch_rows_mod2(c->stream, c, r0, r1), "rms rows");
-        HIPCHK(c, launch_finalize(c->stream, c, 1, r0, r1), "finalize");
-    }
+    if (what & OBS_RMS) HIPCHK(c, launch_obs_norm(c->stream, c, true), "rms");
     return DBEC_OK;
 }
 

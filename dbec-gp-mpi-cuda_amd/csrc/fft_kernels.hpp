@@ -486,7 +486,8 @@ k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict
     // potdd(|kx|, |ky|, kz): the table rows [kz][|ky|] are contiguous in |kx|
     const int Ny2 = Ny / 2;
     const int ky = PL ? y / yq + 8 * (y % yq) : y, ka = ky <= Ny2 ? ky : Ny - ky;
-    const R *pk = potddq + ((long)kz * pot_rows(Ny, PL ? yq : 0) + pot_row(ka, PL ? yq : 0)) * NXH;
+    const int tq = PL && pot_digit_rows<R>() ? yq : 0;
+    const R *pk = potddq + ((long)kz * pot_rows(Ny, tq) + pot_row(ka, tq)) * NXH;
     R pw[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {

@@ -79,6 +79,7 @@ struct dbec_ctx {
     std::vector<double> h_potdd_half;              // [kx][ky][kz<=Nz/2], for dbec_get_table
     bool scale_pending = false;  // psi must be multiplied by scal[SC_SCALE]
     bool view = false;           // buffers belong to another owner (request-loop slot)
+    double *h_scal = nullptr;    // pinned host copy of the scalars (SC_COUNT + 2), null in request-loop contexts
     bool planes = false;         // the plane kernels carry the step (plane_ok at creation)
     bool phi_valid = false;
     dbec::Buffers b;
@@ -92,8 +93,11 @@ namespace dbec {
 // The rows |ky| of one kz in potddq: in order, or (yq = Ny / 8 > 0, the plane
 // kernels' digit order) row (|ky| & 7) (yq/2 + 1) + |ky| / 8, so that the lanes
 // of the x convolution, which hold y frequencies 8 apart there, read adjacent
-// rows; rows 8 apart (2080 bytes at 128 FP32) crowd two L2 channels: xconv of 16
-// solves at 128^3 mixed 69 us against 46.
+// rows: rows 8 apart (4160 bytes at 128 FP64) crowd two L2 channels.  FP64 tables
+// only: a mixed context also convolves with the spectrum in natural order (its
+// standalone calcpsidd2), and its rows are half as far apart.
+template <typename R>
+__host__ __device__ constexpr bool pot_digit_rows() { return sizeof(R) == 8; }
 __host__ __device__ inline int pot_rows(int Ny, int yq) { return yq ? 8 * (yq / 2 + 1) : Ny / 2 + 1; }
 __host__ __device__ inline int pot_row(int ka, int yq) { return yq ? (ka & 7) * (yq / 2 + 1) + (ka >> 3) : ka; }
 

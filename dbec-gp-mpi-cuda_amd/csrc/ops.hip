@@ -609,13 +609,6 @@ hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves 
 }
 
 // ---------------------------------------------------------------------------
-// Reductions.  Every integral is the Simpson sum of the reference
-// (diffint.cu:37-51), written as weights w[i] (h/3 times 1,4,2,...,4,1 plus the
-// even-N end correction) so that integral = sum_x wx sum_y wy sum_z wz f.
-// Rows are summed by one wavefront each (lane-strided, then a fixed
-// shuffle tree), columns and the total by fixed-order loops and a fixed LDS
-// tree: the result is reproducible bit for bit from run to run.
-
 __device__ __forceinline__ double mod2_of(double v) { return v * v; }
 __device__ __forceinline__ double mod2_of(float v) { return (double)v * (double)v; }
 __device__ __forceinline__ double mod2_of(cpx<double> v) {
@@ -626,254 +619,6 @@ __device__ __forceinline__ double mod2_of(cpx<float> v) {
     double a = hypot((double)v.x, (double)v.y);
     return a * a;
 }
-__device__ __forceinline__ double amp_of(double v) { return v; }
-__device__ __forceinline__ double amp_of(float v) { return (double)v; }
-__device__ __forceinline__ double amp_of(cpx<double> v) { return hypot(v.x, v.y); }
-__device__ __forceinline__ double amp_of(cpx<float> v) { return hypot((double)v.x, (double)v.y); }
-
-// rows0[y][x] = sum_z wz |psi|^2 ; rowsz[y][x] = sum_z wz z^2 |psi|^2
-template <typename P>
-__global__ void __launch_bounds__(256)
-k_rows_mod2(const P *__restrict__ psi, const double *__restrict__ wz, const double *__restrict__ z2,
-            double *__restrict__ rows0, double *__restrict__ rowsz, int Nx, int Ny, int Nz) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * 4 + wave;
-    if (row >= (long)Nx * Ny) return;
-    const P *r = psi + row * Nz;
-    double a0 = 0.0, az = 0.0;
-    for (int k = lane; k < Nz; k += 64) {
-        const double m = mod2_of(r[k]) * wz[k];
-        a0 += m;
-        az += m * z2[k];
-    }
-    a0 = wave_sum(a0);
-    az = wave_sum(az);
-    if (lane == 0) {
-        const int x = (int)(row / Ny), y = (int)(row % Ny);
-        rows0[(long)y * Nx + x] = a0;
-        if (rowsz) rowsz[(long)y * Nx + x] = az;
-    }
-}
-
-hipError_t launch_rows_mod2(hipStream_t s, const dbec_ctx *c, double *rows0, double *rowsz) {
-    const auto &b = c->b;
-    const double *wz = b.wgt + c->Nx + c->Ny, *z2 = b.sq + c->Nx + c->Ny;
-    dim3 block(256), grid((unsigned)((c->Nx * c->Ny + 3) / 4));
-    const int Nx = (int)c->Nx, Ny = (int)c->Ny, Nz = (int)c->Nz;
-    const bool f32 = c->prec == DBEC_MIXED;
-    if (c->mode == DBEC_IMAG) {
-        if (f32) k_rows_mod2<float><<<grid, block, 0, s>>>(static_cast<const float *>(b.psi), wz, z2, rows0, rowsz, Nx, Ny, Nz);
-        else k_rows_mod2<double><<<grid, block, 0, s>>>(static_cast<const double *>(b.psi), wz, z2, rows0, rowsz, Nx, Ny, Nz);
-    } else {
-        if (f32)
-            k_rows_mod2<cpx<float>><<<grid, block, 0, s>>>(static_cast<const cpx<float> *>(b.psi), wz, z2, rows0, rowsz, Nx, Ny, Nz);
-        else
-            k_rows_mod2<cpx<double>><<<grid, block, 0, s>>>(static_cast<const cpx<double> *>(b.psi), wz, z2, rows0, rowsz, Nx, Ny, Nz);
-    }
-    return hipGetLastError();
-}
-
-// Components a derivative is taken of: |psi| (the reference's calcmuen), or
-// the real or imaginary part (the phase-gradient energy of real time).
-enum { COMP_AMP = 0, COMP_RE = 1, COMP_IM = 2 };
-template <int C> __device__ __forceinline__ double comp_of(double v) { return v; }
-template <int C> __device__ __forceinline__ double comp_of(float v) { return (double)v; }
-template <int C> __device__ __forceinline__ double comp_of(cpx<double> v) {
-    return C == COMP_RE ? v.x : (C == COMP_IM ? v.y : amp_of(v));
-}
-template <int C> __device__ __forceinline__ double comp_of(cpx<float> v) {
-    return C == COMP_RE ? (double)v.x : (C == COMP_IM ? (double)v.y : amp_of(v));
-}
-
-// Five-point derivative with the boundary rule of calcmuen_kernel1x
-// (imag3d.cu:1303-1332): 0 at both ends, centred 3-point at 1 and N-2.
-template <int C = COMP_AMP, typename P>
-__device__ __forceinline__ double deriv5(const P *__restrict__ f, int i, int n, long st, double h) {
-    if (i == 0 || i == n - 1) return 0.0;
-    if (i == 1) return (comp_of<C>(f[2 * st]) - comp_of<C>(f[0])) / (2.0 * h);
-    if (i == n - 2) return (comp_of<C>(f[(long)(n - 1) * st]) - comp_of<C>(f[(long)(n - 3) * st])) / (2.0 * h);
-    return (comp_of<C>(f[(long)(i - 2) * st]) - 8.0 * comp_of<C>(f[(long)(i - 1) * st]) +
-            8.0 * comp_of<C>(f[(long)(i + 1) * st]) - comp_of<C>(f[(long)(i + 2) * st])) / (12.0 * h);
-}
-
-// Kinetic density sum over the axes of (d psi)^2 / (3 - par) at (i, j, k) of
-// the row `row`: of |psi|, or with PHASE of the real and imaginary parts.
-template <int C, typename P>
-__device__ __forceinline__ double kin_comp(const P *__restrict__ psi, int i, int j, int k, long row, int Nx, int Ny,
-                                           int Nz, const MuenConst &mc) {
-    const long NyNz = (long)Ny * Nz;
-    const double dxv = deriv5<C>(psi + (long)j * Nz + k, i, Nx, NyNz, mc.dx);
-    double d = (dxv * dxv) / mc.kin;
-    const double dyv = deriv5<C>(psi + (long)i * NyNz + k, j, Ny, (long)Nz, mc.dy);
-    d += (dyv * dyv) / mc.kin;
-    const double dzv = deriv5<C>(psi + row * Nz, k, Nz, 1L, mc.dz);
-    d += (dzv * dzv) / mc.kin;
-    return d;
-}
-
-// Per-row z integrals of the chemical potential and energy densities
-// (calcmuen_kernel1x/1y/1z and kernel2, imag3d.cu:1293-1450; real3d.cu
-// 1382-1543, where real time differentiates |psi|).
-// PHASE (complex psi): the kinetic density of the real and imaginary parts
-// (|grad psi|^2) instead of that of |psi|.
-template <typename P, typename R, bool PHASE = false>
-__global__ void __launch_bounds__(256)
-k_rows_muen(const P *__restrict__ psi, const R *__restrict__ phi, const double *__restrict__ sq,
-            const double *__restrict__ wz, TrapConst tc, MuenConst mc, double *__restrict__ rmu,
-            double *__restrict__ ren, int Nx, int Ny, int Nz) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * 4 + wave;
-    if (row >= (long)Nx * Ny) return;
-    const int i = (int)(row / Ny), j = (int)(row % Ny);
-    double amu = 0.0, aen = 0.0;
-    for (int k = lane; k < Nz; k += 64) {
-        const long n = row * Nz + k;
-        double d;
-        if constexpr (PHASE)
-            d = kin_comp<COMP_RE>(psi, i, j, k, row, Nx, Ny, Nz, mc) + kin_comp<COMP_IM>(psi, i, j, k, row, Nx, Ny, Nz, mc);
-        else
-            d = kin_comp<COMP_AMP>(psi, i, j, k, row, Nx, Ny, Nz, mc);
-        double psi2 = amp_of(psi[n]);
-        psi2 *= psi2;
-        const double psi2lin = psi2 * mc.g;
-        const double psidd2lin = ((double)phi[n] / mc.nd) * mc.gd;
-        const double pot = trap(tc, sq[i], sq[Nx + j], sq[Nx + Ny + k]);
-        const double tmu = (pot + psi2lin + psidd2lin) * psi2 + d;
-        const double ten = (pot + 0.5 * psi2lin + 0.5 * psidd2lin) * psi2 + d;
-        amu += wz[k] * tmu;
-        aen += wz[k] * ten;
-    }
-    amu = wave_sum(amu);
-    aen = wave_sum(aen);
-    if (lane == 0) {
-        rmu[(long)j * Nx + i] = amu;
-        ren[(long)j * Nx + i] = aen;
-    }
-}
-
-hipError_t launch_rows_muen(hipStream_t s, const dbec_ctx *c, double *rmu, double *ren, bool phase) {
-    const auto &b = c->b;
-    TrapConst tc;
-    tc.half_par = 0.5 * c->p.par;
-    tc.g2 = c->p.vgamma * c->p.vgamma;
-    tc.n2 = c->p.vnu * c->p.vnu;
-    tc.l2 = c->p.vlambda * c->p.vlambda;
-    MuenConst mc;
-    mc.dx = c->p.dx;
-    mc.dy = c->p.dy;
-    mc.dz = c->p.dz;
-    mc.kin = 3.0 - c->p.par;
-    mc.g = c->g;
-    mc.gd = c->gd;
-    mc.nd = (double)(c->Nx * c->Ny * c->Nz);
-    const double *wz = b.wgt + c->Nx + c->Ny;
-    dim3 block(256), grid((unsigned)((c->Nx * c->Ny + 3) / 4));
-    const int Nx = (int)c->Nx, Ny = (int)c->Ny, Nz = (int)c->Nz;
-    const bool f32 = c->prec == DBEC_MIXED;
-    if (c->mode == DBEC_IMAG) {
-        if (f32)
-            k_rows_muen<float, float><<<grid, block, 0, s>>>(static_cast<const float *>(b.psi), static_cast<const float *>(b.phi),
-                                                             b.sq, wz, tc, mc, rmu, ren, Nx, Ny, Nz);
-        else
-            k_rows_muen<double, double><<<grid, block, 0, s>>>(static_cast<const double *>(b.psi),
-                                                               static_cast<const double *>(b.phi), b.sq, wz, tc, mc, rmu,
-                                                               ren, Nx, Ny, Nz);
-    } else if (phase) {
-        if (f32)
-            k_rows_muen<cpx<float>, float, true><<<grid, block, 0, s>>>(static_cast<const cpx<float> *>(b.psi),
-                                                                        static_cast<const float *>(b.phi), b.sq, wz,
-                                                                        tc, mc, rmu, ren, Nx, Ny, Nz);
-        else
-            k_rows_muen<cpx<double>, double, true><<<grid, block, 0, s>>>(static_cast<const cpx<double> *>(b.psi),
-                                                                          static_cast<const double *>(b.phi), b.sq,
-                                                                          wz, tc, mc, rmu, ren, Nx, Ny, Nz);
-    } else {
-        if (f32)
-            k_rows_muen<cpx<float>, float><<<grid, block, 0, s>>>(static_cast<const cpx<float> *>(b.psi),
-                                                                  static_cast<const float *>(b.phi), b.sq, wz, tc, mc,
-                                                                  rmu, ren, Nx, Ny, Nz);
-        else
-            k_rows_muen<cpx<double>, double><<<grid, block, 0, s>>>(static_cast<const cpx<double> *>(b.psi),
-                                                                    static_cast<const double *>(b.phi), b.sq, wz, tc,
-                                                                    mc, rmu, ren, Nx, Ny, Nz);
-    }
-    return hipGetLastError();
-}
-
-// Column and total sums over the row integrals, one workgroup.
-//   NORM:    scal[NORM] = sqrt(I0), scal[SCALE] = 1 / scal[NORM]        (I0 from A)
-//   MOMENTS: scal[NORM], scal[RX/RY/RZ] = sqrt(<x^2>, <y^2>, <z^2>), scal[R0]
-//   MUEN:    scal[MU] = integral of A, scal[EN] = integral of B
-template <int MODE>
-__global__ void __launch_bounds__(256)
-k_finalize(const double *__restrict__ A, const double *__restrict__ B, const double *__restrict__ wx,
-           const double *__restrict__ wy, const double *__restrict__ x2, const double *__restrict__ y2,
-           double *__restrict__ scal, int Nx, int Ny) {
-    __shared__ double s0[256], s1[256], s2[256], s3[256];
-    const int tid = threadIdx.x;
-    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    for (int x = tid; x < Nx; x += 256) {
-        double c0 = 0.0, c1 = 0.0, c2 = 0.0;
-        for (int y = 0; y < Ny; y++) {
-            const double a = A[(long)y * Nx + x];
-            c0 += wy[y] * a;
-            if (MODE == 1) {
-                c1 += wy[y] * y2[y] * a;
-                c2 += wy[y] * B[(long)y * Nx + x];
-            }
-            if (MODE == 2) c1 += wy[y] * B[(long)y * Nx + x];
-        }
-        p0 += wx[x] * c0;
-        if (MODE == 1) {
-            p1 += wx[x] * x2[x] * c0;
-            p2 += wx[x] * c1;
-            p3 += wx[x] * c2;
-        }
-        if (MODE == 2) p1 += wx[x] * c1;
-    }
-    s0[tid] = p0;
-    s1[tid] = p1;
-    s2[tid] = p2;
-    s3[tid] = p3;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) {
-            s0[tid] += s0[tid + o];
-            s1[tid] += s1[tid + o];
-            s2[tid] += s2[tid + o];
-            s3[tid] += s3[tid + o];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        if (MODE == 0) {
-            const double norm = sqrt(s0[0]);
-            scal[SC_NORM] = norm;
-            scal[SC_SCALE] = 1.0 / norm;
-        } else if (MODE == 1) {
-            scal[SC_NORM] = sqrt(s0[0]);
-            const double rx = sqrt(s1[0]), ry = sqrt(s2[0]), rz = sqrt(s3[0]);
-            scal[SC_RX] = rx;
-            scal[SC_RY] = ry;
-            scal[SC_RZ] = rz;
-            scal[SC_R0] = sqrt(rx * rx + ry * ry + rz * rz);
-        } else {
-            scal[SC_MU] = s0[0];
-            scal[SC_EN] = s1[0];
-        }
-    }
-}
-
-hipError_t launch_finalize(hipStream_t s, const dbec_ctx *c, int mode, const double *A, const double *B) {
-    const auto &b = c->b;
-    const double *wx = b.wgt, *wy = b.wgt + c->Nx, *x2 = b.sq, *y2 = b.sq + c->Nx;
-    const int Nx = (int)c->Nx, Ny = (int)c->Ny;
-    if (mode == 0) k_finalize<0><<<1, 256, 0, s>>>(A, B, wx, wy, x2, y2, b.scal, Nx, Ny);
-    else if (mode == 1) k_finalize<1><<<1, 256, 0, s>>>(A, B, wx, wy, x2, y2, b.scal, Nx, Ny);
-    else k_finalize<2><<<1, 256, 0, s>>>(A, B, wx, wy, x2, y2, b.scal, Nx, Ny);
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // Density extracts of the output writers (outden*, outpsi2*, imag3d.cu:1944-2399).
 // out[a][b] = sum over `axis` of w * |psi|^2, remaining indices in [x][y][z] order.

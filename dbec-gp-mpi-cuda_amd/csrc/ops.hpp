@@ -9,9 +9,6 @@
 
 namespace dbec {
 
-struct MuenConst {
-    double dx, dy, dz, kin, g, gd, nd;  // kin = 3 - par
-};
 template <typename V>
 struct SweepConst {
     V A0r, A, mA;  // diagonal of the explicit half, off-diagonal, and its negative
@@ -68,11 +65,15 @@ hipError_t launch_plane_inv(const dbec_ctx *c, const Solves &v, bool phi);
 hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves &v, int tiles);
 TrapConst trap_const(const dbec_ctx *c);
 NuConst nu_const(const dbec_ctx *c);
-hipError_t launch_rows_mod2(hipStream_t s, const dbec_ctx *c, double *rows0, double *rowsz);
-// phase: complex psi's kinetic density |grad psi|^2 instead of (grad |psi|)^2
-hipError_t launch_rows_muen(hipStream_t s, const dbec_ctx *c, double *rmu, double *ren, bool phase = false);
-// mode 0: norm and 1/norm; 1: norm and rms moments; 2: mu and E
-hipError_t launch_finalize(hipStream_t s, const dbec_ctx *c, int mode, const double *A, const double *B);
+// Observables (observe.hip): scal[NORM], scal[SCALE], or with moments
+// scal[NORM] and the rms values; scal[MU], scal[EN] from psi and phi (phase:
+// complex psi's kinetic density |grad psi|^2 instead of (grad |psi|)^2).  The
+// row buffer takes the partial sums; c->h_scal (may be null) the results too.
+hipError_t launch_obs_norm(hipStream_t s, const dbec_ctx *c, bool moments);
+hipError_t launch_obs_muen(hipStream_t s, const dbec_ctx *c, bool phase);
+// device scalars, or psi[n] (entries SC_COUNT, SC_COUNT + 1), to c->h_scal
+hipError_t launch_export_scalars(hipStream_t s, const dbec_ctx *c);
+hipError_t launch_export_point(hipStream_t s, const dbec_ctx *c, long n);
 hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, double *out);
 hipError_t launch_reduce2(hipStream_t s, const double *in, long n0, long n1, int axis, const double *w, double *out);
 hipError_t launch_mod2(hipStream_t s, const dbec_ctx *c, double *out);

@@ -367,9 +367,7 @@ struct dbec_server {
         if (e == hipSuccess) e = launch_set_scalar(v->stream, v->b.scal + SC_SCALE, 1.0);
         if (e == hipSuccess && v->mode == DBEC_IMAG) {
             // imag3d normalises psi0 (imag3d.cu:239): the first step reads psi / norm
-            double *r0 = v->b.rows;
-            e = launch_rows_mod2(v->stream, v, r0, nullptr);
-            if (e == hipSuccess) e = launch_finalize(v->stream, v, 0, r0, nullptr);
+            e = launch_obs_norm(v->stream, v, false);
         }
         if (e != hipSuccess) return fail(std::string("admission: ") + hipGetErrorString(e));
         j->t_start = now_since(t0);
