@@ -758,13 +758,6 @@ int autotune(dbec_ctx *c) {
     return DBEC_OK;
 }
 
-// Host-side selection of every o-th entry of a row-major 2-D array.
-void pick2(const std::vector<double> &m, long n0, long n1, long o0, long o1, double *out) {
-    long w = 0;
-    for (long a = 0; a < n0; a += o0)
-        for (long b2 = 0; b2 < n1; b2 += o1) out[w++] = m[a * n1 + b2];
-}
-
 }  // namespace
 
 extern "C" {
@@ -1042,117 +1035,31 @@ long dbec_density_count(const dbec_ctx *c, int kind, long ox, long oy, long oz) 
     }
 }
 
-int dbec_density(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) {
-    if (!c || !out) return fail(c, DBEC_EINVAL, "null argument");
-    if (dbec_density_count(c, kind, ox, oy, oz) < 0) return fail(c, DBEC_EINVAL, "bad density request");
-    (void)hipSetDevice(c->device);
-    CHK(materialize_scale(c));
+}  // extern "C"
+
+namespace {
+
+// Doubles of scratch that the weighted sums of an extract take; 0 for sampled
+// values of |psi|^2.
+long density_sums(const dbec_ctx *c, int kind) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
-    const double *wx = c->b.wgt, *wy = c->b.wgt + Nx;
-    size_t need;
     switch (kind) {
-    case DBEC_DEN_X: case DBEC_DEN_Y: case DBEC_DEN_XY: need = Nx * Ny + std::max(Nx, Ny); break;
-    case DBEC_DEN_Z: case DBEC_DEN_XZ: need = Nx * Nz + Nz; break;
-    case DBEC_DEN_YZ: need = Ny * Nz; break;
-    default: need = c->N; break;
+    case DBEC_DEN_XY: return Nx * Ny;
+    case DBEC_DEN_X: return Nx * Ny + Nx;
+    case DBEC_DEN_Y: return Nx * Ny + Ny;
+    case DBEC_DEN_XZ: return Nx * Nz;
+    case DBEC_DEN_Z: return Nx * Nz + Nz;
+    case DBEC_DEN_YZ: return Ny * Nz;
+    default: return 0;
     }
-    double *d = nullptr;
-    HIPCHK(c, hipMalloc(&d, need * sizeof(double)), "density scratch");
-    std::vector<double> h;
-    hipError_t e = hipSuccess;
-    auto fetch = [&](const double *src, size_t n) {
-        h.resize(n);
-        if (e == hipSuccess) e = hipMemcpyAsync(h.data(), src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    };
-    switch (kind) {
-    case DBEC_DEN_X:
-    case DBEC_DEN_Y:
-    case DBEC_DEN_XY:
-        e = launch_reduce3(c->stream, c, 2, d);  // [x][y]
-        if (kind == DBEC_DEN_XY) {
-            fetch(d, Nx * Ny);
-            if (e == hipSuccess) pick2(h, Nx, Ny, ox, oy, out);
-        } else if (kind == DBEC_DEN_X) {
-            if (e == hipSuccess) e = launch_reduce2(c->stream, d, Nx, Ny, 1, wy, d + Nx * Ny);
-            fetch(d + Nx * Ny, Nx);
-            if (e == hipSuccess) pick2(h, Nx, 1, ox, 1, out);
-        } else {
-            if (e == hipSuccess) e = launch_reduce2(c->stream, d, Nx, Ny, 0, wx, d + Nx * Ny);
-            fetch(d + Nx * Ny, Ny);
-            if (e == hipSuccess) pick2(h, Ny, 1, oy, 1, out);
-        }
-        break;
-    case DBEC_DEN_Z:
-    case DBEC_DEN_XZ:
-        e = launch_reduce3(c->stream, c, 1, d);  // [x][z]
-        if (kind == DBEC_DEN_XZ) {
-            fetch(d, Nx * Nz);
-            if (e == hipSuccess) pick2(h, Nx, Nz, ox, oz, out);
-        } else {
-            if (e == hipSuccess) e = launch_reduce2(c->stream, d, Nx, Nz, 0, wx, d + Nx * Nz);
-            fetch(d + Nx * Nz, Nz);
-            if (e == hipSuccess) pick2(h, Nz, 1, oz, 1, out);
-        }
-        break;
-    case DBEC_DEN_YZ:
-        e = launch_reduce3(c->stream, c, 0, d);  // [y][z]
-        fetch(d, Ny * Nz);
-        if (e == hipSuccess) pick2(h, Ny, Nz, oy, oz, out);
-        break;
-    default: {
-        e = launch_mod2(c->stream, c, d);
-        fetch(d, c->N);
-        if (e != hipSuccess) break;
-        long w = 0;
-        if (kind == DBEC_CUT_XY0) {
-            for (long i = 0; i < Nx; i += ox)
-                for (long j = 0; j < Ny; j += oy) out[w++] = h[(i * Ny + j) * Nz + Nz / 2];
-        } else if (kind == DBEC_CUT_X0Z) {
-            for (long i = 0; i < Nx; i += ox)
-                for (long k = 0; k < Nz; k += oz) out[w++] = h[(i * Ny + Ny / 2) * Nz + k];
-        } else if (kind == DBEC_CUT_0YZ) {
-            for (long j = 0; j < Ny; j += oy)
-                for (long k = 0; k < Nz; k += oz) out[w++] = h[((Nx / 2) * Ny + j) * Nz + k];
-        } else {
-            for (long i = 0; i < Nx; i += ox)
-                for (long j = 0; j < Ny; j += oy)
-                    for (long k = 0; k < Nz; k += oz) out[w++] = h[(i * Ny + j) * Nz + k];
-        }
-    } break;
-    }
-    (void)hipFree(d);
-    if (e != hipSuccess) return hip_fail(c, e, "density");
-    return DBEC_OK;
 }
 
-int dbec_density_noalloc(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) {
-    if (!c || !out) return fail(c, DBEC_EINVAL, "null argument");
-    const long cnt = dbec_density_count(c, kind, ox, oy, oz);
-    if (cnt < 0) return fail(c, DBEC_EINVAL, "bad density request");
-    (void)hipSetDevice(c->device);
-    double *d = scratch_of(c->device);
-    if (!d) return fail(c, DBEC_EDEVICE, "dbec_density_noalloc: the device scratch of this GPU has no address");
+// One extract through `d` (cap doubles): sums, sampling and the copy to `out`.
+// The sampled 3-D extract runs in slabs of x where it does not fit.
+int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, double *d, long cap) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
     const long sx = (Nx + ox - 1) / ox, sy = (Ny + oy - 1) / oy, sz = (Nz + oz - 1) / oz;
-    // doubles of scratch: the weighted sums of the extract, then its sampled values
-    long sums;
-    switch (kind) {
-    case DBEC_DEN_XY: sums = Nx * Ny; break;
-    case DBEC_DEN_X: sums = Nx * Ny + Nx; break;
-    case DBEC_DEN_Y: sums = Nx * Ny + Ny; break;
-    case DBEC_DEN_XZ: sums = Nx * Nz; break;
-    case DBEC_DEN_Z: sums = Nx * Nz + Nz; break;
-    case DBEC_DEN_YZ: sums = Ny * Nz; break;
-    default: sums = 0; break;
-    }
-    const long cap = (long)(DBEC_NOALLOC_SCRATCH_BYTES / sizeof(double));
-    if (sums + cnt > cap)
-        return fail(c, DBEC_EINVAL,
-                    "dbec_density_noalloc: this extract needs " + std::to_string((sums + cnt) * (long)sizeof(double)) +
-                        " bytes of device scratch, more than its " + std::to_string((long)DBEC_NOALLOC_SCRATCH_BYTES) +
-                        " bytes (use dbec_density or coarser output steps)");
-    CHK(materialize_scale(c));
+    const long sums = density_sums(c, kind), cnt = dbec_density_count(c, kind, ox, oy, oz);
     const double *wx = c->b.wgt, *wy = c->b.wgt + Nx;
     double *dst = d + sums;
     hipStream_t s = c->stream;
@@ -1187,26 +1094,61 @@ int dbec_density_noalloc(dbec_ctx *c, int kind, long ox, long oy, long oz, doubl
         break;
     default: {
         long start[3] = {0, 0, 0}, step[3] = {ox, oy, oz}, n[3] = {sx, sy, sz};
-        if (kind == DBEC_CUT_XY0) {
-            start[2] = Nz / 2;
-            step[2] = 1;
-            n[2] = 1;
-        } else if (kind == DBEC_CUT_X0Z) {
-            start[1] = Ny / 2;
-            step[1] = 1;
-            n[1] = 1;
-        } else if (kind == DBEC_CUT_0YZ) {
-            start[0] = Nx / 2;
-            step[0] = 1;
-            n[0] = 1;
+        const int fixed = kind == DBEC_CUT_XY0 ? 2 : (kind == DBEC_CUT_X0Z ? 1 : (kind == DBEC_CUT_0YZ ? 0 : -1));
+        if (fixed >= 0) {
+            start[fixed] = (fixed == 0 ? Nx : (fixed == 1 ? Ny : Nz)) / 2;
+            step[fixed] = 1;
+            n[fixed] = 1;
         }
-        e = launch_pick_mod2(s, c, start, step, n, dst);
-    } break;
+        const long slab = n[1] * n[2], per = std::min(n[0], cap / slab), total = n[0];
+        for (long a = 0; a < total && e == hipSuccess; a += per) {
+            n[0] = std::min(per, total - a);
+            e = launch_pick_mod2(s, c, start, step, n, d);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(out + a * slab, d, (size_t)(n[0] * slab) * sizeof(double), hipMemcpyDeviceToHost, s);
+            start[0] += n[0] * step[0];
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return hip_fail(c, e, "density");
+        return DBEC_OK;
+    }
     }
     if (e == hipSuccess) e = hipMemcpyAsync(out, dst, (size_t)cnt * sizeof(double), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return hip_fail(c, e, "density (no allocation)");
+    if (e != hipSuccess) return hip_fail(c, e, "density");
     return DBEC_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+// The scratch is the spectrum, which holds nothing between calls: at least 9
+// Nx Ny doubles, enough for every extract but the 3-D one, which takes slabs.
+int dbec_density(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) {
+    if (!c || !out) return fail(c, DBEC_EINVAL, "null argument");
+    if (dbec_density_count(c, kind, ox, oy, oz) < 0) return fail(c, DBEC_EINVAL, "bad density request");
+    (void)hipSetDevice(c->device);
+    CHK(materialize_scale(c));
+    const long cap = (long)((size_t)c->Nkz * c->Nx * c->Ny * 2 * real_elem(c) / sizeof(double));
+    return density_via(c, kind, ox, oy, oz, out, static_cast<double *>(c->b.spec), cap);
+}
+
+int dbec_density_noalloc(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) {
+    if (!c || !out) return fail(c, DBEC_EINVAL, "null argument");
+    const long cnt = dbec_density_count(c, kind, ox, oy, oz);
+    if (cnt < 0) return fail(c, DBEC_EINVAL, "bad density request");
+    (void)hipSetDevice(c->device);
+    double *d = scratch_of(c->device);
+    if (!d) return fail(c, DBEC_EDEVICE, "dbec_density_noalloc: the device scratch of this GPU has no address");
+    const long need = density_sums(c, kind) + cnt, cap = (long)(DBEC_NOALLOC_SCRATCH_BYTES / sizeof(double));
+    if (need > cap)
+        return fail(c, DBEC_EINVAL,
+                    "dbec_density_noalloc: this extract needs " + std::to_string(need * (long)sizeof(double)) +
+                        " bytes of device scratch, more than its " + std::to_string((long)DBEC_NOALLOC_SCRATCH_BYTES) +
+                        " bytes (use dbec_density or coarser output steps)");
+    CHK(materialize_scale(c));
+    return density_via(c, kind, ox, oy, oz, out, d, cap);
 }
 
 int dbec_get_table(dbec_ctx *c, int which, int axis, double *out) {

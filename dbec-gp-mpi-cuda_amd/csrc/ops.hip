@@ -608,142 +608,4 @@ hipError_t launch_norm_from_cols(hipStream_t s, const dbec_ctx *c, const Solves 
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ double mod2_of(double v) { return v * v; }
-__device__ __forceinline__ double mod2_of(float v) { return (double)v * (double)v; }
-__device__ __forceinline__ double mod2_of(cpx<double> v) {
-    double a = hypot(v.x, v.y);
-    return a * a;
-}
-__device__ __forceinline__ double mod2_of(cpx<float> v) {
-    double a = hypot((double)v.x, (double)v.y);
-    return a * a;
-}
-// ---------------------------------------------------------------------------
-// Density extracts of the output writers (outden*, outpsi2*, imag3d.cu:1944-2399).
-// out[a][b] = sum over `axis` of w * |psi|^2, remaining indices in [x][y][z] order.
-template <typename P>
-__global__ void k_reduce3(const P *__restrict__ psi, int axis, const double *__restrict__ w, double *__restrict__ out,
-                          int Nx, int Ny, int Nz) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long NyNz = (long)Ny * Nz;
-    double acc = 0.0;
-    if (axis == 2) {
-        if (t >= (long)Nx * Ny) return;
-        const P *r = psi + t * Nz;
-        for (int k = 0; k < Nz; k++) acc += w[k] * mod2_of(r[k]);
-    } else if (axis == 1) {
-        if (t >= (long)Nx * Nz) return;
-        const long i = t / Nz, k = t % Nz;
-        for (int j = 0; j < Ny; j++) acc += w[j] * mod2_of(psi[i * NyNz + (long)j * Nz + k]);
-    } else {
-        if (t >= (long)Ny * Nz) return;
-        for (int i = 0; i < Nx; i++) acc += w[i] * mod2_of(psi[(long)i * NyNz + t]);
-    }
-    out[t] = acc;
-}
-
-// out[a] = sum_b w[b] in[a][b] (axis 1) or out[b] = sum_a w[a] in[a][b] (axis 0)
-__global__ void k_reduce2(const double *__restrict__ in, int n0, int n1, int axis, const double *__restrict__ w,
-                          double *__restrict__ out) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    double acc = 0.0;
-    if (axis == 1) {
-        if (t >= n0) return;
-        for (int b = 0; b < n1; b++) acc += w[b] * in[(long)t * n1 + b];
-    } else {
-        if (t >= n1) return;
-        for (int a = 0; a < n0; a++) acc += w[a] * in[(long)a * n1 + t];
-    }
-    out[t] = acc;
-}
-
-template <typename P>
-__global__ void k_mod2(const P *__restrict__ psi, double *__restrict__ out, long n) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) out[t] = mod2_of(psi[t]);
-}
-
-template <typename P>
-static hipError_t reduce3_t(hipStream_t s, const P *psi, int axis, const double *w, double *out, long Nx, long Ny, long Nz) {
-    const long n = axis == 2 ? Nx * Ny : (axis == 1 ? Nx * Nz : Ny * Nz);
-    k_reduce3<P><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(psi, axis, w, out, (int)Nx, (int)Ny, (int)Nz);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, double *out) {
-    const double *w = c->b.wgt + (axis == 0 ? 0 : (axis == 1 ? c->Nx : c->Nx + c->Ny));
-    const bool f32 = c->prec == DBEC_MIXED;
-    if (c->mode == DBEC_IMAG)
-        return f32 ? reduce3_t(s, static_cast<const float *>(c->b.psi), axis, w, out, c->Nx, c->Ny, c->Nz)
-                   : reduce3_t(s, static_cast<const double *>(c->b.psi), axis, w, out, c->Nx, c->Ny, c->Nz);
-    return f32 ? reduce3_t(s, static_cast<const cpx<float> *>(c->b.psi), axis, w, out, c->Nx, c->Ny, c->Nz)
-               : reduce3_t(s, static_cast<const cpx<double> *>(c->b.psi), axis, w, out, c->Nx, c->Ny, c->Nz);
-}
-
-hipError_t launch_reduce2(hipStream_t s, const double *in, long n0, long n1, int axis, const double *w, double *out) {
-    const long n = axis == 1 ? n0 : n1;
-    k_reduce2<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, (int)n0, (int)n1, axis, w, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_mod2(hipStream_t s, const dbec_ctx *c, double *out) {
-    const unsigned g = (unsigned)((c->N + 255) / 256);
-    const bool f32 = c->prec == DBEC_MIXED;
-    if (c->mode == DBEC_IMAG) {
-        if (f32) k_mod2<float><<<g, 256, 0, s>>>(static_cast<const float *>(c->b.psi), out, c->N);
-        else k_mod2<double><<<g, 256, 0, s>>>(static_cast<const double *>(c->b.psi), out, c->N);
-    } else {
-        if (f32) k_mod2<cpx<float>><<<g, 256, 0, s>>>(static_cast<const cpx<float> *>(c->b.psi), out, c->N);
-        else k_mod2<cpx<double>><<<g, 256, 0, s>>>(static_cast<const cpx<double> *>(c->b.psi), out, c->N);
-    }
-    return hipGetLastError();
-}
-
-
-// Sampled extracts on the device (the allocation-free density entry point):
-// dst[a][b][k] = |psi|^2 at (x0 + a ox, y0 + b oy, z0 + k oz), the same
-// mod2_of as k_mod2, so the values equal those of the full extract bit for bit.
-template <typename P>
-__global__ void k_pick_mod2(const P *__restrict__ psi, long x0, long y0, long z0, long ox, long oy, long oz, long cy,
-                            long cz, long n, double *__restrict__ dst, long Ny, long Nz) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const long a = t / (cy * cz), b = (t / cz) % cy, k = t % cz;
-    dst[t] = mod2_of(psi[((x0 + a * ox) * Ny + y0 + b * oy) * Nz + z0 + k * oz]);
-}
-
-hipError_t launch_pick_mod2(hipStream_t s, const dbec_ctx *c, const long start[3], const long step[3],
-                            const long cnt[3], double *dst) {
-    const long n = cnt[0] * cnt[1] * cnt[2];
-    if (n <= 0) return hipSuccess;
-    const unsigned g = (unsigned)((n + 255) / 256);
-    const bool f32 = c->prec == DBEC_MIXED;
-#define DBEC_PICK_ARGS start[0], start[1], start[2], step[0], step[1], step[2], cnt[1], cnt[2], n, dst, c->Ny, c->Nz
-    if (c->mode == DBEC_IMAG) {
-        if (f32) k_pick_mod2<float><<<g, 256, 0, s>>>(static_cast<const float *>(c->b.psi), DBEC_PICK_ARGS);
-        else k_pick_mod2<double><<<g, 256, 0, s>>>(static_cast<const double *>(c->b.psi), DBEC_PICK_ARGS);
-    } else {
-        if (f32) k_pick_mod2<cpx<float>><<<g, 256, 0, s>>>(static_cast<const cpx<float> *>(c->b.psi), DBEC_PICK_ARGS);
-        else k_pick_mod2<cpx<double>><<<g, 256, 0, s>>>(static_cast<const cpx<double> *>(c->b.psi), DBEC_PICK_ARGS);
-    }
-#undef DBEC_PICK_ARGS
-    return hipGetLastError();
-}
-
-// dst[a][b] = src[(a o0) n1 + b o1], a < c0, b < c1
-__global__ void k_pick2(const double *__restrict__ src, long n1, long o0, long o1, long c1, long n,
-                        double *__restrict__ dst) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    dst[t] = src[(t / c1) * o0 * n1 + (t % c1) * o1];
-}
-
-hipError_t launch_pick2(hipStream_t s, const double *src, long n1, long o0, long o1, long c0, long c1, double *dst) {
-    const long n = c0 * c1;
-    if (n <= 0) return hipSuccess;
-    k_pick2<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(src, n1, o0, o1, c1, n, dst);
-    return hipGetLastError();
-}
-
 }  // namespace dbec
