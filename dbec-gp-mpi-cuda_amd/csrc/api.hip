@@ -18,6 +18,7 @@
 #include "fft_device.hpp"
 #include "fft_launch.hpp"
 #include "ops.hpp"
+#include "transfer.hpp"
 
 namespace dbec {
 
@@ -546,9 +547,11 @@ int setup(dbec_ctx *c) {
     const int yq = c->planes && (f32 ? pot_digit_rows<float>() : pot_digit_rows<double>()) ? (int)(Ny / 8) : 0;
     const long rows = pot_rows((int)Ny, yq);
     std::vector<double> pqd(qz * rows * qx, 0.0);
+    std::vector<long> row(qy);
+    for (long j = 0; j < qy; j++) row[j] = pot_row((int)j, yq) * qx;
     for (long k = 0; k < qz; k++)
-        for (long j = 0; j < qy; j++)
-            for (long i = 0; i < qx; i++) pqd[(k * rows + pot_row((int)j, yq)) * qx + i] = pq[(k * qx + i) * qy + j];
+        for (long i = 0; i < qx; i++)
+            for (long j = 0; j < qy; j++) pqd[k * rows * qx + row[j] + i] = pq[(k * qx + i) * qy + j];
     // host copy of the half table [kx][ky][kz<=Nz/2] for dbec_get_table
     c->h_potdd_half.resize(Nx * Ny * qz);
     for (long i = 0; i < Nx; i++)
@@ -837,6 +840,7 @@ int core_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stre
         delete c;
         return fail(nullptr, rc, m);
     }
+    staging_user(+1);
     *out = c;
     return DBEC_OK;
 }
@@ -848,7 +852,10 @@ int dbec_destroy(dbec_ctx *c) {
     if (!c) return DBEC_OK;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    if (!c->view) free_buffers(c);
+    if (!c->view) {
+        free_buffers(c);
+        staging_user(-1);
+    }
     if (c->own_stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return DBEC_OK;
@@ -858,15 +865,8 @@ int dbec_set_psi(dbec_ctx *c, const double *psi) {
     if (!c || !psi) return fail(c, DBEC_EINVAL, "null argument");
     (void)hipSetDevice(c->device);
     const size_t nd = (size_t)c->N * (c->mode == DBEC_REAL ? 2 : 1);
-    if (c->prec == DBEC_FP64) {
-        HIPCHK(c, hipMemcpyAsync(c->b.psi, psi, nd * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy psi");
-    } else {
-        std::vector<float> f(psi, psi + nd);
-        HIPCHK(c, hipMemcpyAsync(c->b.psi, f.data(), nd * sizeof(float), hipMemcpyHostToDevice, c->stream), "copy psi");
-    }
-    const double zero = 0.0;  // a new psi starts without exponent shift
-    HIPCHK(c, hipMemcpyAsync(c->b.scal + SC_SHIFT, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream), "copy");
-    HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
+    HIPCHK(c, launch_set_scalar(c->stream, c->b.scal + SC_SHIFT, 0.0), "set psi");  // a new psi starts without exponent shift
+    HIPCHK(c, store_field(c, c->b.psi, psi, nd, c->prec == DBEC_MIXED), "copy psi");
     c->scale_pending = false;
     return DBEC_OK;
 }
@@ -876,15 +876,7 @@ int dbec_get_psi(dbec_ctx *c, double *psi) {
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
     const size_t nd = (size_t)c->N * (c->mode == DBEC_REAL ? 2 : 1);
-    if (c->prec == DBEC_FP64) {
-        HIPCHK(c, hipMemcpyAsync(psi, c->b.psi, nd * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy psi");
-        HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
-    } else {
-        std::vector<float> f(nd);
-        HIPCHK(c, hipMemcpyAsync(f.data(), c->b.psi, nd * sizeof(float), hipMemcpyDeviceToHost, c->stream), "copy psi");
-        HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
-        for (size_t i = 0; i < nd; i++) psi[i] = f[i];
-    }
+    HIPCHK(c, fetch_field(c, psi, c->b.psi, nd, c->prec == DBEC_MIXED), "copy psi");
     return DBEC_OK;
 }
 
@@ -912,15 +904,7 @@ int dbec_calcpsidd2(dbec_ctx *c) {
 int dbec_get_psidd2(dbec_ctx *c, double *phi) {
     if (!c || !phi) return fail(c, DBEC_EINVAL, "null argument");
     (void)hipSetDevice(c->device);
-    if (c->prec == DBEC_FP64) {
-        HIPCHK(c, hipMemcpyAsync(phi, c->b.phi, c->N * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy");
-        HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
-    } else {
-        std::vector<float> f(c->N);
-        HIPCHK(c, hipMemcpyAsync(f.data(), c->b.phi, c->N * sizeof(float), hipMemcpyDeviceToHost, c->stream), "copy");
-        HIPCHK(c, hipStreamSynchronize(c->stream), "synchronize");
-        for (long i = 0; i < c->N; i++) phi[i] = f[i];
-    }
+    HIPCHK(c, fetch_field(c, phi, c->b.phi, (size_t)c->N, c->prec == DBEC_MIXED), "copy");
     return DBEC_OK;
 }
 
@@ -1104,11 +1088,9 @@ int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, d
         for (long a = 0; a < total && e == hipSuccess; a += per) {
             n[0] = std::min(per, total - a);
             e = launch_pick_mod2(s, c, start, step, n, d);
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(out + a * slab, d, (size_t)(n[0] * slab) * sizeof(double), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = fetch_field(c, out + a * slab, d, (size_t)(n[0] * slab), false);
             start[0] += n[0] * step[0];
         }
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return hip_fail(c, e, "density");
         return DBEC_OK;
     }
