@@ -170,13 +170,52 @@ __device__ __forceinline__ void dft16(cpx<R> *v) {
     t = v[11]; v[11] = v[14]; v[14] = t;
 }
 
+// Good-Thomas index maps: n = N2 n1 + N1 n2, k = N2 (N2^-1 mod N1) k1 +
+// N1 (N1^-1 mod N2) k2, all mod N1 N2; no twiddles between the factors.
+template <int DIR, typename R>
+__device__ __forceinline__ void dft6(cpx<R> *v) {
+    cpx<R> a[3] = {v[0], v[2], v[4]}, b[3] = {v[3], v[5], v[1]};
+    dft3<DIR>(a);
+    dft3<DIR>(b);
+    v[0] = a[0] + b[0]; v[3] = a[0] - b[0];
+    v[4] = a[1] + b[1]; v[1] = a[1] - b[1];
+    v[2] = a[2] + b[2]; v[5] = a[2] - b[2];
+}
+template <int DIR, typename R>
+__device__ __forceinline__ void dft10(cpx<R> *v) {
+    cpx<R> a[5] = {v[0], v[2], v[4], v[6], v[8]}, b[5] = {v[5], v[7], v[9], v[1], v[3]};
+    dft5<DIR>(a);
+    dft5<DIR>(b);
+    v[0] = a[0] + b[0]; v[5] = a[0] - b[0];
+    v[6] = a[1] + b[1]; v[1] = a[1] - b[1];
+    v[2] = a[2] + b[2]; v[7] = a[2] - b[2];
+    v[8] = a[3] + b[3]; v[3] = a[3] - b[3];
+    v[4] = a[4] + b[4]; v[9] = a[4] - b[4];
+}
+template <int DIR, typename R>
+__device__ __forceinline__ void dft12(cpx<R> *v) {
+    cpx<R> a[3][4] = {{v[0], v[3], v[6], v[9]}, {v[4], v[7], v[10], v[1]}, {v[8], v[11], v[2], v[5]}};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) dft4<DIR>(a[i][0], a[i][1], a[i][2], a[i][3]);
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2) {
+        cpx<R> t[3] = {a[0][k2], a[1][k2], a[2][k2]};
+        dft3<DIR>(t);
+#pragma unroll
+        for (int k1 = 0; k1 < 3; ++k1) v[(4 * k1 + 9 * k2) % 12] = t[k1];
+    }
+}
+
 template <int RADIX, int DIR, typename R>
 __device__ __forceinline__ void dft(cpx<R> *v) {
     if constexpr (RADIX == 2) dft2<DIR>(v);
     else if constexpr (RADIX == 3) dft3<DIR>(v);
     else if constexpr (RADIX == 4) dft4<DIR>(v[0], v[1], v[2], v[3]);
     else if constexpr (RADIX == 5) dft5<DIR>(v);
+    else if constexpr (RADIX == 6) dft6<DIR>(v);
     else if constexpr (RADIX == 8) dft8<DIR>(v);
+    else if constexpr (RADIX == 10) dft10<DIR>(v);
+    else if constexpr (RADIX == 12) dft12<DIR>(v);
     else if constexpr (RADIX == 16) dft16<DIR>(v);
     else static_assert(RADIX == 2, "unsupported radix");
 }
@@ -333,9 +372,9 @@ __device__ __forceinline__ void stockham_from_reg(cpx<R> *buf, int l, int t, con
 template <int N>
 struct FftPlan;
 
-#define DBEC_FFT_PLAN(NN, TT, ...)                                                           \
+#define DBEC_FFT_PLAN(PLAN, NN, TT, ...)                                                         \
     template <>                                                                              \
-    struct FftPlan<NN> {                                                                     \
+    struct PLAN<NN> {                                                                        \
         static constexpr int T = TT;                                                         \
         template <int L, typename R, bool SWZ = false>                                       \
         static __device__ __forceinline__ int at(int e, int l) {                             \
@@ -357,19 +396,30 @@ struct FftPlan;
         }                                                                                    \
     };
 
-DBEC_FFT_PLAN(16, 1, 16)
-DBEC_FFT_PLAN(32, 4, 8, 4)
-DBEC_FFT_PLAN(48, 12, 4, 4, 3)
-DBEC_FFT_PLAN(64, 16, 4, 4, 4)
-DBEC_FFT_PLAN(80, 20, 4, 4, 5)
-DBEC_FFT_PLAN(96, 12, 8, 4, 3)
-DBEC_FFT_PLAN(128, 16, 8, 16)
-DBEC_FFT_PLAN(160, 20, 8, 4, 5)
-DBEC_FFT_PLAN(192, 24, 8, 8, 3)
-DBEC_FFT_PLAN(256, 32, 8, 8, 4)
-DBEC_FFT_PLAN(320, 40, 8, 8, 5)
-DBEC_FFT_PLAN(384, 24, 16, 8, 3)
-DBEC_FFT_PLAN(512, 64, 8, 8, 8)
+DBEC_FFT_PLAN(FftPlan, 16, 1, 16)
+DBEC_FFT_PLAN(FftPlan, 32, 4, 8, 4)
+DBEC_FFT_PLAN(FftPlan, 48, 12, 4, 4, 3)
+DBEC_FFT_PLAN(FftPlan, 64, 16, 4, 4, 4)
+DBEC_FFT_PLAN(FftPlan, 80, 20, 4, 4, 5)
+DBEC_FFT_PLAN(FftPlan, 96, 12, 8, 4, 3)
+DBEC_FFT_PLAN(FftPlan, 128, 16, 8, 16)
+DBEC_FFT_PLAN(FftPlan, 160, 20, 8, 4, 5)
+DBEC_FFT_PLAN(FftPlan, 192, 24, 8, 8, 3)
+DBEC_FFT_PLAN(FftPlan, 256, 32, 8, 8, 4)
+DBEC_FFT_PLAN(FftPlan, 320, 40, 8, 8, 5)
+DBEC_FFT_PLAN(FftPlan, 384, 24, 16, 8, 3)
+DBEC_FFT_PLAN(FftPlan, 512, 64, 8, 8, 8)
+
+
+// Plan of the z transform fused with the z sweep: T = N / 8, so that L / 2
+// lines of T threads are the sweep's L rows of N / 16 threads.
+template <int N>
+struct FusedPlan : FftPlan<N> {};
+DBEC_FFT_PLAN(FusedPlan, 16, 2, 8, 2)
+DBEC_FFT_PLAN(FusedPlan, 48, 6, 8, 6)
+DBEC_FFT_PLAN(FusedPlan, 64, 8, 8, 8)
+DBEC_FFT_PLAN(FusedPlan, 80, 10, 8, 10)
+DBEC_FFT_PLAN(FusedPlan, 384, 48, 8, 8, 6)
 
 #undef DBEC_FFT_PLAN
 

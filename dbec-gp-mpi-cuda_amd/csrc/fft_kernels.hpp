@@ -27,6 +27,13 @@
 
 namespace dbec {
 
+// largest divisor of n up to 8: the batches of a loop of n loads
+constexpr int batch8(int n) {
+    for (int b = 8; b > 1; --b)
+        if (n % b == 0) return b;
+    return 1;
+}
+
 template <int N, int LM = 1>
 struct FftTile {
     static constexpr int T = FftPlan<N>::T;
@@ -153,135 +160,142 @@ k_zfwd(Solves v, int Nx, int Ny, const cpx<R> *__restrict__ twg, const double *_
 // |psi|^2 of its rows, two rows per complex line, and runs the forward
 // transform and split of k_zfwd on them, so psi is read once for both.  The
 // rows transform unscaled: the next step's norm comes from the column
-// partials (v.fold == 2, first workgroup of the forward y pass).  Built for
-// plans with T = N / 8, where L / 2 lines of T threads are the sweep's L * P
-// threads (P = N / 16 segments per row).
+// partials (v.fold == 2, first workgroup of the forward y pass).  The
+// transform's plan (FusedPlan) has T = N / 8, so its L / 2 lines of T threads
+// are the sweep's L * P threads (P = N / 16 segments per row).
+//
+// Bound by memory, as long as enough rows are in flight: a CU needs about
+// 100 KiB of psi on its way, and what limits that is LDS per workgroup and,
+// with complex FP64, registers.  LDS therefore holds, one after the other in
+// the same bytes: the tables, which the twiddles overwrite once the solve is
+// done; and the tile, the carry exchange while the tile is in registers, and
+// the transform buffer after the tile is stored.  Complex rows are twice the
+// transform buffer, so (half) they pass through a tile of half the rows in
+// two turns, each in registers before the next: 50 instead of 88 KiB a
+// workgroup at N = 256 in FP64.  Complex FP32 rows of less than 256 fit often
+// enough without, and the two turns' barriers measured 2-8 % slower there.
+// Measured (us; before: separate regions for tables, exchange and twiddles,
+// whole tiles; -> now; "+" where the two passes ran unfused before):
+//   rows    grid          FP64           FP32           complex FP64    complex FP32
+//   16    256x384x16      10 + 8 -> 10   9 + 6 -> 8     9 + 10 -> 14    7 + 8 -> 10
+//   48    192x320x48      11 + 10 -> 15  7 + 8 -> 10    13 + 22 -> 24   8 + 10 -> 13
+//   64    512x192x64      18 + 21 -> 29  11 + 11 -> 15  24 + 39 -> 46   14 + 19 -> 24
+//   80    256x384x80      22 + 25 -> 38  13 + 15 -> 23  30 + 47 -> 62   17 + 24 -> 30
+//   192   192^3           39 -> 37       21 -> 20       63 -> 58        31 -> 31
+//   256   256^3           75 -> 72       38 -> 38       214 -> 142      61 -> 58
+//   384   256x256x384     84 + 84 -> 131 38 + 43 -> 61  120 + 160 -> 229 55 + 89 -> 117
+//   512   128x256x512     110 -> 84      50 -> 44       279 -> 151      83 -> 72
 template <int N>
 struct FusedZ {
-    static constexpr bool ok = FftPlan<N>::T * 8 == N;
-    // Two LDS layouts.  FP64 (R = double): the sweep tables and exchange,
-    // the tile / transform buffer (padded), the twiddles; the row partials
-    // of the z integrals sit in the buffer's part past the tile when that is
-    // free (they are summed before the buffer is filled), else with the
-    // exchange.  FP32 spectra (compact: R = float): the tables, which the
-    // twiddles overwrite once the solve is done; the rows' last elements;
-    // the row partials; the tile region, which holds the carry exchange
-    // while the tile sits in registers and the transform buffer after the
-    // tile is stored (swizzled and unpadded where the padded one would not
-    // fit the tile's region: FP32 real lines; padded for complex FP32 rows,
-    // which are wide enough).  Measured at 256^3 and 192^3: the
-    // compact layout is 4-5 % faster with FP32 spectra (more workgroups per
-    // CU) and 8 % slower in FP64 (its two extra barriers).
-    template <typename R>
-    static constexpr bool compact() { return std::is_same<R, float>::value; }
+    static_assert(FusedPlan<N>::T * 8 == N, "fused z plan");
+    // complex rows: half a tile at a time
+    template <typename S>
+    static constexpr bool half() { return !std::is_floating_point<S>::value && (sizeof(S) == 16 || N >= 256); }
     // row partials of the z integrals: real lines (imaginary time) only
     template <typename S>
     static constexpr bool cols() { return std::is_floating_point<S>::value; }
-    template <typename S, typename R, int L>
-    static constexpr size_t tile_b() { return ((size_t)(N + Pk<S>::n) * L * sizeof(S) + 15) & ~size_t(15); }
-    // transform buffer swizzled (unpadded) only in the compact layout and
-    // only where the padded one would not fit in the tile's region (FP32
-    // real lines); complex FP32 rows are wide enough for the padded buffer
-    template <typename S, typename R, int L>
-    static constexpr bool swz() {
-        return compact<R>() && (size_t)N * (L / 2 + 1) * sizeof(cpx<R>) > tile_b<S, R, L>();
+    // wavefronts per SIMD that the registers have to leave room for (what LDS
+    // allows; left to itself the compiler takes more registers than that)
+    template <typename S>
+    static constexpr int waves() {
+        if (cols<S>()) return sizeof(S) == 8 ? 3 : 6;
+        return sizeof(S) == 16 ? 3 : 4;
     }
+    template <typename S, int L>
+    static constexpr size_t tile_b() {
+        return ((size_t)(N + Pk<S>::n) * (half<S>() ? L / 2 : L) * sizeof(S) + 15) & ~size_t(15);
+    }
+    // transform buffer swizzled (unpadded) where the padded one does not fit
+    // in the tile's region
+    template <typename S, typename R, int L>
+    static constexpr bool swz() { return (size_t)N * (L / 2 + 1) * sizeof(cpx<R>) > tile_b<S, L>(); }
+    // the region of the tile, the exchange and the transform buffer
     template <typename S, typename R, int L>
     static constexpr size_t x_b() {
-        constexpr size_t tile = tile_b<S, R, L>();
+        constexpr size_t tile = tile_b<S, L>();
         constexpr size_t buf = (size_t)N * (swz<S, R, L>() ? L / 2 : L / 2 + 1) * sizeof(cpx<R>);
-        constexpr size_t ex = compact<R>() ? 2 * (size_t)L * (N / 16) * sizeof(typename Arith<S>::T) : 0;
+        constexpr size_t ex = 2 * (size_t)L * (N / 16) * sizeof(typename Arith<S>::T);
         constexpr size_t m = tile > buf ? tile : buf;
         return ((m > ex ? m : ex) + 15) & ~size_t(15);
     }
-    // FP64 layout
-    template <typename S, typename R, int L>
-    static constexpr bool exn_in_x() {
-        return x_b<S, R, L>() - tile_b<S, R, L>() >= (size_t)L * (N / 16) * sizeof(double);
-    }
-    template <typename S, typename R, int L>
-    static constexpr size_t sh_b() {
-        using A = typename Arith<S>::T;
-        return (SweepShared<A, 16>::bytes(N, L * (N / 16), L, cols<S>() && !exn_in_x<S, R, L>()) + 15) & ~size_t(15);
-    }
-    // compact layout: tables (or twiddles), last elements, row partials
-    template <typename S, typename R, int L>
+    // tables (or twiddles), last elements, row partials, then the region
+    template <typename S, typename R>
     static constexpr size_t tab_b() {
         using A = typename Arith<S>::T;
         constexpr size_t t = 4 * (size_t)SweepShared<A, 16>::tab_len(N) * sizeof(A), w = (size_t)N * sizeof(cpx<R>);
         return ((t > w ? t : w) + 15) & ~size_t(15);
     }
-    template <typename S, typename R, int L>
+    template <typename S, int L>
     static constexpr size_t exl_b() { return ((size_t)L * sizeof(typename Arith<S>::T) + 15) & ~size_t(15); }
-    template <typename S, typename R, int L>
+    template <typename S, int L>
     static constexpr size_t exn_b() {
         return cols<S>() ? ((size_t)L * (N / 16) * sizeof(double) + 15) & ~size_t(15) : 0;
     }
-    // offset of the tile region
     template <typename S, typename R, int L>
-    static constexpr size_t x_off() {
-        return compact<R>() ? tab_b<S, R, L>() + exl_b<S, R, L>() + exn_b<S, R, L>() : sh_b<S, R, L>();
-    }
+    static constexpr size_t x_off() { return tab_b<S, R>() + exl_b<S, L>() + exn_b<S, L>(); }
     template <typename S, typename R, int L>
-    static constexpr size_t lds() {
-        return x_off<S, R, L>() + x_b<S, R, L>() + (compact<R>() ? 0 : N * sizeof(cpx<R>));
-    }
-    // the kernel exists for rows L: whole transform lines, at most 512
-    // threads, LDS within 160 KiB
+    static constexpr size_t lds() { return x_off<S, R, L>() + x_b<S, R, L>(); }
+    // the kernel exists for rows L: at most 512 threads, LDS within 160 KiB
     template <typename S, typename R, int L>
-    static constexpr bool fits() {
-        return ok && (L / 2) * FftPlan<N>::T == L * (N / 16) && L * (N / 16) <= 512 && lds<S, R, L>() <= 160 * 1024;
-    }
+    static constexpr bool fits() { return L * (N / 16) <= 512 && lds<S, R, L>() <= 160 * 1024; }
 };
 
 template <int N, typename S, typename R, int L, bool COLS>
-__global__ void __launch_bounds__(L *(N / 16))
+__global__ void __launch_bounds__(L *(N / 16), FusedZ<N>::template waves<S>())
 k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, SweepConst<typename Arith<S>::T> k,
               const double *__restrict__ wz, const double *__restrict__ wy, const cpx<R> *__restrict__ twg) {
     using A = typename Arith<S>::T;
+    using F = FusedZ<N>;
+    using Pl = FusedPlan<N>;
     // psi tile rows of N + VE elements: 16-byte aligned, and consecutive rows
     // 4 banks apart, so the packet accesses below are conflict-free
     constexpr int M = 16, VE = Pk<S>::n, KV = M / VE;
     constexpr int P = N / M, WG = L * P, LF = L / 2, RS = N + VE;
-    using Pl = FftPlan<N>;
-    static_assert(FftPlan<N>::T * LF == WG, "one transform thread per sweep thread");
-    using F = FusedZ<N>;
+    constexpr bool HALF = F::template half<S>();
+    // turns through the tile, rows and threads of each
+    constexpr int NH = HALF ? 2 : 1, LH = L / NH, TH = WG / NH;
+    static_assert(Pl::T * LF == WG && KV % NH == 0 && TH * NH == WG, "one transform thread per sweep thread");
     static_assert(COLS == F::template cols<S>(), "z integrals for real lines");
-    constexpr bool CMP = F::template compact<R>();  // compact layout
     constexpr size_t X_OFF = F::template x_off<S, R, L>(), X_B = F::template x_b<S, R, L>();
+    constexpr size_t TAB_B = F::template tab_b<S, R>(), EXL_B = F::template exl_b<S, L>();
     constexpr bool SWZ = F::template swz<S, R, L>();  // swizzled transform buffer
-    static_assert(X_B >= (size_t)RS * L * sizeof(S) && X_B >= (size_t)N * (SWZ ? LF : LF + 1) * sizeof(cpx<R>),
+    static_assert(X_B >= (size_t)RS * LH * sizeof(S) && X_B >= (size_t)N * (SWZ ? LF : LF + 1) * sizeof(cpx<R>),
                   "fused z LDS");
     __shared__ __align__(16) char smem[F::template lds<S, R, L>()];
     const SolveAt sr = solve_at(v);
     S *__restrict__ psi = reinterpret_cast<S *>(sr.psi);
     cpx<R> *__restrict__ spec = reinterpret_cast<cpx<R> *>(sr.spec);
-    SweepShared<A, M> sh(smem, N, WG, L,
-                      (!CMP && F::template exn_in_x<S, R, L>()) ? reinterpret_cast<double *>(smem + X_OFF + F::template tile_b<S, R, L>())
-                                                                 : nullptr);
-    cpx<R> *tw = reinterpret_cast<cpx<R> *>(smem + X_OFF + X_B);
-    if constexpr (CMP) {
-        constexpr size_t TAB_B = F::template tab_b<S, R, L>(), EXL_B = F::template exl_b<S, R, L>();
-        sh.exa = reinterpret_cast<A *>(smem + X_OFF);  // in the tile region while the tile is in registers
-        sh.exb = sh.exa + WG;
-        sh.exl = reinterpret_cast<A *>(smem + TAB_B);
-        sh.exn = reinterpret_cast<double *>(smem + TAB_B + EXL_B);
-        tw = reinterpret_cast<cpx<R> *>(smem);  // over the tables, after the solve
-    }
+    SweepShared<A, M> sh(smem, N, WG, L);
+    sh.exa = reinterpret_cast<A *>(smem + X_OFF);  // in the tile region while the tile is in registers
+    sh.exb = sh.exa + WG;
+    sh.exl = reinterpret_cast<A *>(smem + TAB_B);
+    sh.exn = reinterpret_cast<double *>(smem + TAB_B + EXL_B);
+    cpx<R> *tw = reinterpret_cast<cpx<R> *>(smem);  // over the tables, after the solve
     S *tile = reinterpret_cast<S *>(smem + X_OFF);
     cpx<R> *buf = reinterpret_cast<cpx<R> *>(smem + X_OFF);  // after the tile is stored
     const int tid = threadIdx.x;
-    const int l = tid % L, s = tid / L;
+    const int hh = HALF ? tid / TH : 0, th = HALF ? tid % TH : tid;
+    const int l = hh * LH + th % LH, s = th / LH;
+    // a complex FP64 segment is 256 bytes, so the 16 lanes that one LDS cycle
+    // serves (LH rows of 16 / LH segments) would meet in the same banks: the
+    // segments that share a cycle take their packets in different orders
+    const auto at = [](int row, int e) {
+        if constexpr (HALF && sizeof(S) == 16) e ^= ((e >> 4) & (16 / (LH < 16 ? LH : 16) - 1)) * (LH < 16 ? LH : 0);
+        return row * RS + e;
+    };
     const int yt = (Ny + L - 1) / L;
     const int xrow = blockIdx.x / yt, tno = blockIdx.x % yt, y0 = tno * L;
     const int nl = min(L, Ny - y0);
     const long base = ((long)xrow * Ny + y0) * N;
     const A zero = m_zero(k.A);
     const int npk = nl * N / VE;
+    const int e0 = s * M;
+    const bool act = l < nl;
+    A vv[M], hl, hr;
     const CoefPre<A> cp = coef_pre(tab, N, tid);
-    // compact layout: the twiddles wait in registers until the tables are free
-    constexpr int KT = CMP ? (N + WG - 1) / WG : 1;
-    cpx<R> twr[KT];
+    // the twiddles wait in registers until the tables are free
+    constexpr int KT = (N + WG - 1) / WG;
+    R twx[KT], twy[KT];
     {
         typename Pk<S>::type r[KV];
 #pragma unroll
@@ -289,29 +303,53 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
             const int iv = tid + q * WG;
             r[q] = ld_pk(psi + base + (unsigned)((iv < npk ? iv : 0) * VE));
         }
-        if constexpr (CMP) {
 #pragma unroll
-            for (int q = 0; q < KT; ++q) {
-                const int i = tid + q * WG;
-                twr[q] = twg[i < N ? i : 0];
-            }
+        for (int q = 0; q < KT; ++q) {
+            const int i = tid + q * WG;
+            const cpx<R> w = twg[i < N ? i : 0];
+            twx[q] = w.x;
+            twy[q] = w.y;
         }
         coef_put(sh, cp, tab, N, tid, WG);
-        if constexpr (!CMP) stage_twiddles(tw, twg, N, tid, WG);
+        if constexpr (NH == 1) {
 #pragma unroll
-        for (int q = 0; q < KV; ++q) {
-            const int iv = tid + q * WG;
-            if (iv < npk) {
-                const int e = (iv * VE) % N, row = (iv * VE) / N;
-                st_pk(tile + row * RS + e, r[q]);
+            for (int q = 0; q < KV; ++q) {
+                const int iv = tid + q * WG;
+                if (iv < npk) {
+                    const int e = (iv * VE) % N, row = (iv * VE) / N;
+                    st_pk(tile + row * RS + e, r[q]);
+                }
+            }
+        } else {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            if (h) __syncthreads();  // the last pass's rows are in registers
+#pragma unroll
+            for (int q = h * (KV / NH); q < (h + 1) * (KV / NH); ++q) {
+                const int iv = tid + q * WG;
+                if (iv < npk) {
+                    const int e = (iv * VE) % N, row = (iv * VE) / N;
+                    st_pk(tile + at(row - h * LH, e), r[q]);
+                }
+            }
+            __syncthreads();
+            if (NH == 1 || hh == h) {
+                const int row = l - h * LH;
+                hl = hr = zero;
+#pragma unroll
+                for (int m = 0; m < KV; ++m) {
+                    const typename Pk<S>::type pk = ld_pk(tile + at(row, e0 + m * VE));
+#pragma unroll
+                    for (int j = 0; j < VE; ++j) vv[m * VE + j] = act ? to_a(pk.e[j]) : zero;
+                }
+                if (act && e0 > 0) hl = to_a(tile[at(row, e0 - 1)]);
+                if (act && e0 + M < N) hr = to_a(tile[at(row, e0 + M)]);
             }
         }
+        }
     }
-    __syncthreads();
-    const int e0 = s * M;
-    const bool act = l < nl;
-    A vv[M];
-    {
+    if constexpr (NH == 1) {
+        __syncthreads();
         const S *row = tile + l * RS;
 #pragma unroll
         for (int m = 0; m < KV; ++m) {
@@ -319,25 +357,23 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
 #pragma unroll
             for (int j = 0; j < VE; ++j) vv[m * VE + j] = act ? to_a(pk.e[j]) : zero;
         }
-        const A hl = (act && e0 > 0) ? to_a(row[e0 - 1]) : zero;
-        const A hr = (act && e0 + M < N) ? to_a(row[e0 + M]) : zero;
-        if constexpr (CMP) __syncthreads();  // the tile is in registers; its region takes the carry exchange
-        // batched carry folds for real lines (measured 1.3 us faster at 256 in
-        // both precisions); complex lines keep the loop (slower batched: the
-        // extra registers cost occupancy)
-        constexpr int PC = std::is_floating_point<A>::value ? P : 0;
-        const double acc = seg_solve<A, M, COLS, true, PC>(vv, hl, hr, e0, N, s, l, L, P, sh, k, wz);
-        if constexpr (CMP) __syncthreads();  // every carry is read; the region holds the tile again
-        if (act) {
-            S *orow = tile + l * RS;
+        hl = (act && e0 > 0) ? to_a(row[e0 - 1]) : zero;
+        hr = (act && e0 + M < N) ? to_a(row[e0 + M]) : zero;
+    }
+    {
+        __syncthreads();  // the tile is in registers; its region takes the carry exchange
+        const double acc = seg_solve<A, M, COLS, true>(vv, hl, hr, e0, N, s, l, L, P, sh, k, wz);
+        __syncthreads();  // every carry is read; the region holds the tile again
+        const auto put = [&](int row) {
 #pragma unroll
             for (int m = 0; m < KV; ++m) {
                 typename Pk<S>::type o;
 #pragma unroll
                 for (int j = 0; j < VE; ++j) o.e[j] = from_a<S>(vv[m * VE + j]);
-                st_pk(orow + e0 + m * VE, o);
+                st_pk(tile + at(row, e0 + m * VE), o);
             }
-        }
+        };
+        if (act && (NH == 1 || hh == 0)) put(l);
         if constexpr (COLS) {
             sh.exn[s * L + l] = acc;
             __syncthreads();
@@ -354,22 +390,28 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
         } else {
             __syncthreads();
         }
-    }
 #pragma unroll
-    for (int q = 0; q < KV; ++q) {
-        const int iv = tid + q * WG;
-        if (iv < npk) {
-            const int e = (iv * VE) % N, row = (iv * VE) / N;
-            st_pk(psi + base + (unsigned)(iv * VE), ld_pk(tile + row * RS + e));
+        for (int h = 0; h < NH; ++h) {
+            if (h) {
+                __syncthreads();  // the first rows are stored
+                if (act && hh == h) put(l - h * LH);
+                __syncthreads();
+            }
+#pragma unroll
+            for (int q = h * (KV / NH); q < (h + 1) * (KV / NH); ++q) {
+                const int iv = tid + q * WG;
+                if (iv < npk) {
+                    const int e = (iv * VE) % N, row = (iv * VE) / N;
+                    st_pk(psi + base + (unsigned)(iv * VE), ld_pk(tile + at(row - h * LH, e)));
+                }
+            }
         }
     }
     __syncthreads();  // the tile is stored; its LDS becomes the transform buffer (and the tables the twiddles)
-    if constexpr (CMP) {
 #pragma unroll
-        for (int q = 0; q < KT; ++q) {
-            const int i = tid + q * WG;
-            if (i < N) tw[i] = twr[q];
-        }
+    for (int q = 0; q < KT; ++q) {
+        const int i = tid + q * WG;
+        if (i < N) tw[i] = {twx[q], twy[q]};
     }
     // |psi|^2 of the new rows (zero past the plane's last row): row 2p is the
     // real part, row 2p + 1 the imaginary part of line p
@@ -654,7 +696,7 @@ k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, i
     // the tile's psi (at most 256 bytes per thread) is fetched before the
     // transform, so its latency overlaps the spectrum load and the passes
     constexpr bool PREFETCH = Q * sizeof(P) <= 256;
-    constexpr int C = PREFETCH ? Q : (Q < 8 ? Q : 8);  // psi batch
+    constexpr int C = PREFETCH ? Q : batch8(Q);  // psi batch
     static_assert((2 * L * N) % WG == 0 && Q % C == 0, "zinv_nu tile");
     __shared__ cpx<R> buf[N * lds_slots_per_row<L, SWZ>()];
     // complex FP64 psi with the swizzled buffer: the passes read the
@@ -762,7 +804,7 @@ k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, i
         Pl::template run<+1, L, SWZ>(buf, tid % L, tid / L, tw);
     }
     constexpr int QF = L * N / WG;
-    constexpr int CF = PREFETCH ? QF : (QF < 8 ? QF : 8);
+    constexpr int CF = PREFETCH ? QF : batch8(QF);
     static_assert((L * N) % WG == 0 && QF % CF == 0, "zinv_nu face tile");
 #pragma unroll
     for (int q0 = 0; q0 < QF; q0 += CF) {
@@ -939,7 +981,6 @@ struct FftLaunchImpl {
         case 32: return sweepz_zfwd_t<S, R, COLS, 32>(a);
         case 16: return sweepz_zfwd_t<S, R, COLS, 16>(a);
         case 8: return sweepz_zfwd_t<S, R, COLS, 8>(a);
-        case 4: return sweepz_zfwd_t<S, R, COLS, 4>(a);
         default: return hipErrorInvalidValue;
         }
     }
@@ -958,7 +999,6 @@ struct FftLaunchImpl {
         case 32: return FusedZ<N>::template fits<S, R, 32>();
         case 16: return FusedZ<N>::template fits<S, R, 16>();
         case 8: return FusedZ<N>::template fits<S, R, 8>();
-        case 4: return FusedZ<N>::template fits<S, R, 4>();
         default: return false;
         }
     }

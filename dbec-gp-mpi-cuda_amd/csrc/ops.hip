@@ -395,6 +395,19 @@ int sweep_z_rows(const dbec_ctx *c) {
     return f32 ? z_rows<cpx<float>>(c->Nz) : z_rows<cpx<double>>(c->Nz);
 }
 
+// Rows per workgroup of the fused z kernel: real lines as the z sweep (its
+// column partials are one per workgroup of those rows); complex lines, which
+// have none and pass through half a tile, the most that give at most 256
+// threads (measured at 512 complex FP64: 8 rows 151, the z sweep's 4 rows 200
+// us; at 128: 32 rows 41, 16 rows 46 us; twice the rows, so twice the threads
+// at a barrier: 143 -> 159 us at 256^3, 229 -> 280 at 256x256x384).
+int fused_z_rows(const dbec_ctx *c) {
+    if (c->mode == DBEC_IMAG) return sweep_z_rows(c);
+    int L = 64;
+    while (L > 8 && L * (c->Nz / 16) > 256) L /= 2;
+    return L;
+}
+
 AxisArgs sweep_axis_args(const dbec_ctx *c, int axis) {
     const CoefLayout lay(c->Nx, c->Ny, c->Nz);
     const bool cplx = c->mode == DBEC_REAL;
@@ -420,7 +433,7 @@ void sweep_z_args(const dbec_ctx *c, FftArgs &a) {
         for (int q = 0; q < 2; q++) a.zk[i][q] = z.k[i][q];
     a.wz = c->b.wgt + c->Nx + c->Ny;
     a.wy = c->b.wgt + c->Nx;
-    a.zrows = sweep_z_rows(c);
+    a.zrows = fused_z_rows(c);
 }
 
 long sweep_z_tiles(const dbec_ctx *c) {

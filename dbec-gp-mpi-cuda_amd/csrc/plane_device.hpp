@@ -15,49 +15,6 @@
 
 namespace dbec {
 
-// Good-Thomas index maps: n = N2 n1 + N1 n2, k = N2 (N2^-1 mod N1) k1 +
-// N1 (N1^-1 mod N2) k2, all mod N1 N2; no twiddles between the factors.
-template <int DIR, typename R>
-__device__ __forceinline__ void dft6(cpx<R> *v) {
-    cpx<R> a[3] = {v[0], v[2], v[4]}, b[3] = {v[3], v[5], v[1]};
-    dft3<DIR>(a);
-    dft3<DIR>(b);
-    v[0] = a[0] + b[0]; v[3] = a[0] - b[0];
-    v[4] = a[1] + b[1]; v[1] = a[1] - b[1];
-    v[2] = a[2] + b[2]; v[5] = a[2] - b[2];
-}
-template <int DIR, typename R>
-__device__ __forceinline__ void dft10(cpx<R> *v) {
-    cpx<R> a[5] = {v[0], v[2], v[4], v[6], v[8]}, b[5] = {v[5], v[7], v[9], v[1], v[3]};
-    dft5<DIR>(a);
-    dft5<DIR>(b);
-    v[0] = a[0] + b[0]; v[5] = a[0] - b[0];
-    v[6] = a[1] + b[1]; v[1] = a[1] - b[1];
-    v[2] = a[2] + b[2]; v[7] = a[2] - b[2];
-    v[8] = a[3] + b[3]; v[3] = a[3] - b[3];
-    v[4] = a[4] + b[4]; v[9] = a[4] - b[4];
-}
-template <int DIR, typename R>
-__device__ __forceinline__ void dft12(cpx<R> *v) {
-    cpx<R> a[3][4] = {{v[0], v[3], v[6], v[9]}, {v[4], v[7], v[10], v[1]}, {v[8], v[11], v[2], v[5]}};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) dft4<DIR>(a[i][0], a[i][1], a[i][2], a[i][3]);
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) {
-        cpx<R> t[3] = {a[0][k2], a[1][k2], a[2][k2]};
-        dft3<DIR>(t);
-#pragma unroll
-        for (int k1 = 0; k1 < 3; ++k1) v[(4 * k1 + 9 * k2) % 12] = t[k1];
-    }
-}
-template <int Q, int DIR, typename R>
-__device__ __forceinline__ void dftq(cpx<R> *v) {
-    if constexpr (Q == 6) dft6<DIR>(v);
-    else if constexpr (Q == 10) dft10<DIR>(v);
-    else if constexpr (Q == 12) dft12<DIR>(v);
-    else dft<Q, DIR>(v);
-}
-
 // Index arithmetic in 24-bit multiplies: the 32-bit integer multiply (low or
 // high half) issues at a quarter of the rate, and the planes' run-time strides
 // need several per element.  Every factor here is below 2^24, every product
@@ -135,7 +92,7 @@ __device__ __forceinline__ void passq_t(cpx<R> *buf, int st, const FastDiv &nl, 
         cpx<R> v[Q];
 #pragma unroll
         for (int r = 0; r < Q; ++r) v[r] = p[r * st];
-        dftq<Q, DIR>(v);
+        dft<Q, DIR>(v);
         if constexpr (DIR > 0) {
 #pragma unroll
             for (int j = 1; j < Q; ++j) v[j] = cmulc(v[j], tw[m24(j, c)]);

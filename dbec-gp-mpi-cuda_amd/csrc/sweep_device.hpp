@@ -137,8 +137,7 @@ struct SweepTab {
 
 // LDS layout shared by the sweep kernels with segments of M: the four
 // tables, the carry exchange (one per thread), the last elements, the row
-// partials (one per thread, only with the z integrals; placed elsewhere when
-// the kernel passes exn_at).  A table keeps the M entries of segment s in
+// partials (one per thread, only with the z integrals).  A table keeps the M entries of segment s in
 // slots s (M + PAD) .. s (M + PAD) + M - 1 (slot()).  The lanes of a
 // wavefront read the same entry of several segments at once: unpadded,
 // segments of 256 bytes (16 complex doubles, 32 complex floats) all start in
@@ -161,7 +160,7 @@ struct SweepShared {
     double *exn;
     __host__ __device__ static constexpr int tab_len(int n) { return n + (n / M) * PAD; }
     __host__ __device__ static constexpr int slot(int i) { return i + (i / M) * PAD; }
-    __device__ SweepShared(char *raw, int n, int nthreads, int L, double *exn_at = nullptr) {
+    __device__ SweepShared(char *raw, int n, int nthreads, int L) {
         const int tl = tab_len(n);
         ca = reinterpret_cast<A *>(raw);
         cg = ca + tl;
@@ -170,7 +169,7 @@ struct SweepShared {
         exa = fa + tl;
         exb = exa + nthreads;
         exl = exb + nthreads;
-        exn = exn_at ? exn_at : reinterpret_cast<double *>(exl + L);
+        exn = reinterpret_cast<double *>(exl + L);
     }
     __host__ __device__ static constexpr size_t bytes(int n, int nthreads, int L, bool with_exn) {
         return (4 * (size_t)tab_len(n) + 2 * (size_t)nthreads + L) * sizeof(A) +
@@ -253,10 +252,7 @@ __device__ __forceinline__ cpx<R> sweep_back(const SweepConst<cpx<R>> &k, cpx<R>
 // every iteration keeps the test.  The x / y sweeps of complex lines use the
 // latter: peeled, the compiler schedules them with more registers, which
 // measured slower there (and faster in every other sweep).
-// PC > 0: the line has exactly PC segments, known at compile time (P == PC);
-// the carry folds then load every segment's carry at once and run the same
-// FMA chain predicated, instead of one LDS round trip per step.
-template <typename A, int M, bool COLS, bool PEEL, int PC = 0>
+template <typename A, int M, bool COLS, bool PEEL>
 __device__ __forceinline__ double seg_solve(A (&v)[M], A hl, A hr, int e0, int n, int s, int l, int L, int P,
                                             const SweepShared<A, M> &sh, const SweepConst<A> &k,
                                             const double *__restrict__ wz) {
@@ -294,17 +290,7 @@ __device__ __forceinline__ double seg_solve(A (&v)[M], A hl, A hr, int e0, int n
     if (s == P - 1) sh.exl[l] = v[M - 1];  // cbeta[N-2] = psi[N-1]
     __syncthreads();
     A x = sh.exl[l];
-    if constexpr (PC > 0) {
-        A eb[PC], ea[PC];
-#pragma unroll
-        for (int t = 0; t < PC; ++t) {
-            eb[t] = sh.exb[t * L + l];
-            ea[t] = sh.exa[t * L + l];
-        }
-#pragma unroll
-        for (int t = PC - 1; t > 0; --t)
-            if (t > s) x = m_fma(eb[t], x, ea[t]);
-    } else {
+    {
         // in groups of FB carries loaded at once (the same FMA order as one
         // at a time, without an LDS round trip per step)
         int t = P - 1;
@@ -345,17 +331,7 @@ __device__ __forceinline__ double seg_solve(A (&v)[M], A hl, A hr, int e0, int n
     sh.exb[s * L + l] = sh.fa[tb + (top - e0)];  // the segment's product of calpha
     __syncthreads();
     A y = zero;  // psi'[0] = 0
-    if constexpr (PC > 0) {
-        A eb[PC], ea[PC];
-#pragma unroll
-        for (int t = 0; t < PC - 1; ++t) {
-            eb[t] = sh.exb[t * L + l];
-            ea[t] = sh.exa[t * L + l];
-        }
-#pragma unroll
-        for (int t = 0; t < PC - 1; ++t)
-            if (t < s) y = m_fma(eb[t], y, ea[t]);
-    } else {
+    {
         int t = 0;
         for (; t + (FB - 1) < s; t += FB) {
             A eb[FB], ea[FB];
