@@ -14,6 +14,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace dbec {
 
 template <typename R>
@@ -410,6 +412,54 @@ DBEC_FFT_PLAN(FftPlan, 320, 40, 8, 8, 5)
 DBEC_FFT_PLAN(FftPlan, 384, 24, 16, 8, 3)
 DBEC_FFT_PLAN(FftPlan, 512, 64, 8, 8, 8)
 
+// Other plans of some lengths, for the passes that run faster with them: two
+// passes, or three of nearly equal radices, in place of one that ends in a
+// small radix.  Measured (us, FftPlan -> the other; complex psi "c"):
+//   x convolution     FP64: 48 14 -> 12 (48x160x512), 80 12 -> 11 (80x192x192),
+//                     96 38 -> 36 (96x512x256), 160 18 -> 15 (160^3),
+//                     320 65 -> 54 (320x320x160); 192 24 -> 24, 384 57 -> 64
+//                     and 512 43 -> 46 (512x80x320) keep theirs.  FP32:
+//                     160 12 -> 11, 192 16 -> 14 (192^3), 320 39 -> 32,
+//                     384 37 -> 29 (384x96x384), 512 32 -> 28
+//   y passes          FP64: 320 46 -> 43; 384 28 -> 31 (256x384x80) keeps its.
+//                     FP32: 384 14 -> 12; 320 12 -> 14 (64x320x384) keeps its.
+//                     The short ones keep theirs: fewer threads a workgroup
+//                     make the norm that the first one forms slower.
+//   inverse z + nu    FP64: 320 87 -> 75, c 139 -> 106 (512x80x320), c160
+//                     43 -> 33 (160^3; FftPlanC), 384 159 -> 122 with half the
+//                     lines a workgroup (256x256x384; 177 without); c384
+//                     212 -> 260 keeps its.  FP32: 320 50 -> 38, c 55 -> 49,
+//                     384 98 -> 79, c 124 -> 113
+template <int N>
+struct FftPlanB : FftPlan<N> {};
+DBEC_FFT_PLAN(FftPlanB, 48, 8, 6, 8)
+DBEC_FFT_PLAN(FftPlanB, 80, 10, 8, 10)
+DBEC_FFT_PLAN(FftPlanB, 96, 12, 8, 12)
+DBEC_FFT_PLAN(FftPlanB, 160, 20, 8, 10, 2)
+DBEC_FFT_PLAN(FftPlanB, 192, 24, 8, 6, 4)
+DBEC_FFT_PLAN(FftPlanB, 320, 32, 10, 8, 4)
+DBEC_FFT_PLAN(FftPlanB, 384, 48, 8, 8, 6)
+DBEC_FFT_PLAN(FftPlanB, 512, 32, 16, 8, 4)
+template <int N>
+struct FftPlanC : FftPlan<N> {};
+DBEC_FFT_PLAN(FftPlanC, 160, 16, 10, 16)
+
+template <bool B, int N>
+using PlanIf = std::conditional_t<B, FftPlanB<N>, FftPlan<N>>;
+template <typename R>
+constexpr bool kF32 = std::is_same<R, float>::value || std::is_same<R, cpx<float>>::value;
+// x convolution, y passes (spectrum in R) and the fused inverse z pass (psi in P)
+template <int N, typename R>
+using XPlan = PlanIf<kF32<R> || (N != 192 && N != 384 && N != 512), N>;
+template <int N, typename R>
+using YPlan = PlanIf<kF32<R> ? N == 384 : N == 320, N>;
+template <int N, typename P>
+using ZPlan = std::conditional_t<N == 160 && std::is_same<P, cpx<double>>::value, FftPlanC<N>,
+                                 PlanIf<N == 320 || (N == 384 && !std::is_same<P, cpx<double>>::value), N>>;
+// half the lines per workgroup in the fused inverse z pass: where whole tiles
+// leave a CU 6-8 wavefronts (complex FP64 at 512: 153 -> 140 us, 128x256x512)
+template <int N, typename P>
+constexpr bool kZHalf = (N == 384 && std::is_same<P, double>::value) || (N == 512 && std::is_same<P, cpx<double>>::value);
 
 // Plan of the z transform fused with the z sweep: T = N / 8, so that L / 2
 // lines of T threads are the sweep's L rows of N / 16 threads.

@@ -34,14 +34,15 @@ constexpr int batch8(int n) {
     return 1;
 }
 
-template <int N, int LM = 1>
+template <typename Pl, int LM = 1, bool HALF = false>
 struct FftTile {
-    static constexpr int T = FftPlan<N>::T;
+    static constexpr int T = Pl::T;
     // lines per workgroup: at least 8, and at least one wavefront of threads,
     // times the tile multiplier LM (wider tiles: longer contiguous HBM runs
     // on the strided side, fewer workgroups per CU)
     static constexpr int L0 = (64 + T - 1) / T;
-    static constexpr int L = LM * (L0 <= 8 ? 8 : (L0 <= 16 ? 16 : (L0 <= 32 ? 32 : 64)));
+    static constexpr int L1 = L0 <= 8 ? 8 : (L0 <= 16 ? 16 : (L0 <= 32 ? 32 : 64));
+    static constexpr int L = HALF ? LM * L1 / 2 : LM * L1;
     static constexpr int WG = L * T;
 };
 
@@ -81,9 +82,9 @@ struct PsiTraits<cpx<float>> {
 
 // ---------------------------------------------------------------------------
 template <int N, typename R, typename P, int LM>
-__global__ void __launch_bounds__((FftTile<N, LM>::WG))
+__global__ void __launch_bounds__((FftTile<FftPlan<N>, LM>::WG))
 k_zfwd(Solves v, int Nx, int Ny, const cpx<R> *__restrict__ twg, const double *__restrict__ wx, int tiles) {
-    constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
+    constexpr int L = FftTile<FftPlan<N>, LM>::L, WG = FftTile<FftPlan<N>, LM>::WG;
     using Pl = FftPlan<N>;
     __shared__ cpx<R> buf[N * (L + 1)];
     __shared__ cpx<R> tw[N];
@@ -446,10 +447,10 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
 // first workgroup of each solve's forward pass also forms the last step's
 // norm from the z sweep's column partials, for the x convolution and calcnu.
 template <int N, int DIR, typename R, int LM>
-__global__ void __launch_bounds__((FftTile<N, LM>::WG))
+__global__ void __launch_bounds__((FftTile<YPlan<N, R>, LM>::WG))
 k_ypass(Solves v, long nlines, const cpx<R> *__restrict__ twg, const double *__restrict__ wx, int tiles, int Nx) {
-    constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
-    using Pl = FftPlan<N>;
+    constexpr int L = FftTile<YPlan<N, R>, LM>::L, WG = FftTile<YPlan<N, R>, LM>::WG;
+    using Pl = YPlan<N, R>;
     __shared__ cpx<R> buf[N * (L + 1)];
     __shared__ cpx<R> tw[N];
     cpx<R> *__restrict__ spec = reinterpret_cast<cpx<R> *>(solve_at(v).spec);
@@ -490,11 +491,12 @@ k_ypass(Solves v, long nlines, const cpx<R> *__restrict__ twg, const double *__r
 // yq = Ny / 8; the norm from one partial per x with v.fold == 3); a template
 // parameter, so the other grids' kernel stays as lean as without it.
 template <int N, typename R, int LM, bool PL>
-__global__ void __launch_bounds__((FftTile<N, LM>::WG))
+__global__ void __launch_bounds__((FftTile<XPlan<N, R>, LM>::WG))
 k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict__ twg, const double *__restrict__ wx,
         int yq) {
-    constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
-    constexpr int T = FftPlan<N>::T, K = N / T;  // x values per thread
+    constexpr int L = FftTile<XPlan<N, R>, LM>::L, WG = FftTile<XPlan<N, R>, LM>::WG;
+    using Pl = XPlan<N, R>;
+    constexpr int T = Pl::T, K = N / T;  // x values per thread
     static_assert(L * T == WG, "xconv tile");
     constexpr int NXH = N / 2 + 1;
     __shared__ cpx<R> buf[N * (L + 1)];
@@ -543,14 +545,14 @@ k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict
         s2 = (R)(sc * sc);
         __syncthreads();  // the scratch becomes the transform buffer
     }
-    FftPlan<N>::template run_reg<-1, L>(buf, l, t, tw, r);
+    Pl::template run_reg<-1, L>(buf, l, t, tw, r);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const R w = pw[k] * s2;
         r[k] = {r[k].x * w, r[k].y * w};
     }
     __syncthreads();  // the forward transform's last LDS reads are done
-    FftPlan<N>::template run_reg<+1, L>(buf, l, t, tw, r);
+    Pl::template run_reg<+1, L>(buf, l, t, tw, r);
     if (l < nl) {
 #pragma unroll
         for (int k = 0; k < K; ++k) g[(unsigned)((t + k * T) * Ny)] = r[k];
@@ -565,7 +567,7 @@ k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict
 // the spec indices of A and B and returns which of them exist (bit 0: A,
 // bit 1: B); a missing one reads as zero.  All loads are issued before the
 // first LDS write.
-template <int N, int L, int WG, bool SWZ, typename R, typename SpecIdx>
+template <int N, typename Pl, int L, int WG, bool SWZ, typename R, typename SpecIdx>
 __device__ __forceinline__ void load_hermitian_pairs(cpx<R> *buf, const cpx<R> *__restrict__ spec, int tid,
                                                      const SpecIdx &idx) {
     constexpr int nkz = N / 2 + 1;
@@ -593,8 +595,8 @@ __device__ __forceinline__ void load_hermitian_pairs(cpx<R> *buf, const cpx<R> *
                 a.y = R(0);
                 b.y = R(0);
             }
-            buf[FftPlan<N>::template at<L, R, SWZ>(k, p)] = {a.x - b.y, a.y + b.x};
-            if (k > 0 && k < N / 2) buf[FftPlan<N>::template at<L, R, SWZ>(N - k, p)] = {a.x + b.y, b.x - a.y};
+            buf[Pl::template at<L, R, SWZ>(k, p)] = {a.x - b.y, a.y + b.x};
+            if (k > 0 && k < N / 2) buf[Pl::template at<L, R, SWZ>(N - k, p)] = {a.x + b.y, b.x - a.y};
         }
     }
 }
@@ -602,10 +604,10 @@ __device__ __forceinline__ void load_hermitian_pairs(cpx<R> *buf, const cpx<R> *
 // The same pairs straight into the registers of the first transform pass:
 // v[r] = Z[t + r T] of line p = l (T threads per line), each bin above N/2
 // formed from the spectrum rows of its mirror N - k.
-template <int N, typename R, typename SpecIdx>
+template <int N, typename Pl, typename R, typename SpecIdx>
 __device__ __forceinline__ void load_hermitian_reg(cpx<R> *v, const cpx<R> *__restrict__ spec, int l, int t,
                                                    const SpecIdx &idx) {
-    constexpr int T = FftPlan<N>::T, K = N / T;
+    constexpr int T = Pl::T, K = N / T;
     cpx<R> ra[K], rb[K];
     int m[K];
 #pragma unroll
@@ -631,9 +633,9 @@ __device__ __forceinline__ void load_hermitian_reg(cpx<R> *v, const cpx<R> *__re
 }
 
 template <int N, typename R, int LM>
-__global__ void __launch_bounds__((FftTile<N, LM>::WG))
+__global__ void __launch_bounds__((FftTile<FftPlan<N>, LM>::WG))
 k_zinv(const cpx<R> *__restrict__ spec, R *__restrict__ phi, int Nx, int Ny, const cpx<R> *__restrict__ twg) {
-    constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
+    constexpr int L = FftTile<FftPlan<N>, LM>::L, WG = FftTile<FftPlan<N>, LM>::WG;
     using Pl = FftPlan<N>;
     __shared__ cpx<R> buf[N * (L + 1)];
     __shared__ cpx<R> tw[N];
@@ -643,7 +645,7 @@ k_zinv(const cpx<R> *__restrict__ spec, R *__restrict__ phi, int Nx, int Ny, con
     const int y0 = (blockIdx.x % ytiles) * 2 * L;
     const int nrows = min(2 * L, Ny - y0);
     stage_twiddles(tw, twg, N, tid, WG);
-    load_hermitian_pairs<N, L, WG, false>(buf, spec, tid, [&](int p, int k, unsigned &ia, unsigned &ib) {
+    load_hermitian_pairs<N, Pl, L, WG, false>(buf, spec, tid, [&](int p, int k, unsigned &ia, unsigned &ib) {
         ia = (unsigned)((k * Nx + x) * Ny + y0 + 2 * p);
         ib = ia + 1;
         return (2 * p < nrows ? 1 : 0) | (2 * p + 1 < nrows ? 2 : 0);
@@ -687,11 +689,11 @@ k_zinv(const cpx<R> *__restrict__ spec, R *__restrict__ phi, int Nx, int Ny, con
 // (load_hermitian_reg) instead of through LDS; with SWZ the transform buffer
 // is the swizzled one (lds_at).  Neither changes the results.
 template <int N, typename R, typename P, int LM, bool ZREG, bool SWZ>
-__global__ void __launch_bounds__((FftTile<N, LM>::WG))
+__global__ void __launch_bounds__((FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::WG))
 k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, int nfaceb,
           const cpx<R> *__restrict__ twg) {
-    constexpr int L = FftTile<N, LM>::L, WG = FftTile<N, LM>::WG;
-    using Pl = FftPlan<N>;
+    constexpr int L = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::L, WG = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::WG;
+    using Pl = ZPlan<N, P>;
     constexpr int Q = 2 * L * N / WG;  // psi elements per thread (interior rows)
     // the tile's psi (at most 256 bytes per thread) is fetched before the
     // transform, so its latency overlaps the spectrum load and the passes
@@ -745,11 +747,11 @@ k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, i
             return (2 * p < nrows ? 1 : 0) | (2 * p + 1 < nrows ? 2 : 0);
         };
         if constexpr (ZREG) {
-            cpx<R> zv[N / FftPlan<N>::T];
-            load_hermitian_reg<N>(zv, spec, tid % L, tid / L, idx);
+            cpx<R> zv[N / Pl::T];
+            load_hermitian_reg<N, Pl>(zv, spec, tid % L, tid / L, idx);
             Pl::template run_from_reg<+1, L, SWZ>(buf, tid % L, tid / L, tw, zv);
         } else {
-            load_hermitian_pairs<N, L, WG, SWZ>(buf, spec, tid, idx);
+            load_hermitian_pairs<N, Pl, L, WG, SWZ>(buf, spec, tid, idx);
             __syncthreads();
             Pl::template run<+1, L, SWZ>(buf, tid % L, tid / L, tw);
         }
@@ -795,11 +797,11 @@ k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, i
         return 3;
     };
     if constexpr (ZREG) {
-        cpx<R> zv[N / FftPlan<N>::T];
-        load_hermitian_reg<N>(zv, spec, tid % L, tid / L, fidx);
+        cpx<R> zv[N / Pl::T];
+        load_hermitian_reg<N, Pl>(zv, spec, tid % L, tid / L, fidx);
         Pl::template run_from_reg<+1, L, SWZ>(buf, tid % L, tid / L, tw, zv);
     } else {
-        load_hermitian_pairs<N, L, WG, SWZ>(buf, spec, tid, fidx);
+        load_hermitian_pairs<N, Pl, L, WG, SWZ>(buf, spec, tid, fidx);
         __syncthreads();
         Pl::template run<+1, L, SWZ>(buf, tid % L, tid / L, tw);
     }
@@ -860,11 +862,12 @@ struct FftLaunchImpl {
     // psi); plans of 192 threads or more keep LM = 1 there (measured at
     // 256^3 and 192^3).  FP32 xconv always takes LM = 2, the other FP64
     // passes LM = 1.
-    static constexpr int WIDE = FftTile<N, 1>::WG < 192 ? 2 : 1;
+    template <typename Pl>
+    static constexpr int wide() { return FftTile<Pl, 1>::WG < 192 ? 2 : 1; }
 
     template <int LM>
     static hipError_t zfwd_t(const FftArgs &a) {
-        using Tl = FftTile<N, LM>;
+        using Tl = FftTile<FftPlan<N>, LM>;
         const int ytiles = (int)((a.Ny + 2 * Tl::L - 1) / (2 * Tl::L));
         dim3 grid((unsigned)(a.Nx * ytiles), (unsigned)a.v.nb), block(Tl::WG);
         const int Nx = (int)a.Nx, Ny = (int)a.Ny;
@@ -887,45 +890,36 @@ struct FftLaunchImpl {
     }
     static hipError_t zfwd(const FftArgs &a) {
         static const int l64 = fft_lm("DBEC_FFT_LM_ZFWD64", 0), l32 = fft_lm("DBEC_FFT_LM_ZFWD32", 0);
-        return pick_lm(a, a.fp32 ? l32 : l64, 0, a.fp32 ? WIDE : 1) == 2 ? zfwd_t<2>(a) : zfwd_t<1>(a);
+        return pick_lm(a, a.fp32 ? l32 : l64, 0, a.fp32 ? wide<FftPlan<N>>() : 1) == 2 ? zfwd_t<2>(a) : zfwd_t<1>(a);
     }
     // FP32 spectra use tiles twice as wide, so every strided access still
     // moves 128-256 contiguous bytes.
 
-    template <int LM>
+    template <typename R, int LM>
     static hipError_t ypass_t(int dir, const FftArgs &a) {
-        using Tl = FftTile<N, LM>;
+        using Tl = FftTile<YPlan<N, R>, LM>;
         const long nlines = a.Nkz * a.Nx;
         dim3 grid((unsigned)((nlines + Tl::L - 1) / Tl::L), (unsigned)a.v.nb), block(Tl::WG);
-        if (!a.fp32) {
-            auto *tw = static_cast<const cpx<double> *>(a.tw);
-            if (dir < 0) k_ypass<N, -1, double, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
-            else k_ypass<N, +1, double, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
-        } else {
-            auto *tw = static_cast<const cpx<float> *>(a.tw);
-            if (dir < 0) k_ypass<N, -1, float, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
-            else k_ypass<N, +1, float, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
-        }
+        auto *tw = static_cast<const cpx<R> *>(a.tw);
+        if (dir < 0) k_ypass<N, -1, R, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
+        else k_ypass<N, +1, R, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
         return hipGetLastError();
     }
     static hipError_t ypass(int dir, const FftArgs &a) {
         static const int l64 = fft_lm("DBEC_FFT_LM_YPASS64", 0), l32 = fft_lm("DBEC_FFT_LM_YPASS32", 0);
-        return pick_lm(a, a.fp32 ? l32 : l64, 1, a.fp32 ? WIDE : 1) == 2 ? ypass_t<2>(dir, a) : ypass_t<1>(dir, a);
+        const bool two = pick_lm(a, a.fp32 ? l32 : l64, 1, a.fp32 ? wide<YPlan<N, float>>() : 1) == 2;
+        if (a.fp32) return two ? ypass_t<float, 2>(dir, a) : ypass_t<float, 1>(dir, a);
+        return two ? ypass_t<double, 2>(dir, a) : ypass_t<double, 1>(dir, a);
     }
 
-    template <int LM>
+    template <typename R, int LM>
     static hipError_t xconv_t(const FftArgs &a) {
-        using Tl = FftTile<N, LM>;
+        using Tl = FftTile<XPlan<N, R>, LM>;
         const int ytiles = (int)((a.Ny + Tl::L - 1) / Tl::L);
         dim3 grid((unsigned)(a.Nkz * ytiles), (unsigned)a.v.nb), block(Tl::WG);
         const auto launch = [&](auto planes) {
-            constexpr bool PL = decltype(planes)::value;
-            if (!a.fp32)
-                k_xconv<N, double, LM, PL><<<grid, block, 0, a.stream>>>(
-                    a.v, static_cast<const double *>(a.potddq), (int)a.Ny, static_cast<const cpx<double> *>(a.tw), a.wx, a.yq);
-            else
-                k_xconv<N, float, LM, PL><<<grid, block, 0, a.stream>>>(
-                    a.v, static_cast<const float *>(a.potddq), (int)a.Ny, static_cast<const cpx<float> *>(a.tw), a.wx, a.yq);
+            k_xconv<N, R, LM, decltype(planes)::value><<<grid, block, 0, a.stream>>>(
+                a.v, static_cast<const R *>(a.potddq), (int)a.Ny, static_cast<const cpx<R> *>(a.tw), a.wx, a.yq);
         };
         if (a.yq) launch(std::true_type{});
         else launch(std::false_type{});
@@ -933,7 +927,9 @@ struct FftLaunchImpl {
     }
     static hipError_t xconv(const FftArgs &a) {
         static const int l64 = fft_lm("DBEC_FFT_LM_XCONV64", 0), l32 = fft_lm("DBEC_FFT_LM_XCONV32", 0);
-        return pick_lm(a, a.fp32 ? l32 : l64, 2, a.fp32 ? 2 : 1) == 2 ? xconv_t<2>(a) : xconv_t<1>(a);
+        const bool two = pick_lm(a, a.fp32 ? l32 : l64, 2, a.fp32 ? 2 : 1) == 2;
+        if (a.fp32) return two ? xconv_t<float, 2>(a) : xconv_t<float, 1>(a);
+        return two ? xconv_t<double, 2>(a) : xconv_t<double, 1>(a);
     }
 
     template <typename S, typename R, bool COLS, int L>
@@ -1009,7 +1005,7 @@ struct FftLaunchImpl {
 
     // single solve: spectrum of `one` -> phi
     static hipError_t zinv(const FftArgs &a) {
-        using Tl = FftTile<N, 1>;
+        using Tl = FftTile<FftPlan<N>, 1>;
         const int ytiles = (int)((a.Ny + 2 * Tl::L - 1) / (2 * Tl::L));
         dim3 grid((unsigned)(a.Nx * ytiles)), block(Tl::WG);
         if (!a.fp32)
@@ -1025,7 +1021,7 @@ struct FftLaunchImpl {
 
     template <typename P, typename R, int LM>
     static hipError_t fused_t(const FftArgs &a) {
-        using Tl = FftTile<N, LM>;
+        using Tl = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>;
         const auto *tw = static_cast<const cpx<R> *>(a.tw);
         const int ytiles = (int)((a.Ny + 2 * Tl::L - 1) / (2 * Tl::L));
         const int nmain = (int)((a.Nx - 1) * ytiles);
@@ -1059,7 +1055,9 @@ struct FftLaunchImpl {
     static hipError_t fused(const FftArgs &a) {
         // FP64: narrow tiles for complex psi
         static const int l64 = fft_lm("DBEC_FFT_LM_FUSED64", 0), l32 = fft_lm("DBEC_FFT_LM_FUSED32", 0);
-        const int lm = pick_lm(a, a.fp32 ? l32 : l64, 3, (a.fp32 || !a.cpsi) ? WIDE : 1);
+        const int rule = !a.fp32 ? (a.cpsi ? 1 : wide<ZPlan<N, double>>())
+                                 : (a.cpsi ? wide<ZPlan<N, cpx<float>>>() : wide<ZPlan<N, float>>());
+        const int lm = pick_lm(a, a.fp32 ? l32 : l64, 3, rule);
         return lm == 2 ? fused_lm<2>(a) : fused_lm<1>(a);
     }
 };
