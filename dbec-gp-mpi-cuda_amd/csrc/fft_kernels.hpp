@@ -241,10 +241,21 @@ struct FusedZ {
     static constexpr bool fits() { return L * (N / 16) <= 512 && lds<S, R, L>() <= 160 * 1024; }
 };
 
+// Whether the workgroups run from the largest x down, for psi of `bytes` (all
+// solves of the launch).  The y sweep before it ends with the planes of the
+// largest x, and 256 MiB of last-level cache hold the latest of them: complex
+// psi of 176 MiB or more, which does not stay there as a whole beside the
+// spectrum, is taken from that end (us a step, from the smallest x -> from the
+// largest: complex FP32 482 -> 445 at 256x256x384, 456 -> 420 at 384x256x256,
+// but 361 -> 365 at 512x512x80, 160 MiB; complex FP64 921 -> 901, 917 -> 891,
+// 745 -> 735 at 512x256x160, 574 -> 574 at 256^3).  Real psi of these sizes
+// gains nothing (604 -> 605 at 256x256x384 FP64).
+inline bool z_reversed(bool real, long bytes) { return !real && bytes >= (176L << 20); }
+
 template <int N, typename S, typename R, int L, bool COLS>
 __global__ void __launch_bounds__(L *(N / 16), FusedZ<N>::template waves<S>())
 k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, SweepConst<typename Arith<S>::T> k,
-              const double *__restrict__ wz, const double *__restrict__ wy, const cpx<R> *__restrict__ twg) {
+              const double *__restrict__ wz, const double *__restrict__ wy, const cpx<R> *__restrict__ twg, bool reversed) {
     using A = typename Arith<S>::T;
     using F = FusedZ<N>;
     using Pl = FusedPlan<N>;
@@ -285,7 +296,8 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
         return row * RS + e;
     };
     const int yt = (Ny + L - 1) / L;
-    const int xrow = blockIdx.x / yt, tno = blockIdx.x % yt, y0 = tno * L;
+    const int bid = !COLS && reversed ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
+    const int xrow = bid / yt, tno = bid % yt, y0 = tno * L;
     const int nl = min(L, Ny - y0);
     const long base = ((long)xrow * Ny + y0) * N;
     const A zero = m_zero(k.A);
@@ -945,8 +957,9 @@ struct FftLaunchImpl {
                                   static_cast<const TT *>(a.ztab[2]), static_cast<const TT *>(a.ztab[3])};
             SweepConst<A> k;
             zconst(a, k);
+            const bool reversed = z_reversed(COLS, (long)a.v.nb * a.Nx * a.Ny * N * (long)sizeof(S));
             k_sweepz_zfwd<N, S, R, L, COLS><<<grid, block, 0, a.stream>>>(a.v, (int)a.Nx, (int)a.Ny, tab, k, a.wz, a.wy,
-                                                                         static_cast<const cpx<R> *>(a.tw));
+                                                                         static_cast<const cpx<R> *>(a.tw), reversed);
             return hipGetLastError();
         }
     }

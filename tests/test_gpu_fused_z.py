@@ -40,3 +40,22 @@ def test_every_length(hip_lib, oracle_lib, nz):
             a, b = run(hip_lib, prec, (3,)), run(hip_lib, prec, (1, 1, 1))
             assert rel(a, want) < TOL[prec], (nz, mode, prec)
             assert rel(a, b) < TOL[prec], (nz, mode, prec)
+
+
+def test_from_the_largest_x(hip_lib):
+    """Complex psi of 176 MiB or more is swept from the largest x down."""
+    n = (96, 512, 256)
+    print(f"[gpu-case] fused z, reversed, {n}", flush=True)
+    p = params(n=n, h=tuple(8.0 / k for k in n), dt=0.002, cutoff=3.0)
+    f = field(p, True)
+    f /= np.sqrt(np.sum(np.abs(f) ** 2) * p.dx * p.dy * p.dz)
+    assert f.nbytes >= 176 << 20
+    out = []
+    for calls in ((3,), (1, 1, 1)):
+        with dbecpy.Solver(hip_lib, p, dbecpy.REAL, dbecpy.FP64) as s:
+            s.set_psi(f)
+            s.set_coupling(60.0, 200.0)
+            for k in calls:
+                s.step(k)
+            out.append(s.get_psi())
+    assert rel(out[0], out[1]) < TOL[dbecpy.FP64]
