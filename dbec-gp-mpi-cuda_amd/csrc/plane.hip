@@ -700,15 +700,16 @@ hipError_t inv(const dbec_ctx *c, const Solves &v, bool phi) {
 // choice must not depend on a tuned or batched launch).  Step times, one pass
 // per kernel against planes, us (FP64 imaginary, mixed imaginary, FP64 real,
 // mixed real; - where the plane does not fit LDS):
-//   16x32x32    32  29  33  31   25  23  26  24
-//   64x64x64    40  36  44  38   33  28  36  30
-//   128x96x80   74  55  86  63   57  43  65  47
-//   96x96x96    73  53  83  61   56  41   -  47
-//   128x128x128 98  71 107  82   83  62   -  69
-//   256x128x128 121 92 163  99  116  83   -  84
+//   16x32x32    31  30  33  31   25  24  26  24
+//   64x64x64    38  34  44  35   33  29  36  30
+//   128x96x80   74  55  82  61   57  43  66  48
+//   96x96x96    72  53  83  60   55  40   -  48
+//   128x128x128 98  72 104  83   82  62   -  69
+//   256x128x128 116 93 163  98  116  83   -  84
+//   48x128x128  64  48  74  53   60  42   -  49
 //   16x128x128  43  37  47  38   51  38   -  43
-//   384x96x96   122 100 165 103 132  93   - 110
-//   512x64x64   105 75 116  88   81  59  80  68
+//   384x96x96   121 94 161 102  132  93   - 110
+//   512x64x64   101 73 105  82   80  60  80  68
 // So large planes need 48 of them or more (one workgroup each: fewer leave
 // most of the chip idle during long launches), and past 256 planes, where the
 // launches run in several rounds and bandwidth counts, only small grids gain.

@@ -37,10 +37,12 @@ namespace {
 constexpr size_t kPiece = size_t(2) << 20;  // bytes of a slot, the largest piece; a field goes in 16 pieces or
 constexpr size_t kPieceMin = size_t(256) << 10;  // more down to this size
 // Device bytes up to which the plain way is kept, in us plain / staged by the
-// caller alone: fetch 128^3 FP64 (16 MB) 940 / 650, 64^3 (2 MB) 122 / 122, 96^3
-// mixed (3.5 MB) 381 / 300; store 128^3 FP64 486 / 580, 96^3 mixed 213 / 315,
-// 80x96x160 complex mixed (9.8 MB) 668 / 574.
-constexpr size_t kFetch64 = size_t(4) << 20, kFetch32 = size_t(1) << 20;
+// caller alone: fetch FP64 128^3 (16 MB) 1010 / 693, 96^3 (6.8 MB) 417 / 402,
+// 96x16x192 complex (4.5 MB) 275 / 358, mixed 96^3 (3.5 MB) 381 / 300, 64^3
+// complex (2 MB) 200 / 189, 96x64x64 phi (1.5 MB) 147 / 149, 64^3 phi (1 MB)
+// 100 / 112; store 128^3 FP64 486 / 580, 96^3 mixed 213 / 315, 80x96x160
+// complex mixed (9.8 MB) 668 / 574.
+constexpr size_t kFetch64 = size_t(6) << 20, kFetch32 = size_t(3) << 19;
 constexpr size_t kStore64 = size_t(32) << 20, kStore32 = size_t(4) << 20;
 constexpr size_t kOneThread = size_t(32) << 20;  // host bytes the caller moves alone
 constexpr int kWorkers = 7, kSlotsPerCall = 16, kMaxSlots = 32;
