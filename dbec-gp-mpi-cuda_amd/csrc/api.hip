@@ -219,10 +219,16 @@ FftArgs fft_args(const dbec_ctx *c, int axis, const Solves &v) {
 }
 
 // The x convolution's arguments; planes: the spectrum rows are in the plane
-// kernels' digit order along y.
-FftArgs xconv_args(const dbec_ctx *c, const Solves &v, bool planes) {
+// kernels' digit order along y; phi: for the standalone calcpsidd2.
+FftArgs xconv_args(const dbec_ctx *c, const Solves &v, bool planes, bool phi = false) {
     FftArgs a = fft_args(c, 0, v);
     a.yq = planes ? (int)(c->Ny / 8) : 0;
+    a.phi_plans = phi;
+    return a;
+}
+FftArgs phi_yargs(const dbec_ctx *c, const Solves &v) {
+    FftArgs a = fft_args(c, 1, v);
+    a.phi_plans = true;
     return a;
 }
 
@@ -232,10 +238,10 @@ FftArgs xconv_args(const dbec_ctx *c, const Solves &v, bool planes) {
 // mu of a 48^3 state by 6e-10 of its value).
 bool phi_planes(const dbec_ctx *c) { return c->planes && c->prec == DBEC_FP64; }
 
-int run_xconv(dbec_ctx *c, const Solves &v, bool planes) {
+int run_xconv(dbec_ctx *c, const Solves &v, bool planes, bool phi = false) {
     const double spec_b = (double)c->Nkz * c->Nx * c->Ny * (double)(2 * real_elem(c));
     const double pq = (double)c->Nkz * (c->Nx / 2 + 1) * (c->Ny / 2 + 1) * real_elem(c);
-    HIPCHK(c, timed(c, "xconv", v.nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, xconv_args(c, v, planes)); }), "xconv");
+    HIPCHK(c, timed(c, "xconv", v.nb * (2 * spec_b + pq), [&] { return launch_xconv(c->Nx, xconv_args(c, v, planes, phi)); }), "xconv");
     return DBEC_OK;
 }
 
@@ -254,9 +260,9 @@ int run_calcpsidd2(dbec_ctx *c) {
         return DBEC_OK;
     }
     HIPCHK(c, timed(c, "zfwd", (double)c->N * psi_elem(c) + spec_b, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }), "zfwd");
-    HIPCHK(c, timed(c, "ypass_fwd", 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }), "ypass");
-    CHK(run_xconv(c, v, false));
-    HIPCHK(c, timed(c, "ypass_inv", 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, fft_args(c, 1, v)); }), "ypass");
+    HIPCHK(c, timed(c, "ypass_fwd", 2 * spec_b, [&] { return launch_ypass(c->Ny, -1, phi_yargs(c, v)); }), "ypass");
+    CHK(run_xconv(c, v, false, true));
+    HIPCHK(c, timed(c, "ypass_inv", 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, phi_yargs(c, v)); }), "ypass");
     HIPCHK(c, timed(c, "zinv", spec_b + nre, [&] { return launch_zinv(c->Nz, fft_args(c, 2, v)); }), "zinv");
     const double fb = 2.0 * (double)(c->Ny * c->Nz + c->Nx * c->Nz + c->Nx * c->Ny) * real_elem(c);
     HIPCHK(c, timed(c, "facefix", fb, [&] {
@@ -421,7 +427,7 @@ Cx cx_div(Cx a, Cx b) {
 
 void free_buffers(dbec_ctx *c) {
     Buffers &b = c->b;
-    void *ptrs[] = {b.psi, b.spec, b.phi, b.potddq, b.rows, b.red, b.scal, b.coef, b.wgt, b.sq,
+    void *ptrs[] = {b.psi, b.spec, b.phi, b.potddq, b.rows, b.scal, b.coef, b.wgt, b.sq,
                     b.tw[0], b.tw[1], b.tw[2], b.twf[0], b.twf[1], b.twf[2]};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);

@@ -448,9 +448,11 @@ template <bool B, int N>
 using PlanIf = std::conditional_t<B, FftPlanB<N>, FftPlan<N>>;
 template <typename R>
 constexpr bool kF32 = std::is_same<R, float>::value || std::is_same<R, cpx<float>>::value;
-// x convolution, y passes (spectrum in R) and the fused inverse z pass (psi in P)
+// x convolution, y passes (spectrum in R) and the fused inverse z pass (psi in P).
+// The standalone potential in FP32 runs with FftPlan in every pass
+// (FftArgs::phi_plans): its rounding shows in mu and E, which are FP64.
 template <int N, typename R>
-using XPlan = PlanIf<kF32<R> || (N != 192 && N != 384 && N != 512), N>;
+using XPlan = PlanIf<(N == 192 || N == 384 || N == 512) ? kF32<R> : (N == 48 || N == 80 || N == 96 || N == 160 || N == 320), N>;
 template <int N, typename R>
 using YPlan = PlanIf<kF32<R> ? N == 384 : N == 320, N>;
 template <int N, typename P>

@@ -458,11 +458,10 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
 // With v.fold == 2 (the forward z pass ran fused with the last z sweep) the
 // first workgroup of each solve's forward pass also forms the last step's
 // norm from the z sweep's column partials, for the x convolution and calcnu.
-template <int N, int DIR, typename R, int LM>
-__global__ void __launch_bounds__((FftTile<YPlan<N, R>, LM>::WG))
+template <int N, int DIR, typename R, int LM, typename Pl>
+__global__ void __launch_bounds__((FftTile<Pl, LM>::WG))
 k_ypass(Solves v, long nlines, const cpx<R> *__restrict__ twg, const double *__restrict__ wx, int tiles, int Nx) {
-    constexpr int L = FftTile<YPlan<N, R>, LM>::L, WG = FftTile<YPlan<N, R>, LM>::WG;
-    using Pl = YPlan<N, R>;
+    constexpr int L = FftTile<Pl, LM>::L, WG = FftTile<Pl, LM>::WG;
     __shared__ cpx<R> buf[N * (L + 1)];
     __shared__ cpx<R> tw[N];
     cpx<R> *__restrict__ spec = reinterpret_cast<cpx<R> *>(solve_at(v).spec);
@@ -502,12 +501,11 @@ k_ypass(Solves v, long nlines, const cpx<R> *__restrict__ twg, const double *__r
 // PL: the spectrum's rows come from the plane kernels (digit order along y,
 // yq = Ny / 8; the norm from one partial per x with v.fold == 3); a template
 // parameter, so the other grids' kernel stays as lean as without it.
-template <int N, typename R, int LM, bool PL>
-__global__ void __launch_bounds__((FftTile<XPlan<N, R>, LM>::WG))
+template <int N, typename R, int LM, bool PL, typename Pl>
+__global__ void __launch_bounds__((FftTile<Pl, LM>::WG))
 k_xconv(Solves v, const R *__restrict__ potddq, int Ny, const cpx<R> *__restrict__ twg, const double *__restrict__ wx,
         int yq) {
-    constexpr int L = FftTile<XPlan<N, R>, LM>::L, WG = FftTile<XPlan<N, R>, LM>::WG;
-    using Pl = XPlan<N, R>;
+    constexpr int L = FftTile<Pl, LM>::L, WG = FftTile<Pl, LM>::WG;
     constexpr int T = Pl::T, K = N / T;  // x values per thread
     static_assert(L * T == WG, "xconv tile");
     constexpr int NXH = N / 2 + 1;
@@ -907,14 +905,16 @@ struct FftLaunchImpl {
     // FP32 spectra use tiles twice as wide, so every strided access still
     // moves 128-256 contiguous bytes.
 
-    template <typename R, int LM>
+    template <typename R, int LM, typename Pl = YPlan<N, R>>
     static hipError_t ypass_t(int dir, const FftArgs &a) {
-        using Tl = FftTile<YPlan<N, R>, LM>;
+        if constexpr (kF32<R> && !std::is_same<Pl, FftPlan<N>>::value)
+            if (a.phi_plans) return ypass_t<R, LM, FftPlan<N>>(dir, a);
+        using Tl = FftTile<Pl, LM>;
         const long nlines = a.Nkz * a.Nx;
         dim3 grid((unsigned)((nlines + Tl::L - 1) / Tl::L), (unsigned)a.v.nb), block(Tl::WG);
         auto *tw = static_cast<const cpx<R> *>(a.tw);
-        if (dir < 0) k_ypass<N, -1, R, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
-        else k_ypass<N, +1, R, LM><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
+        if (dir < 0) k_ypass<N, -1, R, LM, Pl><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
+        else k_ypass<N, +1, R, LM, Pl><<<grid, block, 0, a.stream>>>(a.v, nlines, tw, a.wx, a.tiles, (int)a.Nx);
         return hipGetLastError();
     }
     static hipError_t ypass(int dir, const FftArgs &a) {
@@ -924,13 +924,15 @@ struct FftLaunchImpl {
         return two ? ypass_t<double, 2>(dir, a) : ypass_t<double, 1>(dir, a);
     }
 
-    template <typename R, int LM>
+    template <typename R, int LM, typename Pl = XPlan<N, R>>
     static hipError_t xconv_t(const FftArgs &a) {
-        using Tl = FftTile<XPlan<N, R>, LM>;
+        if constexpr (kF32<R> && !std::is_same<Pl, FftPlan<N>>::value)
+            if (a.phi_plans) return xconv_t<R, LM, FftPlan<N>>(a);
+        using Tl = FftTile<Pl, LM>;
         const int ytiles = (int)((a.Ny + Tl::L - 1) / Tl::L);
         dim3 grid((unsigned)(a.Nkz * ytiles), (unsigned)a.v.nb), block(Tl::WG);
         const auto launch = [&](auto planes) {
-            k_xconv<N, R, LM, decltype(planes)::value><<<grid, block, 0, a.stream>>>(
+            k_xconv<N, R, LM, decltype(planes)::value, Pl><<<grid, block, 0, a.stream>>>(
                 a.v, static_cast<const R *>(a.potddq), (int)a.Ny, static_cast<const cpx<R> *>(a.tw), a.wx, a.yq);
         };
         if (a.yq) launch(std::true_type{});

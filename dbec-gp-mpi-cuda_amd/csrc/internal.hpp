@@ -24,14 +24,15 @@ namespace dbec {
 //                           dipolar kernel is even in every k component, so a
 //                           quarter table indexed by |k| holds it exactly;
 //                           rows ky in the order of pot_row
-//   rows   [2][Ny][Nx]      double: per-row z integrals for the reductions
+//   rows   2 Nx Ny          double: the partial sums of the norm (the z sweep's
+//                           [tile][x], the plane kernels' [x]) and of the
+//                           observables (per workgroup)
 struct Buffers {
     void *psi = nullptr;
     void *spec = nullptr;
     void *phi = nullptr;
     void *potddq = nullptr;
     double *rows = nullptr;
-    double *red = nullptr;   // reduction scratch (>= 4 * (Nx + Ny + Nz) doubles)
     double *scal = nullptr;  // device scalars, see SC_* below
     double *coef = nullptr;  // CN coefficients and carry multipliers (CoefLayout), real or complex, FP64
                              // in both precisions (the mixed sweeps round them to FP32 in LDS)
@@ -174,6 +175,9 @@ struct FftArgs {
     // x convolution: > 0 where slot s of a spectrum row holds the y frequency
     // s / yq + 8 (s % yq) (the plane kernels' digit order), 0: s itself
     int yq = 0;
+    // y passes and x convolution in FP32 with the plans of the z passes, as the
+    // standalone calcpsidd2 takes them
+    bool phi_plans = false;
 };
 // Each returns hipSuccess or an error; `n` is the transformed length.
 hipError_t launch_zfwd(long n, const FftArgs &a);    // |psi|^2 -> spec (R2C along z)

@@ -1,4 +1,4 @@
-// ops.hip - pointwise, sweep and reduction kernels of the split step.
+// ops.hip - pointwise kernels, sweeps and the norm of the split step.
 //
 // Reference aliases: imag3d.cu = src/imag3d-mpicuda/imag3d-mpicuda.cu,
 // real3d.cu = src/real3d-mpicuda/real3d-mpicuda.cu, diffint.cu =

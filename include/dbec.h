@@ -133,7 +133,7 @@ int dbec_density(dbec_ctx *ctx, int kind, long outstpx, long outstpy, long outst
  * loops, harnesses that forbid hipMalloc).  The same extracts, equal to
  * dbec_density's bit for bit; the weighted sums and the sampled values live
  * in a fixed device array of DBEC_NOALLOC_SCRATCH_BYTES per GPU, held until
- * the process ends, instead of a buffer allocated per call.  An extract whose
+ * the process ends, instead of the context's spectrum buffer.  An extract whose
  * sums and samples need more fails with DBEC_EINVAL and a message: every 1-D
  * and 2-D kind fits at every supported grid, the sampled 3-D extracts up to
  * 1048576 values.  All calls on one GPU share its array and the call ends
