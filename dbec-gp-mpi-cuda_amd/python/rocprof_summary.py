@@ -51,7 +51,7 @@ def template_args(full, start):
 
 def short_name(full):
     """Kernel name as bench.py reports it, or None for kernels outside the step."""
-    m = re.search(r"dbec::(k_\w+)", full)
+    m = re.search(r"dbec::(?:\(anonymous namespace\)::)?(k_\w+)", full)
     if not m:
         return "copy" if "copyBuffer" in full else None
     k = m.group(1)
@@ -97,7 +97,7 @@ def cmd_stats(args):
 def first_targ(full):
     """The first template argument of a dbec kernel (its transform length or
     storage type), or ''."""
-    m = re.search(r"dbec::(k_\w+)", full)
+    m = re.search(r"dbec::(?:\(anonymous namespace\)::)?(k_\w+)", full)
     if not m or full[m.end():m.end() + 1] != "<":
         return ""
     targs = template_args(full, m.end())
