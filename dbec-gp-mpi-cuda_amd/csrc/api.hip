@@ -246,7 +246,7 @@ int run_xconv(dbec_ctx *c, const Solves &v, bool planes, bool phi = false) {
 }
 
 // calcpsidd2 of the context's own psi (no pending scale): |psi|^2 -> half
-// spectrum -> * potdd -> phi, then the face copies.
+// spectrum -> * potdd -> phi with the face copies.
 int run_calcpsidd2(dbec_ctx *c) {
     const Solves v = solve_ref(c, false);
     const double ce = (double)(2 * real_elem(c));
@@ -264,10 +264,6 @@ int run_calcpsidd2(dbec_ctx *c) {
     CHK(run_xconv(c, v, false, true));
     HIPCHK(c, timed(c, "ypass_inv", 2 * spec_b, [&] { return launch_ypass(c->Ny, +1, phi_yargs(c, v)); }), "ypass");
     HIPCHK(c, timed(c, "zinv", spec_b + nre, [&] { return launch_zinv(c->Nz, fft_args(c, 2, v)); }), "zinv");
-    const double fb = 2.0 * (double)(c->Ny * c->Nz + c->Nx * c->Nz + c->Nx * c->Ny) * real_elem(c);
-    HIPCHK(c, timed(c, "facefix", fb, [&] {
-               return launch_facefix(c->stream, c->b.phi, c->prec == DBEC_MIXED, c->Nx, c->Ny, c->Nz);
-           }), "facefix");
     c->phi_valid = true;
     return DBEC_OK;
 }

@@ -13,40 +13,6 @@
 namespace dbec {
 
 // ---------------------------------------------------------------------------
-// Periodic face copies of the dipolar potential after the inverse transform
-// (calcpsidd2_kernel2a/2b, imag3d.cu:1491-1505, 1591-1625, at one rank):
-//   A: phi[Nx-1][j][k] = phi[0][j][k]  (j < Ny-1, k < Nz-1)
-//   B: phi[i][Ny-1][k] = phi[i][0][k]  (i < Nx-1, k < Nz-1)
-//   C: phi[i][j][Nz-1] = phi[i][j][0]  (i < Nx-1, j < Ny-1)
-// No part reads an element another part writes, so one launch is race free.
-template <typename R>
-__global__ void k_facefix(R *__restrict__ phi, int Nx, int Ny, int Nz) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nA = (long)(Ny - 1) * (Nz - 1), nB = (long)(Nx - 1) * (Nz - 1), nC = (long)(Nx - 1) * (Ny - 1);
-    const long NyNz = (long)Ny * Nz;
-    if (t < nA) {
-        const long j = t / (Nz - 1), k = t % (Nz - 1);
-        phi[(long)(Nx - 1) * NyNz + j * Nz + k] = phi[j * Nz + k];
-    }
-    if (t < nB) {
-        const long i = t / (Nz - 1), k = t % (Nz - 1);
-        phi[i * NyNz + (long)(Ny - 1) * Nz + k] = phi[i * NyNz + k];
-    }
-    if (t < nC) {
-        const long i = t / (Ny - 1), j = t % (Ny - 1);
-        phi[i * NyNz + j * Nz + Nz - 1] = phi[i * NyNz + j * Nz];
-    }
-}
-
-hipError_t launch_facefix(hipStream_t s, void *phi, bool fp32, long Nx, long Ny, long Nz) {
-    long n = std::max((Ny - 1) * (Nz - 1), std::max((Nx - 1) * (Nz - 1), (Nx - 1) * (Ny - 1)));
-    dim3 block(256), grid((unsigned)((n + 255) / 256));
-    if (fp32) k_facefix<float><<<grid, block, 0, s>>>(static_cast<float *>(phi), (int)Nx, (int)Ny, (int)Nz);
-    else k_facefix<double><<<grid, block, 0, s>>>(static_cast<double *>(phi), (int)Nx, (int)Ny, (int)Nz);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // calcnu (calcnu_kernel imag3d.cu:1759-1783; real3d.cu:1856-1883), with psi
 // read as psi * scale when a renormalisation is pending (imaginary time).  The
 // trap is recomputed from the grid (nu_device.hpp).

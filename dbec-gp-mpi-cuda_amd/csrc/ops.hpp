@@ -30,7 +30,6 @@ struct CoefLayout {
     long size() const { return 2 * tot + 4 * totn; }
 };
 
-hipError_t launch_facefix(hipStream_t s, void *phi, bool fp32, long Nx, long Ny, long Nz);
 hipError_t launch_calcnu(hipStream_t s, const dbec_ctx *c, const double *scale);
 hipError_t launch_scale(hipStream_t s, const dbec_ctx *c, const double *scale);
 // *p = v on the stream (a one-thread kernel: also valid under graph capture)
