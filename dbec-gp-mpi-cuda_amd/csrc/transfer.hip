@@ -142,7 +142,8 @@ public:
                 std::lock_guard<std::mutex> lk(mu_);
                 tasks_.push_back(t);
                 try {
-                    while ((int)threads_.size() < kWorkers) threads_.emplace_back([this] { loop(); });
+                    while ((int)threads_.size() < kWorkers)
+                        threads_.emplace_back([this, g = generation_] { loop(g); });
                 } catch (const std::exception &) {  // fewer threads do the same work
                 }
             }
@@ -169,9 +170,11 @@ public:
     ~Workers() { stop(); }
 
 private:
-    void loop() {
+    // born: generation_ when the thread was made.  It may get the lock for the
+    // first time only after stop() has passed (the caller moves every piece
+    // itself then), and must end all the same.
+    void loop(unsigned born) {
         std::unique_lock<std::mutex> lk(mu_);
-        const unsigned born = generation_;
         while (born == generation_) {
             if (tasks_.empty()) {
                 cv_.wait(lk);

@@ -1,0 +1,282 @@
+// Host paths of libdbec_hip without a device: this program defines the HIP
+// entry points that the library imports (the dynamic linker prefers the
+// program's own), with device memory in host memory, copies to and from pinned
+// memory left pending until somebody waits for them, and kernels that do
+// nothing.  test_host_paths.py builds it and runs one scenario a
+// process; a scenario ends with "ok", or with what went wrong.
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+#include <pthread.h>
+#include <unistd.h>
+
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <map>
+#include <mutex>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "dbec.h"
+
+namespace {
+
+std::atomic<int> thread_delay_us{0};
+std::atomic<int> pinned_live{0}, freed_in_flight{0};
+
+struct Op {
+    void *dst;
+    const void *src;
+    size_t n;
+};
+struct Stream {
+    int device;
+    std::deque<Op> ops;
+    size_t queued = 0, ended = 0;
+};
+struct Event {
+    int device;
+    Stream *stream = nullptr;
+    size_t at = 0;
+};
+struct Fake {
+    std::mutex mu;
+    std::map<char *, size_t> pinned;
+    std::set<Stream *> streams;
+};
+Fake &fake() {  // also reached from the library's initialisers, before this program's
+    static Fake *f = new Fake;
+    return *f;
+}
+thread_local int device = 0;
+struct Config {
+    dim3 g, b;
+    size_t shm;
+    hipStream_t s;
+};
+thread_local Config config;
+
+bool is_pinned(const void *p) {
+    auto &m = fake().pinned;
+    auto it = m.upper_bound(const_cast<char *>(static_cast<const char *>(p)));
+    if (it == m.begin()) return false;
+    --it;
+    return static_cast<const char *>(p) < it->first + it->second;
+}
+void drain(Stream *s, size_t upto) {  // mu held
+    while (!s->ops.empty() && s->ended < upto) {
+        const Op o = s->ops.front();
+        s->ops.pop_front();
+        std::memcpy(o.dst, o.src, o.n);
+        ++s->ended;
+    }
+}
+
+}  // namespace
+
+// Threads start as late as the scenario asks for, as they do on a busy host.
+extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
+    using Fn = int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *);
+    static const Fn real = reinterpret_cast<Fn>(dlsym(RTLD_NEXT, "pthread_create"));
+    struct Late {
+        void *(*f)(void *);
+        void *arg;
+    };
+    auto *l = static_cast<Late *>(std::malloc(sizeof(Late)));
+    *l = {f, arg};
+    return real(t, a, [](void *p) -> void * {
+        const Late l = *static_cast<Late *>(p);
+        std::free(p);
+        if (const int us = thread_delay_us) usleep((useconds_t)us);
+        return l.f(l.arg);
+    }, l);
+}
+
+extern "C" {
+
+struct uint3_;
+void **__hipRegisterFatBinary(const void *) {
+    static void *module = nullptr;
+    return &module;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, uint3_ *, uint3_ *, dim3 *, dim3 *,
+                           int *) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t shm, hipStream_t s) {
+    config = {g, b, shm, s};
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shm, hipStream_t *s) {
+    *g = config.g, *b = config.b, *shm = config.shm, *s = config.s;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+
+hipError_t hipGetDeviceCount(int *n) { return *n = 16, hipSuccess; }
+hipError_t hipGetDevice(int *d) { return *d = device, hipSuccess; }
+hipError_t hipSetDevice(int d) {
+    if (d < 0 || d >= 16) return hipErrorInvalidDevice;
+    return device = d, hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t *fr, size_t *tot) { return *fr = *tot = size_t(256) << 30, hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipMalloc(void **p, size_t n) {
+    return (*p = std::calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void *p) { return std::free(p), hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *) {
+    static char *mem = static_cast<char *>(std::calloc(DBEC_NOALLOC_SCRATCH_BYTES, 1));
+    return *p = mem, hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
+    std::lock_guard<std::mutex> lk(fake().mu);
+    fake().pinned[static_cast<char *>(*p)] = n;
+    ++pinned_live;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    for (Stream *s : fake().streams)
+        for (const Op &o : s->ops)
+            if (o.dst == p || o.src == p) {
+                ++freed_in_flight;
+                return hipSuccess;  // the memory stays, so the pending copy is harmless here
+            }
+    fake().pinned.erase(static_cast<char *>(p));
+    --pinned_live;
+    return std::free(p), hipSuccess;
+}
+hipError_t hipStreamCreate(hipStream_t *s) {
+    auto *n = new Stream;
+    n->device = device;
+    std::lock_guard<std::mutex> lk(fake().mu);
+    fake().streams.insert(n);
+    return *s = reinterpret_cast<hipStream_t>(n), hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t h) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    auto *s = reinterpret_cast<Stream *>(h);
+    return drain(s, s->queued), hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t h) {
+    (void)hipStreamSynchronize(h);
+    std::lock_guard<std::mutex> lk(fake().mu);
+    fake().streams.erase(reinterpret_cast<Stream *>(h));
+    return delete reinterpret_cast<Stream *>(h), hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t h) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    auto *s = reinterpret_cast<Stream *>(h);
+    const bool to = is_pinned(dst), from = is_pinned(src);
+    s->ops.push_back({dst, src, n});
+    ++s->queued;
+    if (!to && !from) drain(s, s->queued);  // pageable: the call waits
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t h) {
+    (void)hipStreamSynchronize(h);
+    return std::memset(p, v, n), hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *ev, unsigned) {
+    auto *n = new Event;
+    n->device = device;
+    return *ev = reinterpret_cast<hipEvent_t>(n), hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *ev) { return hipEventCreateWithFlags(ev, 0); }
+hipError_t hipEventDestroy(hipEvent_t ev) { return delete reinterpret_cast<Event *>(ev), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t ev, hipStream_t h) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    auto *e = reinterpret_cast<Event *>(ev);
+    auto *s = reinterpret_cast<Stream *>(h);
+    if (e->device != s->device) return hipErrorInvalidHandle;
+    e->stream = s;
+    e->at = s->queued;
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t ev) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    auto *e = reinterpret_cast<Event *>(ev);
+    if (e->stream) drain(e->stream, e->at);
+    return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t ev) { return hipEventSynchronize(ev); }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t ev, unsigned) { return hipEventSynchronize(ev); }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *) { return hipErrorNotSupported; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *, hipGraph_t, hipGraphNode_t *, char *, size_t) {
+    return hipErrorNotSupported;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+
+}  // extern "C"
+
+namespace {
+
+#define CHECK(c)                                                                       \
+    do {                                                                               \
+        if (!(c)) {                                                                    \
+            std::printf("line %d: %s\n", __LINE__, #c);                                \
+            std::fflush(stdout);                                                       \
+            std::_Exit(1);                                                             \
+        }                                                                              \
+    } while (0)
+
+dbec_ctx *create(long nx, long ny, long nz, dbec_mode mode, dbec_prec prec, int dev = 0) {
+    dbec_params p;
+    std::memset(&p, 0, sizeof p);
+    p.nx = nx, p.ny = ny, p.nz = nz;
+    p.dx = p.dy = p.dz = 0.2;
+    p.dt = 0.002;
+    p.vgamma = p.vnu = p.vlambda = 1.0;
+    p.cutoff = 4.0;
+    p.par = 2.0;
+    p.device = dev;
+    dbec_ctx *c = nullptr;
+    CHECK(dbec_create(&p, mode, prec, nullptr, &c) == DBEC_OK);
+    return c;
+}
+
+void round_trip(dbec_ctx *c, size_t n, int seed) {
+    std::vector<double> a(n), b(n, -1.0);
+    for (size_t i = 0; i < n; ++i) a[i] = (double)((i * 2654435761u + (size_t)seed * 40503u) & 0xfffff);  // floats hold it
+    CHECK(dbec_set_psi(c, a.data()) == DBEC_OK);
+    CHECK(dbec_get_psi(c, b.data()) == DBEC_OK);
+    CHECK(std::memcmp(a.data(), b.data(), n * sizeof(double)) == 0);
+}
+
+// 40 MiB of host doubles: past the bound from which the pool's threads help
+constexpr long BX = 160, BY = 128, BZ = 128;
+constexpr size_t BIG = 2 * size_t(BX * BY * BZ);
+
+// The last context ends before the threads that its transfer started have run.
+void late_threads() {
+    for (int k = 0; k < 3; ++k) {
+        dbec_ctx *c = create(BX, BY, BZ, DBEC_REAL, DBEC_FP64);
+        thread_delay_us = 400000;
+        round_trip(c, BIG, k);
+        CHECK(dbec_destroy(c) == DBEC_OK);
+        thread_delay_us = 0;
+        CHECK(pinned_live == 0);
+    }
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    alarm(100);
+    const std::string s = argc > 1 ? argv[1] : "";
+    if (s == "late_threads") late_threads();
+    else return std::printf("no such scenario\n"), 2;
+    std::printf("ok\n");
+    return 0;
+}

@@ -1,0 +1,36 @@
+"""Host paths of the library that need no device: transfers through the staging
+slots and the pool of threads.  host_paths.cpp stands in for the HIP runtime
+(its entry points come before the real ones in symbol lookup) and runs one
+scenario a process."""
+import os
+import subprocess
+
+import pytest
+
+import dbecpy
+from conftest import PKG, REPO
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    if not os.path.exists(dbecpy.HIP_LIB):
+        pytest.fail(f"{dbecpy.HIP_LIB} is not built; run __graft_entry__.build()")
+    exe = str(tmp_path_factory.mktemp("host_paths") / "host_paths")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(REPO, "include"), "-rdynamic", "-o", exe,
+                    os.path.join(REPO, "tests", "host_paths.cpp"), "-L" + PKG, "-ldbec_hip", "-Wl,-rpath," + PKG,
+                    "-pthread", "-ldl"], check=True)
+    return exe
+
+
+def run(program, scenario, **env):
+    keep = {k: v for k, v in os.environ.items() if not k.startswith("DBEC_")}
+    r = subprocess.run([program, scenario], env={**keep, "DBEC_AUTOTUNE": "0", **env}, capture_output=True, text=True,
+                       timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout, r.stderr[-1000:])
+
+
+def test_last_context_ends_before_the_pool_has_started(program):
+    """The caller may finish a transfer before a thread it started has run; the
+    end of the last context then still has to end that thread."""
+    run(program, "late_threads")
