@@ -22,7 +22,6 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
-#include <deque>
 #include <functional>
 #include <memory>
 #include <mutex>
@@ -135,16 +134,17 @@ struct Task {
 
 class Workers {
 public:
-    // Runs the task on the pool's threads and this one, until every piece is done.
-    void run(const std::shared_ptr<Task> &t, bool alone) {
+    // Runs the task on the pool's threads and this one, until every piece is
+    // done.  Never throws: copies may be on their way to the caller's slots.
+    void run(const std::shared_ptr<Task> &t, bool alone) noexcept {
         if (!alone) {
             {
                 std::lock_guard<std::mutex> lk(mu_);
-                tasks_.push_back(t);
                 try {
+                    tasks_.push_back(t);
                     while ((int)threads_.size() < kWorkers)
                         threads_.emplace_back([this, g = generation_] { loop(g); });
-                } catch (const std::exception &) {  // fewer threads do the same work
+                } catch (const std::exception &) {  // fewer threads, or the caller alone, do the same work
                 }
             }
             cv_.notify_all();
@@ -184,30 +184,36 @@ private:
             lk.unlock();
             t->take_all();
             lk.lock();
-            if (!tasks_.empty() && tasks_.front() == t) tasks_.pop_front();
+            if (!tasks_.empty() && tasks_.front() == t) tasks_.erase(tasks_.begin());
         }
     }
     std::mutex mu_;
     std::condition_variable cv_;
-    std::deque<std::shared_ptr<Task>> tasks_;
+    std::vector<std::shared_ptr<Task>> tasks_;
     std::vector<std::thread> threads_;
     unsigned generation_ = 0;
 };
 
 // Never destroyed: a thread of the host program may still be in a call while
-// the process ends.
+// the process ends.  In static storage: the end of a context must not throw.
 Workers &workers() {
-    static Workers *w = new Workers;
+    alignas(Workers) static unsigned char mem[sizeof(Workers)];
+    static Workers *w = new (mem) Workers;
     return *w;
 }
 
+// The task of n pieces; `work` outlives its run.  Made before the transfer's
+// first copy, after which nothing may throw.
 template <typename F>
-hipError_t run_workers(int device, size_t n, size_t host_bytes, F &&work) {
+std::shared_ptr<Task> make_task(int device, size_t n, F &work) {
     auto t = std::make_shared<Task>();
     t->n = n;
     t->device = device;
     Task *raw = t.get();
     t->work = [&work, raw](size_t i) { return work(i, raw->err); };
+    return t;
+}
+hipError_t run_task(const std::shared_ptr<Task> &t, size_t host_bytes) {
     workers().run(t, host_bytes <= kOneThread);
     return (hipError_t)t->err.load();
 }
@@ -242,26 +248,27 @@ hipError_t fetch_staged(const dbec_ctx *c, double *dst, const char *src, size_t 
         if (e == hipSuccess) queued[i].store(1, std::memory_order_release);
         return e;
     };
+    // the worker of piece i queues piece i + R into the slot it has emptied:
+    // a piece waits only for one that a worker has taken before it
+    const auto piece = [&](size_t i, std::atomic<int> &err) {
+        if (!wait_queued(queued, i, err)) return hipSuccess;
+        const Slot &s = slots[i % R];
+        hipError_t r = hipEventSynchronize(s.ev);
+        if (r != hipSuccess) return r;
+        double *out = dst + i * pc.per;
+        const size_t m = pc.len(i);
+        if (f32) {
+            const float *in = static_cast<const float *>(s.mem);
+            for (size_t k = 0; k < m; ++k) out[k] = (double)in[k];
+        } else {
+            std::memcpy(out, s.mem, m * sizeof(double));
+        }
+        return i + R < pc.count ? queue(i + R) : hipSuccess;
+    };
+    const std::shared_ptr<Task> task = make_task(c->device, pc.count, piece);
     hipError_t e = hipSuccess;
     for (size_t i = 0; i < std::min(R, pc.count) && e == hipSuccess; ++i) e = queue(i);
-    if (e == hipSuccess)
-        // the worker of piece i queues piece i + R into the slot it has emptied:
-        // a piece waits only for one that a worker has taken before it
-        e = run_workers(c->device, pc.count, n * sizeof(double), [&](size_t i, std::atomic<int> &err) {
-            if (!wait_queued(queued, i, err)) return hipSuccess;
-            const Slot &s = slots[i % R];
-            hipError_t r = hipEventSynchronize(s.ev);
-            if (r != hipSuccess) return r;
-            double *out = dst + i * pc.per;
-            const size_t m = pc.len(i);
-            if (f32) {
-                const float *in = static_cast<const float *>(s.mem);
-                for (size_t k = 0; k < m; ++k) out[k] = (double)in[k];
-            } else {
-                std::memcpy(out, s.mem, m * sizeof(double));
-            }
-            return i + R < pc.count ? queue(i + R) : hipSuccess;
-        });
+    if (e == hipSuccess) e = run_task(task, n * sizeof(double));
     const hipError_t w = hipStreamSynchronize(c->stream);
     return e != hipSuccess ? e : w;
 }
@@ -271,7 +278,7 @@ hipError_t store_staged(const dbec_ctx *c, char *dst, const double *src, size_t 
     const Pieces pc(n, el);
     const size_t R = slots.size();
     Flags queued(pc.count);
-    const hipError_t e = run_workers(c->device, pc.count, n * sizeof(double), [&](size_t i, std::atomic<int> &err) {
+    const auto piece = [&](size_t i, std::atomic<int> &err) {
         Slot &s = slots[i % R];
         if (i >= R) {  // the slot's last copy has left it
             if (!wait_queued(queued, i - R, err)) return hipSuccess;
@@ -290,7 +297,8 @@ hipError_t store_staged(const dbec_ctx *c, char *dst, const double *src, size_t 
         if (r == hipSuccess) r = hipEventRecord(s.ev, c->stream);
         if (r == hipSuccess) queued[i].store(1, std::memory_order_release);
         return r;
-    });
+    };
+    const hipError_t e = run_task(make_task(c->device, pc.count, piece), n * sizeof(double));
     const hipError_t w = hipStreamSynchronize(c->stream);
     return e != hipSuccess ? e : w;
 }
@@ -307,7 +315,7 @@ hipError_t staged(const dbec_ctx *c, size_t n, size_t el, size_t plain, F &&run,
         if (slots.empty()) return hipSuccess;
         done = true;
         e = run(slots);
-    } catch (const std::bad_alloc &) {  // before the first copy: the plain way
+    } catch (const std::bad_alloc &) {  // only ever before the first copy: the plain way
         done = false;
     }
     give_back(slots);

@@ -16,6 +16,7 @@
 #include <deque>
 #include <map>
 #include <mutex>
+#include <new>
 #include <set>
 #include <string>
 #include <vector>
@@ -24,8 +25,16 @@
 
 namespace {
 
+thread_local int in_fake = 0;              // allocations of the stand-in itself never fail
+std::atomic<bool> short_of_memory{false};  // allocations fail while a fetched piece is pending
+std::atomic<int> pending_fetches{0};
 std::atomic<int> thread_delay_us{0};
 std::atomic<int> pinned_live{0}, freed_in_flight{0};
+
+struct Enter {
+    Enter() { ++in_fake; }
+    ~Enter() { --in_fake; }
+};
 
 struct Op {
     void *dst;
@@ -71,11 +80,20 @@ void drain(Stream *s, size_t upto) {  // mu held
         const Op o = s->ops.front();
         s->ops.pop_front();
         std::memcpy(o.dst, o.src, o.n);
+        if (is_pinned(o.dst)) --pending_fetches;
         ++s->ended;
     }
 }
 
 }  // namespace
+
+void *operator new(size_t n) {
+    if (!in_fake && short_of_memory && pending_fetches > 0) throw std::bad_alloc();
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 // Threads start as late as the scenario asks for, as they do on a busy host.
 extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
@@ -135,6 +153,7 @@ hipError_t hipGetSymbolAddress(void **p, const void *) {
     return *p = mem, hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    Enter in;
     if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
     std::lock_guard<std::mutex> lk(fake().mu);
     fake().pinned[static_cast<char *>(*p)] = n;
@@ -142,6 +161,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     return hipSuccess;
 }
 hipError_t hipHostFree(void *p) {
+    Enter in;
     std::lock_guard<std::mutex> lk(fake().mu);
     for (Stream *s : fake().streams)
         for (const Op &o : s->ops)
@@ -154,6 +174,7 @@ hipError_t hipHostFree(void *p) {
     return std::free(p), hipSuccess;
 }
 hipError_t hipStreamCreate(hipStream_t *s) {
+    Enter in;
     auto *n = new Stream;
     n->device = device;
     std::lock_guard<std::mutex> lk(fake().mu);
@@ -161,20 +182,24 @@ hipError_t hipStreamCreate(hipStream_t *s) {
     return *s = reinterpret_cast<hipStream_t>(n), hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t h) {
+    Enter in;
     std::lock_guard<std::mutex> lk(fake().mu);
     auto *s = reinterpret_cast<Stream *>(h);
     return drain(s, s->queued), hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t h) {
     (void)hipStreamSynchronize(h);
+    Enter in;
     std::lock_guard<std::mutex> lk(fake().mu);
     fake().streams.erase(reinterpret_cast<Stream *>(h));
     return delete reinterpret_cast<Stream *>(h), hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t h) {
+    Enter in;
     std::lock_guard<std::mutex> lk(fake().mu);
     auto *s = reinterpret_cast<Stream *>(h);
     const bool to = is_pinned(dst), from = is_pinned(src);
+    if (to) ++pending_fetches;
     s->ops.push_back({dst, src, n});
     ++s->queued;
     if (!to && !from) drain(s, s->queued);  // pageable: the call waits
@@ -185,6 +210,7 @@ hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t h) {
     return std::memset(p, v, n), hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *ev, unsigned) {
+    Enter in;
     auto *n = new Event;
     n->device = device;
     return *ev = reinterpret_cast<hipEvent_t>(n), hipSuccess;
@@ -201,6 +227,7 @@ hipError_t hipEventRecord(hipEvent_t ev, hipStream_t h) {
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t ev) {
+    Enter in;
     std::lock_guard<std::mutex> lk(fake().mu);
     auto *e = reinterpret_cast<Event *>(ev);
     if (e->stream) drain(e->stream, e->at);
@@ -270,12 +297,33 @@ void late_threads() {
     }
 }
 
+// No memory is to be had once the first pieces are on their way.
+void memory() {
+    for (int big = 0; big < 2; ++big)
+        for (dbec_prec prec : {DBEC_FP64, DBEC_MIXED}) {
+            const long nx = big ? BX : 48;  // 40 and 12 MiB of host doubles
+            const size_t n = 2 * size_t(nx * BY * BZ);
+            dbec_ctx *c = create(nx, BY, BZ, DBEC_REAL, prec);
+            std::vector<double> a(n), b(n, -1.0);
+            for (size_t i = 0; i < n; ++i) a[i] = (double)(i & 0xffff);
+            CHECK(dbec_set_psi(c, a.data()) == DBEC_OK);
+            short_of_memory = true;
+            CHECK(dbec_get_psi(c, b.data()) == DBEC_OK);
+            CHECK(freed_in_flight == 0);
+            short_of_memory = false;
+            CHECK(std::memcmp(a.data(), b.data(), n * sizeof(double)) == 0);
+            CHECK(dbec_destroy(c) == DBEC_OK);
+            CHECK(pinned_live == 0);
+        }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     alarm(100);
     const std::string s = argc > 1 ? argv[1] : "";
     if (s == "late_threads") late_threads();
+    else if (s == "memory") memory();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

@@ -34,3 +34,9 @@ def test_last_context_ends_before_the_pool_has_started(program):
     """The caller may finish a transfer before a thread it started has run; the
     end of the last context then still has to end that thread."""
     run(program, "late_threads")
+
+
+def test_no_memory_during_a_fetch(program):
+    """Slots go back to the pool only when no copy into them is pending, also
+    where every allocation after the first copy fails."""
+    run(program, "memory")
