@@ -19,6 +19,7 @@
 #include <new>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "dbec.h"
@@ -297,6 +298,24 @@ void late_threads() {
     }
 }
 
+// Contexts come and go in several threads, whose transfers share pool and slots.
+void callers() {
+    thread_delay_us = 2000;
+    std::vector<std::thread> th;
+    for (int t = 0; t < 4; ++t)
+        th.emplace_back([t] {
+            for (int k = 0; k < 3; ++k) {
+                dbec_ctx *c = create(BX, BY, BZ, DBEC_REAL, (t & 1) ? DBEC_MIXED : DBEC_FP64);
+                round_trip(c, BIG, 10 * t + k);
+                round_trip(c, BIG, 10 * t + k + 5);
+                CHECK(dbec_destroy(c) == DBEC_OK);
+            }
+        });
+    for (auto &t : th) t.join();
+    CHECK(pinned_live == 0);
+    CHECK(freed_in_flight == 0);
+}
+
 // No memory is to be had once the first pieces are on their way.
 void memory() {
     for (int big = 0; big < 2; ++big)
@@ -323,6 +342,7 @@ int main(int argc, char **argv) {
     alarm(100);
     const std::string s = argc > 1 ? argv[1] : "";
     if (s == "late_threads") late_threads();
+    else if (s == "callers") callers();
     else if (s == "memory") memory();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");

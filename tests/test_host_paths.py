@@ -40,3 +40,9 @@ def test_no_memory_during_a_fetch(program):
     """Slots go back to the pool only when no copy into them is pending, also
     where every allocation after the first copy fails."""
     run(program, "memory")
+
+
+def test_contexts_of_several_threads(program):
+    """Four threads whose transfers, past the bound from which the pool's
+    threads help, run at once, while contexts come and go under them."""
+    run(program, "callers")
