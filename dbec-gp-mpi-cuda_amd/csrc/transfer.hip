@@ -62,8 +62,9 @@ void destroy(Slot &s) {
     s = Slot();
 }
 
-// Up to `want` slots of the device; fewer, or none, where the pool is at its
-// bound or memory is short.
+// Up to `want` slots of the device: its free ones, new ones up to the pool's
+// bound, then free ones of other devices (the memory serves every device, an
+// event only its own).  Fewer, or none, where all are in use or memory is short.
 std::vector<Slot> acquire(int device, int want) {
     std::vector<Slot> got;
     got.reserve(want);
@@ -83,6 +84,21 @@ std::vector<Slot> acquire(int device, int want) {
             break;
         }
         ++g_slots;
+        got.push_back(s);
+    }
+    while ((int)got.size() < want && !g_free.empty()) {
+        Slot s = g_free.back();
+        g_free.pop_back();
+        (void)hipEventDestroy(s.ev);
+        s.ev = nullptr;
+        s.device = device;
+        if (hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) {
+            s.ev = nullptr;
+            destroy(s);
+            --g_slots;
+            (void)hipGetLastError();
+            break;
+        }
         got.push_back(s);
     }
     return got;

@@ -31,6 +31,7 @@ std::atomic<bool> short_of_memory{false};  // allocations fail while a fetched p
 std::atomic<int> pending_fetches{0};
 std::atomic<int> thread_delay_us{0};
 std::atomic<int> pinned_live{0}, freed_in_flight{0};
+std::atomic<int> staged_copies[16];
 
 struct Enter {
     Enter() { ++in_fake; }
@@ -200,6 +201,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, h
     std::lock_guard<std::mutex> lk(fake().mu);
     auto *s = reinterpret_cast<Stream *>(h);
     const bool to = is_pinned(dst), from = is_pinned(src);
+    if (to || from) ++staged_copies[s->device];
     if (to) ++pending_fetches;
     s->ops.push_back({dst, src, n});
     ++s->queued;
@@ -336,6 +338,21 @@ void memory() {
         }
 }
 
+// Contexts on more devices than the slots' bound would serve at once.
+void devices() {
+    std::vector<dbec_ctx *> c;
+    for (int d = 0; d < 5; ++d) c.push_back(create(64, BY, BZ, DBEC_REAL, DBEC_FP64, d));
+    for (int k = 0; k < 2; ++k)
+        for (int d = 0; d < 5; ++d) {
+            const int before = staged_copies[d];
+            round_trip(c[d], 2 * size_t(64 * BY * BZ), d + k);
+            CHECK(staged_copies[d] > before);
+            CHECK(pinned_live <= 32 + 5);  // the slots, and each context's scalars
+        }
+    for (dbec_ctx *x : c) CHECK(dbec_destroy(x) == DBEC_OK);
+    CHECK(pinned_live == 0);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -344,6 +361,7 @@ int main(int argc, char **argv) {
     if (s == "late_threads") late_threads();
     else if (s == "callers") callers();
     else if (s == "memory") memory();
+    else if (s == "devices") devices();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

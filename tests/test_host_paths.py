@@ -46,3 +46,9 @@ def test_contexts_of_several_threads(program):
     """Four threads whose transfers, past the bound from which the pool's
     threads help, run at once, while contexts come and go under them."""
     run(program, "callers")
+
+
+def test_slots_move_between_devices(program):
+    """Contexts on five devices, one transfer at a time, with slots for two
+    devices' transfers in the pool: none is left to the plain way."""
+    run(program, "devices")
