@@ -1043,8 +1043,9 @@ long density_sums(const dbec_ctx *c, int kind) {
 }
 
 // One extract through `d` (cap doubles): sums, sampling and the copy to `out`.
-// The sampled 3-D extract runs in slabs of x where it does not fit.
-int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, double *d, long cap) {
+// The sampled 3-D extract runs in slabs of x where it does not fit.  plain: no
+// staging buffers for the copy (dbec_density_noalloc allocates nothing).
+int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, double *d, long cap, bool plain) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
     const long sx = (Nx + ox - 1) / ox, sy = (Ny + oy - 1) / oy, sz = (Nz + oz - 1) / oz;
     const long sums = density_sums(c, kind), cnt = dbec_density_count(c, kind, ox, oy, oz);
@@ -1092,15 +1093,15 @@ int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, d
         for (long a = 0; a < total && e == hipSuccess; a += per) {
             n[0] = std::min(per, total - a);
             e = launch_pick_mod2(s, c, start, step, n, d);
-            if (e == hipSuccess) e = fetch_field(c, out + a * slab, d, (size_t)(n[0] * slab), false);
+            const size_t m = (size_t)(n[0] * slab);
+            if (e == hipSuccess) e = plain ? fetch_plain(c, out + a * slab, d, m) : fetch_field(c, out + a * slab, d, m, false);
             start[0] += n[0] * step[0];
         }
         if (e != hipSuccess) return hip_fail(c, e, "density");
         return DBEC_OK;
     }
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(out, dst, (size_t)cnt * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = fetch_plain(c, out, dst, (size_t)cnt);
     if (e != hipSuccess) return hip_fail(c, e, "density");
     return DBEC_OK;
 }
@@ -1117,7 +1118,7 @@ int dbec_density(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) 
     (void)hipSetDevice(c->device);
     CHK(materialize_scale(c));
     const long cap = (long)((size_t)c->Nkz * c->Nx * c->Ny * 2 * real_elem(c) / sizeof(double));
-    return density_via(c, kind, ox, oy, oz, out, static_cast<double *>(c->b.spec), cap);
+    return density_via(c, kind, ox, oy, oz, out, static_cast<double *>(c->b.spec), cap, false);
 }
 
 int dbec_density_noalloc(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out) {
@@ -1134,7 +1135,7 @@ int dbec_density_noalloc(dbec_ctx *c, int kind, long ox, long oy, long oz, doubl
                         " bytes of device scratch, more than its " + std::to_string((long)DBEC_NOALLOC_SCRATCH_BYTES) +
                         " bytes (use dbec_density or coarser output steps)");
     CHK(materialize_scale(c));
-    return density_via(c, kind, ox, oy, oz, out, d, cap);
+    return density_via(c, kind, ox, oy, oz, out, d, cap, true);
 }
 
 int dbec_get_table(dbec_ctx *c, int which, int axis, double *out) {

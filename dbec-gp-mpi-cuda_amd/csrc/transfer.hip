@@ -346,16 +346,18 @@ hipError_t fetch_field(const dbec_ctx *c, double *dst, const void *src, size_t n
         return fetch_staged(c, dst, static_cast<const char *>(src), n, f32, s);
     }, done);
     if (done) return e;
-    if (!f32) {
-        e = hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-        return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
-    }
+    if (!f32) return fetch_plain(c, dst, static_cast<const double *>(src), n);
     std::vector<float> f(n);
     e = hipMemcpyAsync(f.data(), src, n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess)
         for (size_t i = 0; i < n; i++) dst[i] = f[i];
     return e;
+}
+
+hipError_t fetch_plain(const dbec_ctx *c, double *dst, const double *src, size_t n) {
+    const hipError_t e = hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
 }
 
 hipError_t store_field(const dbec_ctx *c, void *dst, const double *src, size_t n, bool f32) {

@@ -31,6 +31,7 @@ std::atomic<bool> short_of_memory{false};  // allocations fail while a fetched p
 std::atomic<int> pending_fetches{0};
 std::atomic<int> thread_delay_us{0};
 std::atomic<int> pinned_live{0}, freed_in_flight{0};
+std::atomic<int> allocs{0};  // host and device memory, events
 std::atomic<int> staged_copies[16];
 
 struct Enter {
@@ -91,6 +92,7 @@ void drain(Stream *s, size_t upto) {  // mu held
 
 void *operator new(size_t n) {
     if (!in_fake && short_of_memory && pending_fetches > 0) throw std::bad_alloc();
+    if (!in_fake) ++allocs;
     if (void *p = std::malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }
@@ -147,6 +149,7 @@ hipError_t hipMemGetInfo(size_t *fr, size_t *tot) { return *fr = *tot = size_t(2
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stand-in error"; }
 hipError_t hipMalloc(void **p, size_t n) {
+    ++allocs;
     return (*p = std::calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void *p) { return std::free(p), hipSuccess; }
@@ -159,7 +162,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
     std::lock_guard<std::mutex> lk(fake().mu);
     fake().pinned[static_cast<char *>(*p)] = n;
-    ++pinned_live;
+    ++allocs, ++pinned_live;
     return hipSuccess;
 }
 hipError_t hipHostFree(void *p) {
@@ -216,6 +219,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *ev, unsigned) {
     Enter in;
     auto *n = new Event;
     n->device = device;
+    ++allocs;
     return *ev = reinterpret_cast<hipEvent_t>(n), hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *ev) { return hipEventCreateWithFlags(ev, 0); }
@@ -353,6 +357,18 @@ void devices() {
     CHECK(pinned_live == 0);
 }
 
+// The largest extract that the no-allocation entry point takes: 8 MiB.
+void noalloc() {
+    dbec_ctx *c = create(64, BY, BZ, DBEC_IMAG, DBEC_FP64);
+    CHECK(dbec_density_count(c, DBEC_DEN_XYZ, 1, 1, 1) * (long)sizeof(double) == DBEC_NOALLOC_SCRATCH_BYTES);
+    std::vector<double> out(DBEC_NOALLOC_SCRATCH_BYTES / sizeof(double));
+    const int before = allocs;
+    for (int kind = DBEC_DEN_X; kind <= DBEC_DEN_XYZ; ++kind)
+        CHECK(dbec_density_noalloc(c, kind, 1, 1, 1, out.data()) == DBEC_OK);
+    CHECK(allocs == before);
+    CHECK(dbec_destroy(c) == DBEC_OK);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -362,6 +378,7 @@ int main(int argc, char **argv) {
     else if (s == "callers") callers();
     else if (s == "memory") memory();
     else if (s == "devices") devices();
+    else if (s == "noalloc") noalloc();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

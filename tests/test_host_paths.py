@@ -52,3 +52,9 @@ def test_slots_move_between_devices(program):
     """Contexts on five devices, one transfer at a time, with slots for two
     devices' transfers in the pool: none is left to the plain way."""
     run(program, "devices")
+
+
+def test_noalloc_density_allocates_nothing(program):
+    """dbec_density_noalloc up to its largest extract: no device or host memory
+    and no event."""
+    run(program, "noalloc")
