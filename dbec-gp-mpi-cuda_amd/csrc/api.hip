@@ -1008,9 +1008,12 @@ int dbec_step(dbec_ctx *c, long nsteps, double g_stp, double gd_stp, double *nor
     return DBEC_OK;
 }
 
+// Samples of an axis of n points at every o-th, for every o >= 1.
+static long samples(long n, long o) { return (n - 1) / o + 1; }
+
 long dbec_density_count(const dbec_ctx *c, int kind, long ox, long oy, long oz) {
     if (!c || ox < 1 || oy < 1 || oz < 1) return -1;
-    long sx = (c->Nx + ox - 1) / ox, sy = (c->Ny + oy - 1) / oy, sz = (c->Nz + oz - 1) / oz;
+    const long sx = samples(c->Nx, ox), sy = samples(c->Ny, oy), sz = samples(c->Nz, oz);
     switch (kind) {
     case DBEC_DEN_X: return sx;
     case DBEC_DEN_Y: return sy;
@@ -1047,7 +1050,7 @@ long density_sums(const dbec_ctx *c, int kind) {
 // staging buffers for the copy (dbec_density_noalloc allocates nothing).
 int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, double *d, long cap, bool plain) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
-    const long sx = (Nx + ox - 1) / ox, sy = (Ny + oy - 1) / oy, sz = (Nz + oz - 1) / oz;
+    const long sx = samples(Nx, ox), sy = samples(Ny, oy), sz = samples(Nz, oz);
     const long sums = density_sums(c, kind), cnt = dbec_density_count(c, kind, ox, oy, oz);
     const double *wx = c->b.wgt, *wy = c->b.wgt + Nx;
     double *dst = d + sums;

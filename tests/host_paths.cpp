@@ -10,6 +10,7 @@
 #include <unistd.h>
 
 #include <atomic>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -369,6 +370,22 @@ void noalloc() {
     CHECK(dbec_destroy(c) == DBEC_OK);
 }
 
+// Output steps as large as they come: one sample per axis.
+void long_steps() {
+    dbec_ctx *c = create(16, 32, 16, DBEC_IMAG, DBEC_FP64);
+    for (long o : {1000L, LONG_MAX - 20, LONG_MAX})
+        for (int kind = DBEC_DEN_X; kind <= DBEC_DEN_XYZ; ++kind) {
+            CHECK(dbec_density_count(c, kind, o, o, o) == 1);
+            double out[2] = {-1.0, -1.0};
+            CHECK(dbec_density(c, kind, o, o, o, out) == DBEC_OK);
+            CHECK(out[0] == 0.0 && out[1] == -1.0);
+            out[0] = -1.0;
+            CHECK(dbec_density_noalloc(c, kind, o, o, o, out) == DBEC_OK);
+            CHECK(out[0] == 0.0 && out[1] == -1.0);
+        }
+    CHECK(dbec_destroy(c) == DBEC_OK);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -379,6 +396,7 @@ int main(int argc, char **argv) {
     else if (s == "memory") memory();
     else if (s == "devices") devices();
     else if (s == "noalloc") noalloc();
+    else if (s == "long_steps") long_steps();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

@@ -58,3 +58,7 @@ def test_noalloc_density_allocates_nothing(program):
     """dbec_density_noalloc up to its largest extract: no device or host memory
     and no event."""
     run(program, "noalloc")
+
+
+def test_output_steps_up_to_the_largest(program):
+    run(program, "long_steps")
