@@ -294,17 +294,23 @@ int run_sweep(dbec_ctx *c, int axis, const Solves &v, bool cols) {
     return DBEC_OK;
 }
 
+// DBEC_FUSE_Z=0: a step's end and the start of the next one run as kernels of
+// their own, on every grid (so without the plane kernels).
+bool fuse_on() {
+    static const bool on = [] {
+        const char *e = getenv("DBEC_FUSE_Z");
+        return !e || std::strcmp(e, "0") != 0;
+    }();
+    return on;
+}
+
 // Whether the z sweep of a step runs fused with the next step's forward z pass
 // (every length has the kernel; DBEC_FUSE_Z=0 turns it off, and so do bounds
 // on the z sweep's rows that the kernel is not built for).  Measured where it
 // once ran unfused: 35 -> 24 us at 192x320x48, 281 -> 229 at 256x256x384
 // (complex FP64); never slower.
 bool fuse_z(const dbec_ctx *c) {
-    static const bool on = [] {
-        const char *e = getenv("DBEC_FUSE_Z");
-        return !e || std::strcmp(e, "0") != 0;
-    }();
-    return on && sweepz_zfwd_fusable(c->Nz, c->prec == DBEC_MIXED, c->mode == DBEC_REAL, fused_z_rows(c));
+    return fuse_on() && sweepz_zfwd_fusable(c->Nz, c->prec == DBEC_MIXED, c->mode == DBEC_REAL, fused_z_rows(c));
 }
 
 // Whether a step's end runs fused with the start of the next step.
@@ -816,7 +822,7 @@ int core_create(const dbec_params *p, dbec_mode mode, dbec_prec prec, void *stre
     c->N = c->Nx * c->Ny * c->Nz;
     c->Nkz = c->Nz / 2 + 1;
     c->pi = (p->pi != 0.) ? p->pi : 3.14159265358979;
-    c->planes = plane_ok(c, shared);
+    c->planes = fuse_on() && plane_ok(c, shared);
     if (stream) {
         c->stream = static_cast<hipStream_t>(stream);
     } else {

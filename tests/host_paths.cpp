@@ -1,8 +1,8 @@
 // Host paths of libdbec_hip without a device: this program defines the HIP
 // entry points that the library imports (the dynamic linker prefers the
 // program's own), with device memory in host memory, copies to and from pinned
-// memory left pending until somebody waits for them, and kernels that do
-// nothing.  test_host_paths.py builds it and runs one scenario a
+// memory left pending until somebody waits for them, and kernels that only
+// leave their name.  test_host_paths.py builds it and runs one scenario a
 // process; a scenario ends with "ok", or with what went wrong.
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
@@ -59,6 +59,8 @@ struct Fake {
     std::mutex mu;
     std::map<char *, size_t> pinned;
     std::set<Stream *> streams;
+    std::map<const void *, std::string> kernels;
+    std::map<std::string, unsigned> launched;  // mangled name -> threads per workgroup
 };
 Fake &fake() {  // also reached from the library's initialisers, before this program's
     static Fake *f = new Fake;
@@ -126,8 +128,11 @@ void **__hipRegisterFatBinary(const void *) {
     return &module;
 }
 void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, uint3_ *, uint3_ *, dim3 *, dim3 *,
-                           int *) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, uint3_ *, uint3_ *, dim3 *,
+                           dim3 *, int *) {
+    Enter in;
+    fake().kernels[host] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t shm, hipStream_t s) {
     config = {g, b, shm, s};
@@ -137,7 +142,12 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shm, hipStream_t 
     *g = config.g, *b = config.b, *shm = config.shm, *s = config.s;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *f, dim3, dim3 b, void **, size_t, hipStream_t) {
+    Enter in;
+    std::lock_guard<std::mutex> lk(fake().mu);
+    fake().launched[fake().kernels[f]] = b.x * b.y * b.z;
+    return hipSuccess;
+}
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 
 hipError_t hipGetDeviceCount(int *n) { return *n = 16, hipSuccess; }
@@ -386,6 +396,33 @@ void long_steps() {
     CHECK(dbec_destroy(c) == DBEC_OK);
 }
 
+// Threads per workgroup of the kernel `name` in a call of three steps, 0 if it
+// did not run.
+unsigned launched(const char *name) {
+    for (auto &k : fake().launched)
+        if (k.first.find(std::to_string(std::strlen(name)) + name) != std::string::npos) return k.second;
+    return 0;
+}
+void steps(long nx, long ny, long nz, dbec_mode mode, dbec_prec prec) {
+    dbec_ctx *c = create(nx, ny, nz, mode, prec);
+    fake().launched.clear();
+    CHECK(dbec_step(c, 3, 0.0, 0.0, nullptr) == DBEC_OK);
+    CHECK(dbec_destroy(c) == DBEC_OK);
+}
+bool fused() { return launched("k_plane_fwd") || launched("k_plane_inv") || launched("k_sweepz_zfwd"); }
+
+// The kernels of a step's end and the next one's start.
+void fuse(bool on) {
+    for (dbec_mode mode : {DBEC_IMAG, DBEC_REAL})
+        for (dbec_prec prec : {DBEC_FP64, DBEC_MIXED})
+            for (long ny : {64, 160}) {  // a grid of the plane kernels, and one past them
+                steps(64, ny, 64, mode, prec);
+                CHECK(fused() == on);
+                CHECK((launched("k_plane_fwd") > 0) == (on && ny == 64));
+                CHECK((launched("k_sweep_z") && launched("k_zfwd")) || on);
+            }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -397,6 +434,8 @@ int main(int argc, char **argv) {
     else if (s == "devices") devices();
     else if (s == "noalloc") noalloc();
     else if (s == "long_steps") long_steps();
+    else if (s == "fused") fuse(true);
+    else if (s == "unfused") fuse(false);
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

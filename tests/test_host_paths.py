@@ -1,7 +1,7 @@
 """Host paths of the library that need no device: transfers through the staging
-slots and the pool of threads.  host_paths.cpp stands in for the HIP runtime
-(its entry points come before the real ones in symbol lookup) and runs one
-scenario a process."""
+slots and the pool of threads, and which kernels a step launches.
+host_paths.cpp stands in for the HIP runtime (its entry points come before the
+real ones in symbol lookup) and runs one scenario a process."""
 import os
 import subprocess
 
@@ -62,3 +62,10 @@ def test_noalloc_density_allocates_nothing(program):
 
 def test_output_steps_up_to_the_largest(program):
     run(program, "long_steps")
+
+
+def test_fuse_z_switch(program):
+    """DBEC_FUSE_Z=0 runs a step's z sweep and the next one's forward z pass as
+    two kernels, on the grids of the plane kernels too."""
+    run(program, "fused")
+    run(program, "unfused", DBEC_FUSE_Z="0")
