@@ -191,7 +191,7 @@ struct FusedZ {
     static_assert(FusedPlan<N>::T * 8 == N, "fused z plan");
     // complex rows: half a tile at a time
     template <typename S>
-    static constexpr bool half() { return !std::is_floating_point<S>::value && (sizeof(S) == 16 || N >= 256); }
+    static constexpr bool half() { return fused_z_half<S>(N); }
     // row partials of the z integrals: real lines (imaginary time) only
     template <typename S>
     static constexpr bool cols() { return std::is_floating_point<S>::value; }

@@ -342,14 +342,16 @@ static int env_int(const char *name, int dflt) {
     return e ? atoi(e) : dflt;
 }
 
+// half: the tile holds half of the rows at a time.
 template <typename S>
-static int z_rows(long n) {
+static int z_rows(long n, bool half = false) {
     static const int max_threads = env_int("DBEC_SWEEP_Z_THREADS", 256);
     static const long tile_max = 1024L * env_int("DBEC_SWEEP_Z_TILE_KB", 64);
     const int M = z_seg_len(n);
     const int P = (int)(n / M);
+    const auto tile = [&](int L) { return (long)(n + Pk<S>::n) * (half ? L / 2 : L) * (long)sizeof(S); };
     int L = 64;
-    while (L > 4 && ((long)L * P > max_threads || (long)(n + Pk<S>::n) * L * (long)sizeof(S) > tile_max)) L /= 2;
+    while (L > 4 && ((long)L * P > max_threads || tile(L) > tile_max)) L /= 2;
     return L;
 }
 
@@ -362,16 +364,15 @@ int sweep_z_rows(const dbec_ctx *c) {
 }
 
 // Rows per workgroup of the fused z kernel: real lines as the z sweep (its
-// column partials are one per workgroup of those rows); complex lines, which
-// have none and pass through half a tile, the most that give at most 256
-// threads (measured at 512 complex FP64: 8 rows 151, the z sweep's 4 rows 200
+// column partials are one per workgroup of those rows); complex lines by the
+// same bounds on their own tile, which mostly holds half of the rows, so by
+// default the most that give at most 256 threads (measured at 512 complex FP64: 8 rows 151, the z sweep's 4 rows 200
 // us; at 128: 32 rows 41, 16 rows 46 us; twice the rows, so twice the threads
 // at a barrier: 143 -> 159 us at 256^3, 229 -> 280 at 256x256x384).
 int fused_z_rows(const dbec_ctx *c) {
     if (c->mode == DBEC_IMAG) return sweep_z_rows(c);
-    int L = 64;
-    while (L > 8 && L * (c->Nz / 16) > 256) L /= 2;
-    return L;
+    return c->prec == DBEC_MIXED ? z_rows<cpx<float>>(c->Nz, fused_z_half<cpx<float>>(c->Nz))
+                                 : z_rows<cpx<double>>(c->Nz, fused_z_half<cpx<double>>(c->Nz));
 }
 
 AxisArgs sweep_axis_args(const dbec_ctx *c, int axis) {

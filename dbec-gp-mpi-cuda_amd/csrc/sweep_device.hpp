@@ -135,6 +135,14 @@ struct SweepTab {
     const typename TabOf<A>::T *ca, *cg, *gb, *fa;
 };
 
+// Whether the z sweep fused with the forward z transform takes rows of n
+// through a tile of half of them at a time: complex ones, but in FP32 only from
+// 256 on.
+template <typename S>
+__host__ __device__ constexpr bool fused_z_half(long n) {
+    return !std::is_floating_point<S>::value && (sizeof(S) == 16 || n >= 256);
+}
+
 // LDS layout shared by the sweep kernels with segments of M: the four
 // tables, the carry exchange (one per thread), the last elements, the row
 // partials (one per thread, only with the z integrals).  A table keeps the M entries of segment s in

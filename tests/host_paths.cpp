@@ -423,6 +423,14 @@ void fuse(bool on) {
             }
 }
 
+// Bounds on the z sweep's rows, from the environment: threads per workgroup of
+// the fused kernel of complex lines, or 0 for the two kernels in its place.
+void rows(dbec_prec prec, unsigned want) {
+    steps(16, 160, 256, DBEC_REAL, prec);
+    CHECK(launched("k_sweepz_zfwd") == want);
+    CHECK(want || (launched("k_sweep_z") && launched("k_zfwd")));
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -436,6 +444,7 @@ int main(int argc, char **argv) {
     else if (s == "long_steps") long_steps();
     else if (s == "fused") fuse(true);
     else if (s == "unfused") fuse(false);
+    else if (s == "rows") rows((dbec_prec)std::atoi(argv[2]), (unsigned)std::atoi(argv[3]));
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

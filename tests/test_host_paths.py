@@ -23,9 +23,9 @@ def program(tmp_path_factory):
     return exe
 
 
-def run(program, scenario, **env):
+def run(program, scenario, *args, **env):
     keep = {k: v for k, v in os.environ.items() if not k.startswith("DBEC_")}
-    r = subprocess.run([program, scenario], env={**keep, "DBEC_AUTOTUNE": "0", **env}, capture_output=True, text=True,
+    r = subprocess.run([program, scenario, *args], env={**keep, "DBEC_AUTOTUNE": "0", **env}, capture_output=True, text=True,
                        timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout, r.stderr[-1000:])
 
@@ -69,3 +69,16 @@ def test_fuse_z_switch(program):
     two kernels, on the grids of the plane kernels too."""
     run(program, "fused")
     run(program, "unfused", DBEC_FUSE_Z="0")
+
+
+@pytest.mark.parametrize("prec,tile_kb", [(dbecpy.FP64, 33), (dbecpy.MIXED, 17)], ids=["fp64", "mixed"])
+def test_bounds_of_the_z_sweep_rows(program, prec, tile_kb):
+    """DBEC_SWEEP_Z_THREADS and DBEC_SWEEP_Z_TILE_KB bound the rows of the fused
+    kernel of complex lines as those of real ones: by default 16 rows of 256
+    (16 threads each, a tile of 8 rows), 8 below a bound that 16 do not meet,
+    and the two kernels where 8 do not meet it either."""
+    for want, bound in (("256", {}), ("128", {"DBEC_SWEEP_Z_THREADS": "128"}), ("0", {"DBEC_SWEEP_Z_THREADS": "64"}),
+                        ("256", {"DBEC_SWEEP_Z_TILE_KB": str(tile_kb)}),
+                        ("128", {"DBEC_SWEEP_Z_TILE_KB": str(tile_kb - 1)}),
+                        ("0", {"DBEC_SWEEP_Z_TILE_KB": str(tile_kb // 2 - 1)})):
+        run(program, "rows", str(prec), want, **bound)
