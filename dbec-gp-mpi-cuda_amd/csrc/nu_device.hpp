@@ -81,7 +81,7 @@ __device__ __forceinline__ double trap(const TrapConst &tc, double x2, double y2
 // exp(shift): a constant factor that the renormalisation after the sweeps
 // removes again (the sweeps are linear); the mixed form uses it to keep FP32
 // psi away from overflow, the FP64 form passes 0 (exact: x + 0 = x).
-__device__ __forceinline__ double nu_imag(double psitmp, double phi, double pot, const NuConst &nc) {
+__device__ __forceinline__ double nu_imag(double psitmp, double phi, double pot, const NuConst &nc, bool kept) {
     const double psi2lin = psitmp * psitmp * nc.g;
     const double psidd2lin = div_nd(phi, nc) * nc.gd;
     const double pottmp = nc.dt * (pot + psi2lin + psidd2lin);
@@ -91,7 +91,7 @@ __device__ __forceinline__ double nu_imag(double psitmp, double phi, double pot,
     // shift follows dt * mu, so e stays O(1) on a converging state.
     if (nc.cap && e > 80.0) {
         e = 80.0;
-        *nc.capped = 1.0;
+        if (kept) *nc.capped = 1.0;
     }
     return psitmp * exp(e);
 }
@@ -172,27 +172,32 @@ __device__ __forceinline__ cpx<double> nu_real(cpx<double> v, double phi, double
 }
 
 // Generic over the storage of psi: double / float (imaginary time, with the
-// pending renormalisation s) and cpx<double> / cpx<float> (real time).
-__device__ __forceinline__ double nu_apply(double v, double s, double phi, double pot, const NuConst &nc) {
-    return nu_imag(v * s, phi, pot, nc);
+// pending renormalisation s) and cpx<double> / cpx<float> (real time).  kept:
+// the value is stored; one that is not must not flag a capped exponent.
+__device__ __forceinline__ double nu_apply(double v, double s, double phi, double pot, const NuConst &nc,
+                                           bool kept = true) {
+    return nu_imag(v * s, phi, pot, nc, kept);
 }
-__device__ __forceinline__ cpx<double> nu_apply(cpx<double> v, double, double phi, double pot, const NuConst &nc) {
+__device__ __forceinline__ cpx<double> nu_apply(cpx<double> v, double, double phi, double pot, const NuConst &nc,
+                                                bool = true) {
     return nu_real(v, phi, pot, nc);
 }
 // The mixed form evaluates the nonlinear factor in FP32 (single-precision
 // exp / sincos) from FP32 phi and the FP32 constants of nu_prepare; the
 // renormalisation and the trap potential are formed in FP64 first.
-__device__ __forceinline__ float nu_apply(float v, double s, float phi, double pot, const NuConst &nc) {
+__device__ __forceinline__ float nu_apply(float v, double s, float phi, double pot, const NuConst &nc,
+                                          bool kept = true) {
     const float p = (float)((double)v * s);
     const float lin = (float)pot + p * p * nc.gf + phi * nc.gdnf;
     float e = -nc.dtf * lin + nc.shiftf;
     if (nc.cap && e > 80.0f) {
         e = 80.0f;
-        *nc.capped = 1.0;
+        if (kept) *nc.capped = 1.0;
     }
     return p * expf(e);
 }
-__device__ __forceinline__ cpx<float> nu_apply(cpx<float> v, double, float phi, double pot, const NuConst &nc) {
+__device__ __forceinline__ cpx<float> nu_apply(cpx<float> v, double, float phi, double pot, const NuConst &nc,
+                                               bool = true) {
     const float a2 = v.x * v.x + v.y * v.y;
     const float lin = (float)pot + a2 * nc.gf + phi * nc.gdnf;
     float sn, cs;

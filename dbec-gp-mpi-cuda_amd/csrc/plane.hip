@@ -471,11 +471,11 @@ k_plane_inv(Solves v, PlaneDims g, const double *__restrict__ sq, NuConst nc, R 
     if constexpr (PHI) out = phi + (extra ? far : (long)x * Ny * Nz);
     else out = psi;
     const double *row = extra ? sqr + Ny : sqr;
-    const auto value = [&](int y, int z, P p0, R f) {
+    const auto value = [&](int y, int z, P p0, R f, bool kept) {
         if constexpr (PHI) return f;
-        else return nu_apply(p0, s, f, trap_sum(tc, row[y], sqz[z]), nc);
+        else return nu_apply(p0, s, f, trap_sum(tc, row[y], sqz[z]), nc, kept);
     };
-    if (rim) out[(Ny - 1) * Nz + tid] = value(Ny - 1, tid, pr, zb[m24(tid, LP)].x);
+    if (rim) out[(Ny - 1) * Nz + tid] = value(Ny - 1, tid, pr, zb[m24(tid, LP)].x, true);
     // own: the plane transformed; else the points y < Ny-1, z < Nz-1 of plane Nx-1
 #pragma unroll 1
     for (bool own = !extra;; own = false) {
@@ -501,7 +501,7 @@ k_plane_inv(Solves v, PlaneDims g, const double *__restrict__ sq, NuConst nc, R 
                 const bool put = i < points && (own ? (x < Nx - 1 ? !(yl && !zl) : (yl || zl)) : !(yl || zl));
                 const int zs = (own && x < Nx - 1 && zl && !yl) ? 0 : z;
                 const R *c = reinterpret_cast<const R *>(&zb[m24(zs, LP) + m24(r >> 1, nj) + jj]) + (r & 1);
-                ov[w] = value(y, z, pv[gr][w], *c);
+                ov[w] = value(y, z, pv[gr][w], *c, put);
                 at[w] = put ? m24(y, Nz) + z : -1;
             }
 #pragma unroll
