@@ -62,9 +62,9 @@ hipError_t launch_sweepz_zfwd(long n, const FftArgs &a) {
     default: return hipErrorInvalidValue;
     }
 }
-bool sweepz_zfwd_fusable(long n, bool fp32, bool cpsi, int zrows) {
+bool sweepz_zfwd_fusable(long n, bool fp32, bool cpsi, int rows, int rows_half) {
     switch (n) {
-#define DBEC_X(NN) case NN: return FftLaunch<NN>::fusable(fp32, cpsi, zrows);
+#define DBEC_X(NN) case NN: return FftLaunch<NN>::fusable(fp32, cpsi, rows, rows_half);
         DBEC_FOR_EACH_FFT_LEN(DBEC_X)
 #undef DBEC_X
     default: return false;
@@ -310,7 +310,8 @@ bool fuse_on() {
 // once ran unfused: 35 -> 24 us at 192x320x48, 281 -> 229 at 256x256x384
 // (complex FP64); never slower.
 bool fuse_z(const dbec_ctx *c) {
-    return fuse_on() && sweepz_zfwd_fusable(c->Nz, c->prec == DBEC_MIXED, c->mode == DBEC_REAL, fused_z_rows(c));
+    return fuse_on() &&
+           sweepz_zfwd_fusable(c->Nz, c->prec == DBEC_MIXED, c->mode == DBEC_REAL, sweep_z_rows(c), fused_z_rows_half(c));
 }
 
 // Whether a step's end runs fused with the start of the next step.

@@ -172,8 +172,8 @@ k_zfwd(Solves v, int Nx, int Ny, const cpx<R> *__restrict__ twg, const double *_
 // done; and the tile, the carry exchange while the tile is in registers, and
 // the transform buffer after the tile is stored.  Complex rows are twice the
 // transform buffer, so (half) they pass through a tile of half the rows in
-// two turns, each in registers before the next: 50 instead of 88 KiB a
-// workgroup at N = 256 in FP64.  Complex FP32 rows of less than 256 fit often
+// two turns, each in registers before the next: 50 instead of 83 KiB a
+// workgroup of 16 rows at N = 256 in FP64.  Complex FP32 rows of less than 256 fit often
 // enough without, and the two turns' barriers measured 2-8 % slower there.
 // Measured (us; before: separate regions for tables, exchange and twiddles,
 // whole tiles; -> now; "+" where the two passes ran unfused before):
@@ -186,12 +186,9 @@ k_zfwd(Solves v, int Nx, int Ny, const cpx<R> *__restrict__ twg, const double *_
 //   256   256^3           75 -> 72       38 -> 38       214 -> 142      61 -> 58
 //   384   256x256x384     84 + 84 -> 131 38 + 43 -> 61  120 + 160 -> 229 55 + 89 -> 117
 //   512   128x256x512     110 -> 84      50 -> 44       279 -> 151      83 -> 72
-template <int N>
+template <int N, bool HALF>
 struct FusedZ {
     static_assert(FusedPlan<N>::T * 8 == N, "fused z plan");
-    // complex rows: half a tile at a time
-    template <typename S>
-    static constexpr bool half() { return fused_z_half<S>(N); }
     // row partials of the z integrals: real lines (imaginary time) only
     template <typename S>
     static constexpr bool cols() { return std::is_floating_point<S>::value; }
@@ -199,12 +196,13 @@ struct FusedZ {
     // allows; left to itself the compiler takes more registers than that)
     template <typename S>
     static constexpr int waves() {
+        if (!HALF && fused_z_half<S>(N)) return sizeof(S) == 16 ? 2 : 3;
         if (cols<S>()) return sizeof(S) == 8 ? 3 : 6;
         return sizeof(S) == 16 ? 3 : 4;
     }
     template <typename S, int L>
     static constexpr size_t tile_b() {
-        return ((size_t)(N + Pk<S>::n) * (half<S>() ? L / 2 : L) * sizeof(S) + 15) & ~size_t(15);
+        return ((size_t)(N + Pk<S>::n) * (HALF ? L / 2 : L) * sizeof(S) + 15) & ~size_t(15);
     }
     // transform buffer swizzled (unpadded) where the padded one does not fit
     // in the tile's region
@@ -236,9 +234,18 @@ struct FusedZ {
     static constexpr size_t x_off() { return tab_b<S, R>() + exl_b<S, L>() + exn_b<S, L>(); }
     template <typename S, typename R, int L>
     static constexpr size_t lds() { return x_off<S, R, L>() + x_b<S, R, L>(); }
-    // the kernel exists for rows L: at most 512 threads, LDS within 160 KiB
+    // the kernel exists for rows L: at most 512 threads, LDS within 160 KiB,
+    // half tiles only of the rows that are to take them
     template <typename S, typename R, int L>
-    static constexpr bool fits() { return L * (N / 16) <= 512 && lds<S, R, L>() <= 160 * 1024; }
+    static constexpr bool fits() {
+        return L * (N / 16) <= 512 && lds<S, R, L>() <= 160 * 1024 && (!HALF || fused_z_half<S>(N));
+    }
+    // workgroups that a CU holds at once by LDS and registers; 0: no kernel
+    template <typename S, typename R, int L>
+    static constexpr int per_cu() {
+        constexpr int by_lds = (int)(160 * 1024 / lds<S, R, L>()), by_reg = 4 * waves<S>() / ((L * (N / 16) + 63) / 64);
+        return !fits<S, R, L>() ? 0 : (by_lds < by_reg ? by_lds : by_reg);
+    }
 };
 
 // Whether the workgroups run from the largest x down, for psi of `bytes` (all
@@ -252,18 +259,17 @@ struct FusedZ {
 // gains nothing (604 -> 605 at 256x256x384 FP64).
 inline bool z_reversed(bool real, long bytes) { return !real && bytes >= (176L << 20); }
 
-template <int N, typename S, typename R, int L, bool COLS>
-__global__ void __launch_bounds__(L *(N / 16), FusedZ<N>::template waves<S>())
+template <int N, typename S, typename R, int L, bool COLS, bool HALF>
+__global__ void __launch_bounds__(L *(N / 16), (FusedZ<N, HALF>::template waves<S>()))
 k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, SweepConst<typename Arith<S>::T> k,
               const double *__restrict__ wz, const double *__restrict__ wy, const cpx<R> *__restrict__ twg, bool reversed) {
     using A = typename Arith<S>::T;
-    using F = FusedZ<N>;
+    using F = FusedZ<N, HALF>;
     using Pl = FusedPlan<N>;
     // psi tile rows of N + VE elements: 16-byte aligned, and consecutive rows
     // 4 banks apart, so the packet accesses below are conflict-free
     constexpr int M = 16, VE = Pk<S>::n, KV = M / VE;
     constexpr int P = N / M, WG = L * P, LF = L / 2, RS = N + VE;
-    constexpr bool HALF = F::template half<S>();
     // turns through the tile, rows and threads of each
     constexpr int NH = HALF ? 2 : 1, LH = L / NH, TH = WG / NH;
     static_assert(Pl::T * LF == WG && KV % NH == 0 && TH * NH == WG, "one transform thread per sweep thread");
@@ -960,10 +966,10 @@ struct FftLaunchImpl {
         return two ? xconv_t<double, 2>(a) : xconv_t<double, 1>(a);
     }
 
-    template <typename S, typename R, bool COLS, int L>
+    template <typename S, typename R, bool COLS, int L, bool HALF>
     static hipError_t sweepz_zfwd_t(const FftArgs &a) {
         using A = typename Arith<S>::T;
-        if constexpr (!FusedZ<N>::template fits<S, R, L>()) {
+        if constexpr (!FusedZ<N, HALF>::template fits<S, R, L>()) {
             return hipErrorInvalidValue;
         } else {
             const int yt = (int)((a.Ny + L - 1) / L);
@@ -974,8 +980,8 @@ struct FftLaunchImpl {
             SweepConst<A> k;
             zconst(a, k);
             const bool reversed = z_reversed(COLS, (long)a.v.nb * a.Nx * a.Ny * N * (long)sizeof(S));
-            k_sweepz_zfwd<N, S, R, L, COLS><<<grid, block, 0, a.stream>>>(a.v, (int)a.Nx, (int)a.Ny, tab, k, a.wz, a.wy,
-                                                                         static_cast<const cpx<R> *>(a.tw), reversed);
+            k_sweepz_zfwd<N, S, R, L, COLS, HALF><<<grid, block, 0, a.stream>>>(
+                a.v, (int)a.Nx, (int)a.Ny, tab, k, a.wz, a.wy, static_cast<const cpx<R> *>(a.tw), reversed);
             return hipGetLastError();
         }
     }
@@ -999,37 +1005,61 @@ struct FftLaunchImpl {
         k.A = {(float)a.zk[1][0], (float)a.zk[1][1]};
         k.mA = {(float)a.zk[2][0], (float)a.zk[2][1]};
     }
-    template <typename S, typename R, bool COLS>
-    static hipError_t sweepz_zfwd_rows(const FftArgs &a) {
-        switch (a.zrows) {
-        case 64: return sweepz_zfwd_t<S, R, COLS, 64>(a);
-        case 32: return sweepz_zfwd_t<S, R, COLS, 32>(a);
-        case 16: return sweepz_zfwd_t<S, R, COLS, 16>(a);
-        case 8: return sweepz_zfwd_t<S, R, COLS, 8>(a);
+    template <typename S, typename R, bool COLS, bool HALF>
+    static hipError_t sweepz_zfwd_rows(const FftArgs &a, int rows) {
+        switch (rows) {
+        case 64: return sweepz_zfwd_t<S, R, COLS, 64, HALF>(a);
+        case 32: return sweepz_zfwd_t<S, R, COLS, 32, HALF>(a);
+        case 16: return sweepz_zfwd_t<S, R, COLS, 16, HALF>(a);
+        case 8: return sweepz_zfwd_t<S, R, COLS, 8, HALF>(a);
         default: return hipErrorInvalidValue;
         }
     }
-    static hipError_t sweepz_zfwd(const FftArgs &a) {
-        if (!a.fp32) {
-            if (a.cpsi) return sweepz_zfwd_rows<cpx<double>, double, false>(a);
-            return sweepz_zfwd_rows<double, double, true>(a);
+    template <typename S, typename R, bool HALF>
+    static int per_cu(int zrows) {
+        switch (zrows) {
+        case 64: return FusedZ<N, HALF>::template per_cu<S, R, 64>();
+        case 32: return FusedZ<N, HALF>::template per_cu<S, R, 32>();
+        case 16: return FusedZ<N, HALF>::template per_cu<S, R, 16>();
+        case 8: return FusedZ<N, HALF>::template per_cu<S, R, 8>();
+        default: return 0;
         }
-        if (a.cpsi) return sweepz_zfwd_rows<cpx<float>, float, false>(a);
-        return sweepz_zfwd_rows<float, float, true>(a);
+    }
+    // Whole or half tiles (of complex rows that have both; the results are the
+    // same).  Half tiles put more rows on a CU, but each row takes two turns
+    // more at the barriers: whole ones serve a launch that needs no more
+    // rounds of the chip with them, in FP64 up to two rounds, in FP32 one.
+    // Measured, half / whole (us): complex FP64 64x32x160 13.4 / 11.0,
+    // 48x160x160 17.6 / 15.0, 48x160x320 35.0 / 31.3 (one, one and two rounds
+    // with either), 160x64x160 21.2 / 22.2, 96x160x256 34.6 / 41.8 (one with
+    // half, two with whole tiles); complex FP32 160x64x256 15.3 / 14.0,
+    // 96x160x256 18.1 / 20.7, and two rounds with either at 160x64x512
+    // 28.5 / 30.3, 96x160x384 31.5 / 32.6.
+    template <typename S, typename R, bool COLS>
+    static hipError_t sweepz_zfwd_tile(const FftArgs &a) {
+        const int kw = per_cu<S, R, false>(a.zrows), kh = per_cu<S, R, true>(a.zrows_half);
+        const auto rounds = [&](int rows, int k) {
+            const long wgs = (long)a.v.nb * a.Nx * ((a.Ny + rows - 1) / rows), all = 256L * k;
+            return (wgs + all - 1) / all;
+        };
+        bool half = kw == 0;
+        if (kw && kh) {
+            const long w = rounds(a.zrows, kw);
+            half = w > rounds(a.zrows_half, kh) || w > (sizeof(R) == 8 ? 2 : 1);
+        }
+        if (!half) return sweepz_zfwd_rows<S, R, COLS, false>(a, a.zrows);
+        if constexpr (fused_z_half<S>(N)) return sweepz_zfwd_rows<S, R, COLS, true>(a, a.zrows_half);
+        else return hipErrorInvalidValue;
+    }
+    static hipError_t sweepz_zfwd(const FftArgs &a) {
+        if (!a.fp32) return a.cpsi ? sweepz_zfwd_tile<cpx<double>, double, false>(a) : sweepz_zfwd_tile<double, double, true>(a);
+        return a.cpsi ? sweepz_zfwd_tile<cpx<float>, float, false>(a) : sweepz_zfwd_tile<float, float, true>(a);
     }
     template <typename S, typename R>
-    static bool fits_rows(int zrows) {
-        switch (zrows) {
-        case 64: return FusedZ<N>::template fits<S, R, 64>();
-        case 32: return FusedZ<N>::template fits<S, R, 32>();
-        case 16: return FusedZ<N>::template fits<S, R, 16>();
-        case 8: return FusedZ<N>::template fits<S, R, 8>();
-        default: return false;
-        }
-    }
-    static bool fusable(bool fp32, bool cpsi, int zrows) {
-        if (!fp32) return cpsi ? fits_rows<cpx<double>, double>(zrows) : fits_rows<double, double>(zrows);
-        return cpsi ? fits_rows<cpx<float>, float>(zrows) : fits_rows<float, float>(zrows);
+    static bool has_rows(int whole, int half) { return per_cu<S, R, false>(whole) || per_cu<S, R, true>(half); }
+    static bool fusable(bool fp32, bool cpsi, int rows, int rows_half) {
+        if (!fp32) return cpsi ? has_rows<cpx<double>, double>(rows, rows_half) : has_rows<double, double>(rows, rows_half);
+        return cpsi ? has_rows<cpx<float>, float>(rows, rows_half) : has_rows<float, float>(rows, rows_half);
     }
 
     // single solve: spectrum of `one` -> phi
@@ -1104,6 +1134,8 @@ hipError_t FftLaunch<N>::fused(const FftArgs &a) { return FftLaunchImpl<N>::fuse
 template <int N>
 hipError_t FftLaunch<N>::sweepz_zfwd(const FftArgs &a) { return FftLaunchImpl<N>::sweepz_zfwd(a); }
 template <int N>
-bool FftLaunch<N>::fusable(bool fp32, bool cpsi, int zrows) { return FftLaunchImpl<N>::fusable(fp32, cpsi, zrows); }
+bool FftLaunch<N>::fusable(bool fp32, bool cpsi, int rows, int rows_half) {
+    return FftLaunchImpl<N>::fusable(fp32, cpsi, rows, rows_half);
+}
 
 }  // namespace dbec

@@ -171,7 +171,7 @@ struct FftArgs {
     const void *ztab[4];
     double zk[3][2];
     const double *wz, *wy;
-    int zrows;
+    int zrows, zrows_half;  // with a tile of all rows, and of half of them at a time (0: not these rows)
     // x convolution: > 0 where slot s of a spectrum row holds the y frequency
     // s / yq + 8 (s % yq) (the plane kernels' digit order), 0: s itself
     int yq = 0;
@@ -189,8 +189,8 @@ hipError_t launch_zinv(long n, const FftArgs &a);    // spec -> phi (C2R along z
 // copies of phi, in one launch.
 hipError_t launch_zinv_nu(long n, const FftArgs &a);
 // The z sweep of one step fused with the forward z pass of the next; whether
-// length n has it for the precision and z sweep rows per workgroup.
+// length n has it for the precision and either of the rows per workgroup.
 hipError_t launch_sweepz_zfwd(long n, const FftArgs &a);
-bool sweepz_zfwd_fusable(long n, bool fp32, bool cpsi, int zrows);
+bool sweepz_zfwd_fusable(long n, bool fp32, bool cpsi, int rows, int rows_half);
 
 }  // namespace dbec

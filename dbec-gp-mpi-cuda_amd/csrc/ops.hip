@@ -363,16 +363,16 @@ int sweep_z_rows(const dbec_ctx *c) {
     return f32 ? z_rows<cpx<float>>(c->Nz) : z_rows<cpx<double>>(c->Nz);
 }
 
-// Rows per workgroup of the fused z kernel: real lines as the z sweep (its
-// column partials are one per workgroup of those rows); complex lines by the
-// same bounds on their own tile, which mostly holds half of the rows, so by
-// default the most that give at most 256 threads (measured at 512 complex FP64: 8 rows 151, the z sweep's 4 rows 200
-// us; at 128: 32 rows 41, 16 rows 46 us; twice the rows, so twice the threads
-// at a barrier: 143 -> 159 us at 256^3, 229 -> 280 at 256x256x384).
-int fused_z_rows(const dbec_ctx *c) {
-    if (c->mode == DBEC_IMAG) return sweep_z_rows(c);
-    return c->prec == DBEC_MIXED ? z_rows<cpx<float>>(c->Nz, fused_z_half<cpx<float>>(c->Nz))
-                                 : z_rows<cpx<double>>(c->Nz, fused_z_half<cpx<double>>(c->Nz));
+// Rows per workgroup of the fused z kernel where its tile holds half of them
+// at a time (complex lines), by the same bounds, which by default leave the most
+// that give at most 256 threads (measured at 512 complex FP64: 8 rows 151, 4
+// rows 200 us; at 128: 32 rows 41, 16 rows 46 us; twice the rows, so twice the
+// threads at a barrier: 143 -> 159 us at 256^3, 229 -> 280 at 256x256x384).
+// 0: no half tiles.  With whole tiles it takes the z sweep's rows.
+int fused_z_rows_half(const dbec_ctx *c) {
+    if (c->mode == DBEC_IMAG) return 0;
+    if (c->prec == DBEC_MIXED) return fused_z_half<cpx<float>>(c->Nz) ? z_rows<cpx<float>>(c->Nz, true) : 0;
+    return fused_z_half<cpx<double>>(c->Nz) ? z_rows<cpx<double>>(c->Nz, true) : 0;
 }
 
 AxisArgs sweep_axis_args(const dbec_ctx *c, int axis) {
@@ -400,7 +400,8 @@ void sweep_z_args(const dbec_ctx *c, FftArgs &a) {
         for (int q = 0; q < 2; q++) a.zk[i][q] = z.k[i][q];
     a.wz = c->b.wgt + c->Nx + c->Ny;
     a.wy = c->b.wgt + c->Nx;
-    a.zrows = fused_z_rows(c);
+    a.zrows = sweep_z_rows(c);
+    a.zrows_half = fused_z_rows_half(c);
 }
 
 long sweep_z_tiles(const dbec_ctx *c) {

@@ -42,7 +42,7 @@ hipError_t launch_sweep(hipStream_t s, const dbec_ctx *c, int axis, const Solves
 // number of y tiles of the z sweep (rows of the column partials)
 long sweep_z_tiles(const dbec_ctx *c);
 int sweep_z_rows(const dbec_ctx *c);
-int fused_z_rows(const dbec_ctx *c);
+int fused_z_rows_half(const dbec_ctx *c);
 // The z sweep's tables, constants, weights and rows per workgroup for the
 // z sweep fused with the forward z pass.
 void sweep_z_args(const dbec_ctx *c, FftArgs &a);

@@ -426,9 +426,30 @@ void fuse(bool on) {
 // Bounds on the z sweep's rows, from the environment: threads per workgroup of
 // the fused kernel of complex lines, or 0 for the two kernels in its place.
 void rows(dbec_prec prec, unsigned want) {
-    steps(16, 160, 256, DBEC_REAL, prec);
+    steps(96, 160, 256, DBEC_REAL, prec);
     CHECK(launched("k_sweepz_zfwd") == want);
     CHECK(want || (launched("k_sweep_z") && launched("k_zfwd")));
+}
+
+// Whole or half tiles of complex rows: whole ones where the launch needs no
+// more rounds of the chip with them.
+void tiles() {
+    const struct {
+        long nx, ny, nz;
+        bool half[2];  // FP64, mixed
+    } cases[] = {{16, 160, 16, {false, false}},  {320, 512, 16, {true, false}},  {192, 160, 64, {false, false}},
+                 {256, 320, 64, {true, false}},  {48, 160, 160, {false, false}}, {64, 160, 160, {true, false}},
+                 {16, 160, 256, {false, false}}, {80, 160, 256, {true, true}},   {48, 160, 320, {false, false}},
+                 {80, 160, 320, {true, true}},   {16, 160, 512, {true, false}}};
+    for (auto &k : cases)
+        for (dbec_prec prec : {DBEC_FP64, DBEC_MIXED}) {
+            steps(k.nx, k.ny, k.nz, DBEC_REAL, prec);
+            CHECK(launched("k_sweepz_zfwd") > 0);
+            bool half = false;  // the kernel's last template argument
+            for (auto &n : fake().launched)
+                half |= n.first.find("k_sweepz_zfwd") != std::string::npos && n.first.find("Lb1EEEv") != std::string::npos;
+            CHECK(half == k.half[prec]);
+        }
 }
 
 }  // namespace
@@ -445,6 +466,7 @@ int main(int argc, char **argv) {
     else if (s == "fused") fuse(true);
     else if (s == "unfused") fuse(false);
     else if (s == "rows") rows((dbec_prec)std::atoi(argv[2]), (unsigned)std::atoi(argv[3]));
+    else if (s == "tiles") tiles();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

@@ -82,3 +82,7 @@ def test_bounds_of_the_z_sweep_rows(program, prec, tile_kb):
                         ("128", {"DBEC_SWEEP_Z_TILE_KB": str(tile_kb - 1)}),
                         ("0", {"DBEC_SWEEP_Z_TILE_KB": str(tile_kb // 2 - 1)})):
         run(program, "rows", str(prec), want, **bound)
+
+
+def test_whole_and_half_tiles(program):
+    run(program, "tiles")
