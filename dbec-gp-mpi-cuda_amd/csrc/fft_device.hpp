@@ -458,6 +458,24 @@ using YPlan = PlanIf<kF32<R> ? N == 384 : N == 320, N>;
 template <int N, typename P>
 using ZPlan = std::conditional_t<N == 160 && std::is_same<P, cpx<double>>::value, FftPlanC<N>,
                                  PlanIf<N == 320 || (N == 384 && !std::is_same<P, cpx<double>>::value), N>>;
+// Lines up to which a grid keeps FftPlan in the x convolution (ky, kz) and rows
+// up to which it does in the inverse z pass (x, y), 0: none.  The other plans
+// have fewer threads a line, each with more to do, which a launch of one or two
+// workgroups a CU only waits for.  Measured (us, FftPlan / the other):
+//   x convolution  FP64: 320 8.2 / 9.3 at 1296 lines, 11.9 / 12.8 at 3104, 16.7 /
+//                  16.0 at 5184, 27.5 / 22.0 at 7840.  FP32: 320 7.5 / 8.6 at 1296,
+//                  13.9 / 14.1 at 7840, 23.1 / 20.3 at 12960; 512 8.7 / 9.6 at
+//                  1296, 10.9 / 11.1 at 3104, 19.7 / 16.0 at 6208
+//   inverse z + nu c160 FP64 9.9 / 12.2 at 2048 rows, 13.6 / 14.4 at 7680, 21.6 /
+//                  19.1 at 10240.  320 FP64: 11.8 / 12.3 and c 13.0 / 14.0 at
+//                  2560, 20.5 / 20.6 and c 24.9 / 22.5 at 7680; FP32 8.8 / 9.8 at
+//                  2560, 12.9 / 13.1 and c 15.6 / 16.4 at 7680, 23.8 / 21.1 at 15360
+// By the grid alone, not by the solves of a launch: the plans round differently.
+template <int N, typename R>
+constexpr long kXPlanLines = N == 320 ? (kF32<R> ? 8192 : 4096) : (N == 512 && kF32<R> ? 4096 : 0);
+template <int N, typename P>
+constexpr long kZPlanRows = N == 320 ? (kF32<P> ? 8192 : 4096) : (N == 160 && std::is_same<P, cpx<double>>::value ? 8192 : 0);
+
 // half the lines per workgroup in the fused inverse z pass: where whole tiles
 // leave a CU 6-8 wavefronts (complex FP64 at 512: 153 -> 140 us, 128x256x512)
 template <int N, typename P>

@@ -718,12 +718,11 @@ k_zinv(const cpx<R> *__restrict__ spec, R *__restrict__ phi, int Nx, int Ny, con
 // pairs go straight into the registers of the first transform pass
 // (load_hermitian_reg) instead of through LDS; with SWZ the transform buffer
 // is the swizzled one (lds_at).  Neither changes the results.
-template <int N, typename R, typename P, int LM, bool ZREG, bool SWZ>
-__global__ void __launch_bounds__((FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::WG))
+template <int N, typename R, typename P, int LM, bool ZREG, bool SWZ, typename Pl>
+__global__ void __launch_bounds__((FftTile<Pl, LM, kZHalf<N, P>>::WG))
 k_zinv_nu(Solves v, const double *__restrict__ sq, NuConst nc, int Nx, int Ny, int nfaceb,
           const cpx<R> *__restrict__ twg) {
-    constexpr int L = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::L, WG = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>::WG;
-    using Pl = ZPlan<N, P>;
+    constexpr int L = FftTile<Pl, LM, kZHalf<N, P>>::L, WG = FftTile<Pl, LM, kZHalf<N, P>>::WG;
     constexpr int Q = 2 * L * N / WG;  // psi elements per thread (interior rows)
     // the tile's psi (at most 256 bytes per thread) is fetched before the
     // transform, so its latency overlaps the spectrum load and the passes
@@ -946,8 +945,8 @@ struct FftLaunchImpl {
 
     template <typename R, int LM, typename Pl = XPlan<N, R>>
     static hipError_t xconv_t(const FftArgs &a) {
-        if constexpr (kF32<R> && !std::is_same<Pl, FftPlan<N>>::value)
-            if (a.phi_plans) return xconv_t<R, LM, FftPlan<N>>(a);
+        if constexpr ((kF32<R> || kXPlanLines<N, R> > 0) && !std::is_same<Pl, FftPlan<N>>::value)
+            if ((kF32<R> && a.phi_plans) || a.Nkz * a.Ny <= kXPlanLines<N, R>) return xconv_t<R, LM, FftPlan<N>>(a);
         using Tl = FftTile<Pl, LM>;
         const int ytiles = (int)((a.Ny + Tl::L - 1) / Tl::L);
         dim3 grid((unsigned)(a.Nkz * ytiles), (unsigned)a.v.nb), block(Tl::WG);
@@ -1078,9 +1077,11 @@ struct FftLaunchImpl {
         return hipGetLastError();
     }
 
-    template <typename P, typename R, int LM>
+    template <typename P, typename R, int LM, typename Pl = ZPlan<N, P>>
     static hipError_t fused_t(const FftArgs &a) {
-        using Tl = FftTile<ZPlan<N, P>, LM, kZHalf<N, P>>;
+        if constexpr (kZPlanRows<N, P> > 0 && !std::is_same<Pl, FftPlan<N>>::value)
+            if (a.Nx * a.Ny <= kZPlanRows<N, P>) return fused_t<P, R, LM, FftPlan<N>>(a);
+        using Tl = FftTile<Pl, LM, kZHalf<N, P>>;
         const auto *tw = static_cast<const cpx<R> *>(a.tw);
         const int ytiles = (int)((a.Ny + 2 * Tl::L - 1) / (2 * Tl::L));
         const int nmain = (int)((a.Nx - 1) * ytiles);
@@ -1097,13 +1098,13 @@ struct FftLaunchImpl {
         if constexpr (std::is_same<R, double>::value) {
             static const int env = fft_swz_env();
             if (env >= 0 ? env == 1 : a.tune.zinv_swz == 1) {
-                k_zinv_nu<N, R, P, LM, ZREG, true><<<grid, block, 0, a.stream>>>(a.v, a.sq, a.nc, (int)a.Nx, (int)a.Ny,
-                                                                                  nfaceb, tw);
+                k_zinv_nu<N, R, P, LM, ZREG, true, Pl><<<grid, block, 0, a.stream>>>(a.v, a.sq, a.nc, (int)a.Nx,
+                                                                                      (int)a.Ny, nfaceb, tw);
                 return hipGetLastError();
             }
         }
-        k_zinv_nu<N, R, P, LM, ZREG, false><<<grid, block, 0, a.stream>>>(a.v, a.sq, a.nc, (int)a.Nx, (int)a.Ny,
-                                                                           nfaceb, tw);
+        k_zinv_nu<N, R, P, LM, ZREG, false, Pl><<<grid, block, 0, a.stream>>>(a.v, a.sq, a.nc, (int)a.Nx, (int)a.Ny,
+                                                                               nfaceb, tw);
         return hipGetLastError();
     }
     template <int LM>
