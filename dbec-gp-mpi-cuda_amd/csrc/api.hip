@@ -1037,8 +1037,8 @@ long dbec_density_count(const dbec_ctx *c, int kind, long ox, long oy, long oz) 
 
 namespace {
 
-// Doubles of scratch that the weighted sums of an extract take; 0 for sampled
-// values of |psi|^2.
+// Doubles of scratch that the weighted sums of an extract may take beside the
+// extract itself; 0 for sampled values of |psi|^2.
 long density_sums(const dbec_ctx *c, int kind) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
     switch (kind) {
@@ -1058,38 +1058,35 @@ long density_sums(const dbec_ctx *c, int kind) {
 int density_via(dbec_ctx *c, int kind, long ox, long oy, long oz, double *out, double *d, long cap, bool plain) {
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz;
     const long sx = samples(Nx, ox), sy = samples(Ny, oy), sz = samples(Nz, oz);
-    const long sums = density_sums(c, kind), cnt = dbec_density_count(c, kind, ox, oy, oz);
+    const long cnt = dbec_density_count(c, kind, ox, oy, oz);
     const double *wx = c->b.wgt, *wy = c->b.wgt + Nx;
-    double *dst = d + sums;
+    double *dst = d;  // the extract; 1-D ones lie past the 2-D sums they come from
     hipStream_t s = c->stream;
     hipError_t e = hipSuccess;
     switch (kind) {
     case DBEC_DEN_XY:
-        e = launch_reduce3(s, c, 2, d);  // [x][y]
-        if (e == hipSuccess) e = launch_pick2(s, d, Ny, ox, oy, sx, sy, dst);
+        e = launch_reduce3(s, c, 2, ox, oy, d);
         break;
     case DBEC_DEN_X:
-        e = launch_reduce3(s, c, 2, d);
-        if (e == hipSuccess) e = launch_reduce2(s, d, Nx, Ny, 1, wy, d + Nx * Ny);
-        if (e == hipSuccess) e = launch_pick2(s, d + Nx * Ny, 1, ox, 1, sx, 1, dst);
+        e = launch_reduce3(s, c, 2, ox, 1, d);
+        dst = d + sx * Ny;
+        if (e == hipSuccess) e = launch_reduce2(s, d, sx, Ny, 1, wy, dst);
         break;
     case DBEC_DEN_Y:
-        e = launch_reduce3(s, c, 2, d);
-        if (e == hipSuccess) e = launch_reduce2(s, d, Nx, Ny, 0, wx, d + Nx * Ny);
-        if (e == hipSuccess) e = launch_pick2(s, d + Nx * Ny, 1, oy, 1, sy, 1, dst);
+        e = launch_reduce3(s, c, 2, 1, oy, d);
+        dst = d + Nx * sy;
+        if (e == hipSuccess) e = launch_reduce2(s, d, Nx, sy, 0, wx, dst);
         break;
     case DBEC_DEN_XZ:
-        e = launch_reduce3(s, c, 1, d);  // [x][z]
-        if (e == hipSuccess) e = launch_pick2(s, d, Nz, ox, oz, sx, sz, dst);
+        e = launch_reduce3(s, c, 1, ox, oz, d);
         break;
     case DBEC_DEN_Z:
-        e = launch_reduce3(s, c, 1, d);
-        if (e == hipSuccess) e = launch_reduce2(s, d, Nx, Nz, 0, wx, d + Nx * Nz);
-        if (e == hipSuccess) e = launch_pick2(s, d + Nx * Nz, 1, oz, 1, sz, 1, dst);
+        e = launch_reduce3(s, c, 1, 1, oz, d);
+        dst = d + Nx * sz;
+        if (e == hipSuccess) e = launch_reduce2(s, d, Nx, sz, 0, wx, dst);
         break;
     case DBEC_DEN_YZ:
-        e = launch_reduce3(s, c, 0, d);  // [y][z]
-        if (e == hipSuccess) e = launch_pick2(s, d, Nz, oy, oz, sy, sz, dst);
+        e = launch_reduce3(s, c, 0, oy, oz, d);
         break;
     default: {
         long start[3] = {0, 0, 0}, step[3] = {ox, oy, oz}, n[3] = {sx, sy, sz};

@@ -7,7 +7,9 @@
 // lanes along z and 8 wavefronts per workgroup that share the summed axis.
 // One thread per output, which walked its row alone, took 55 us at 256^3
 // FP64 for the 3-D sums and 55 us more for the 2-D ones.  Sums run in a fixed
-// order, so results repeat bit for bit.
+// order, so results repeat bit for bit.  The sums form the sampled outputs
+// only, packed (a launch of their own to pick those from all cost 1.5-2 us of
+// the 27-30 that an extract takes at 16^3).
 #include <type_traits>
 
 #include "ops.hpp"
@@ -25,14 +27,16 @@ __device__ __forceinline__ double mod2_of(cpx<float> v) {
     return fma((double)v.x, (double)v.x, (double)v.y * (double)v.y);
 }
 
-// out[row] = sum_z w[z] |psi|^2, a wavefront per row
+// out[a][b] = sum_z w[z] |psi|^2 at (a ox, b oy), a wavefront per row
 template <typename P>
 __global__ void __launch_bounds__(256)
-k_sum_z(const P *__restrict__ psi, const double *__restrict__ w, double *__restrict__ out, int rows, int Nz) {
+k_sum_z(const P *__restrict__ psi, const double *__restrict__ w, double *__restrict__ out, int rows, int cb, int ox,
+        int oy, int Ny, int Nz) {
     constexpr int VE = Pk<P>::n;
     const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
     if (row >= rows) return;  // uniform in the wavefront
-    const P *r = psi + (long)row * Nz;
+    const int a = row / cb, b = row - a * cb;
+    const P *r = psi + ((long)(a * ox) * Ny + b * oy) * Nz;
     double acc = 0.0;
     for (int c = lane; c < Nz / VE; c += 64) {
         const typename Pk<P>::type v = ld_pk(r + c * VE);
@@ -43,12 +47,12 @@ k_sum_z(const P *__restrict__ psi, const double *__restrict__ w, double *__restr
     if (lane == 0) out[row] = acc;
 }
 
-// out[o][z] = sum_a w[a] |psi|^2 at o * os + a * as + z: lanes along z, the 8
-// wavefronts of a workgroup share the summed axis
+// out[o][k] = sum_a w[a] |psi|^2 at o * os + a * as + k oz (k < cz): lanes along
+// z, the 8 wavefronts of a workgroup share the summed axis
 template <typename P>
 __global__ void __launch_bounds__(512)
 k_sum_strided(const P *__restrict__ psi, const double *__restrict__ w, double *__restrict__ out, int na, long as,
-              long os, int Nz) {
+              long os, int Nz, int oz, int cz) {
     __shared__ double sh[8][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int zt = (Nz + 63) / 64, o = (int)blockIdx.x / zt, z = ((int)blockIdx.x % zt) * 64 + lane;
@@ -58,11 +62,11 @@ k_sum_strided(const P *__restrict__ psi, const double *__restrict__ w, double *_
     for (int a = wave; a < na; a += 8) acc = fma(w[a], mod2_of(p[(long)a * as]), acc);
     sh[wave][lane] = acc;
     __syncthreads();
-    if (wave == 0 && z < Nz) {
+    if (wave == 0 && z < Nz && z % oz == 0) {
         double t = 0.0;
 #pragma unroll
         for (int q = 0; q < 8; ++q) t += sh[q][lane];
-        out[(long)o * Nz + z] = t;
+        out[(long)o * cz + z / oz] = t;
     }
 }
 
@@ -105,14 +109,6 @@ k_pick_mod2(const P *__restrict__ psi, int x0, int y0, int z0, int ox, int oy, i
     dst[t] = mod2_of(psi[((long)(x0 + (int)a * ox) * Ny + y0 + (int)b * oy) * Nz + z0 + (int)k * oz]);
 }
 
-// dst[a][b] = src[(a o0) n1 + b o1], a < c0, b < c1
-__global__ void k_pick2(const double *__restrict__ src, long n1, long o0, long o1, long c1, long n,
-                        double *__restrict__ dst) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    dst[t] = src[(t / c1) * o0 * n1 + (t % c1) * o1];
-}
-
 template <typename F>
 hipError_t with_psi(const dbec_ctx *c, F &&f) {
     const bool f32 = c->prec == DBEC_MIXED;
@@ -128,17 +124,24 @@ hipError_t with_psi(const dbec_ctx *c, F &&f) {
 
 }  // namespace
 
-hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, double *out) {
+hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, long o0, long o1, double *out) {
     const double *w = c->b.wgt + (axis == 0 ? 0 : (axis == 1 ? c->Nx : c->Nx + c->Ny));
     const long Nx = c->Nx, Ny = c->Ny, Nz = c->Nz, zt = (Nz + 63) / 64;
+    const long n0 = axis == 0 ? Ny : Nx, n1 = axis == 2 ? Ny : Nz;
+    o0 = std::min(o0, n0);  // (one sample either way)
+    o1 = std::min(o1, n1);
+    const long c0 = (n0 - 1) / o0 + 1, c1 = (n1 - 1) / o1 + 1;
     return with_psi(c, [&](auto *psi) {
         using P = typename std::remove_cv<typename std::remove_pointer<decltype(psi)>::type>::type;
         if (axis == 2)
-            k_sum_z<P><<<(unsigned)((Nx * Ny + 3) / 4), 256, 0, s>>>(psi, w, out, (int)(Nx * Ny), (int)Nz);
+            k_sum_z<P><<<(unsigned)((c0 * c1 + 3) / 4), 256, 0, s>>>(psi, w, out, (int)(c0 * c1), (int)c1, (int)o0, (int)o1,
+                                                                     (int)Ny, (int)Nz);
         else if (axis == 1)  // out[x][z]
-            k_sum_strided<P><<<(unsigned)(Nx * zt), 512, 0, s>>>(psi, w, out, (int)Ny, Nz, Ny * Nz, (int)Nz);
+            k_sum_strided<P><<<(unsigned)(c0 * zt), 512, 0, s>>>(psi, w, out, (int)Ny, Nz, o0 * Ny * Nz, (int)Nz, (int)o1,
+                                                                 (int)c1);
         else  // out[y][z]
-            k_sum_strided<P><<<(unsigned)(Ny * zt), 512, 0, s>>>(psi, w, out, (int)Nx, Ny * Nz, Nz, (int)Nz);
+            k_sum_strided<P><<<(unsigned)(c0 * zt), 512, 0, s>>>(psi, w, out, (int)Nx, Ny * Nz, o0 * Nz, (int)Nz, (int)o1,
+                                                                 (int)c1);
     });
 }
 
@@ -159,13 +162,6 @@ hipError_t launch_pick_mod2(hipStream_t s, const dbec_ctx *c, const long start[3
                                                                    (unsigned)cnt[1], (unsigned)cnt[2], (unsigned)n, dst,
                                                                    (int)c->Ny, (int)c->Nz);
     });
-}
-
-hipError_t launch_pick2(hipStream_t s, const double *src, long n1, long o0, long o1, long c0, long c1, double *dst) {
-    const long n = c0 * c1;
-    if (n <= 0) return hipSuccess;
-    k_pick2<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(src, n1, o0, o1, c1, n, dst);
-    return hipGetLastError();
 }
 
 }  // namespace dbec

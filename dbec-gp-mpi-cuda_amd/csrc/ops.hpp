@@ -74,15 +74,13 @@ hipError_t launch_obs_muen(hipStream_t s, const dbec_ctx *c, bool phase);
 // device scalars, or psi[n] (entries SC_COUNT, SC_COUNT + 1), to c->h_scal
 hipError_t launch_export_scalars(hipStream_t s, const dbec_ctx *c);
 hipError_t launch_export_point(hipStream_t s, const dbec_ctx *c, long n);
-// Density extracts (density.hip): out[a][b] = sum over `axis` of w |psi|^2 (the
-// other indices in [x][y][z] order), out[a] = sum_b w[b] in[a][b] (axis 1) or
-// out[b] = sum_a w[a] in[a][b] (axis 0).
-hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, double *out);
+// Density extracts (density.hip): out[a][b] = sum over `axis` of w |psi|^2 at
+// every o0-th and o1-th of the other indices (in [x][y][z] order), out[a] =
+// sum_b w[b] in[a][b] (axis 1) or out[b] = sum_a w[a] in[a][b] (axis 0).
+hipError_t launch_reduce3(hipStream_t s, const dbec_ctx *c, int axis, long o0, long o1, double *out);
 hipError_t launch_reduce2(hipStream_t s, const double *in, long n0, long n1, int axis, const double *w, double *out);
 // dst[a][b][k] = |psi|^2 at (start + (a, b, k) * step), (a, b, k) < cnt
 hipError_t launch_pick_mod2(hipStream_t s, const dbec_ctx *c, const long start[3], const long step[3],
                             const long cnt[3], double *dst);
-// dst[a][b] = src[(a o0) n1 + b o1], a < c0, b < c1
-hipError_t launch_pick2(hipStream_t s, const double *src, long n1, long o0, long o1, long c0, long c1, double *dst);
 
 }  // namespace dbec
