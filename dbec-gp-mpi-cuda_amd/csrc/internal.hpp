@@ -83,6 +83,7 @@ struct dbec_ctx {
     double *h_scal = nullptr;    // pinned host copy of the scalars (SC_COUNT + 2), null in request-loop contexts
     bool planes = false;         // the plane kernels carry the step (plane_ok at creation)
     bool phi_valid = false;
+    size_t spec_bytes = 0;       // of b.spec (not in request-loop slots)
     dbec::Buffers b;
     dbec::Tuning tune;
     dbec::KernelTimer *timer = nullptr;  // set while dbec_profile_step records

@@ -34,6 +34,7 @@ std::atomic<int> thread_delay_us{0};
 std::atomic<int> pinned_live{0}, freed_in_flight{0};
 std::atomic<int> allocs{0};  // host and device memory, events
 std::atomic<int> staged_copies[16];
+std::atomic<int> copies{0};
 
 struct Enter {
     Enter() { ++in_fake; }
@@ -215,6 +216,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, h
     std::lock_guard<std::mutex> lk(fake().mu);
     auto *s = reinterpret_cast<Stream *>(h);
     const bool to = is_pinned(dst), from = is_pinned(src);
+    ++copies;
     if (to || from) ++staged_copies[s->device];
     if (to) ++pending_fetches;
     s->ops.push_back({dst, src, n});
@@ -452,6 +454,19 @@ void tiles() {
         }
 }
 
+// The 3-D extract of a small grid is one launch and one copy in either precision.
+void one_slab() {
+    for (dbec_prec prec : {DBEC_FP64, DBEC_MIXED})
+        for (long n : {16L, 64L}) {
+            dbec_ctx *c = create(n, n, n, DBEC_IMAG, prec);
+            std::vector<double> out((size_t)(n * n * n));
+            const int before = copies;
+            CHECK(dbec_density(c, DBEC_DEN_XYZ, 1, 1, 1, out.data()) == DBEC_OK);
+            CHECK(copies == before + 1);
+            CHECK(dbec_destroy(c) == DBEC_OK);
+        }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -467,6 +482,7 @@ int main(int argc, char **argv) {
     else if (s == "unfused") fuse(false);
     else if (s == "rows") rows((dbec_prec)std::atoi(argv[2]), (unsigned)std::atoi(argv[3]));
     else if (s == "tiles") tiles();
+    else if (s == "one_slab") one_slab();
     else return std::printf("no such scenario\n"), 2;
     std::printf("ok\n");
     return 0;

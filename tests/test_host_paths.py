@@ -86,3 +86,7 @@ def test_bounds_of_the_z_sweep_rows(program, prec, tile_kb):
 
 def test_whole_and_half_tiles(program):
     run(program, "tiles")
+
+
+def test_small_densities_in_one_slab(program):
+    run(program, "one_slab")
