@@ -469,12 +469,13 @@ using ZPlan = std::conditional_t<N == 160 && std::is_same<P, cpx<double>>::value
 //   inverse z + nu c160 FP64 9.9 / 12.2 at 2048 rows, 13.6 / 14.4 at 7680, 21.6 /
 //                  19.1 at 10240.  320 FP64: 11.8 / 12.3 and c 13.0 / 14.0 at
 //                  2560, 20.5 / 20.6 and c 24.9 / 22.5 at 7680; FP32 8.8 / 9.8 at
-//                  2560, 12.9 / 13.1 and c 15.6 / 16.4 at 7680, 23.8 / 21.1 at 15360
+//                  2560, 12.9 / 13.1 and c 15.6 / 16.4 at 7680, 16.1 / 17.1 at
+//                  10240, 23.8 / 21.1 and c 25.8 / 22.6 at 15360
 // By the grid alone, not by the solves of a launch: the plans round differently.
 template <int N, typename R>
 constexpr long kXPlanLines = N == 320 ? (kF32<R> ? 8192 : 4096) : (N == 512 && kF32<R> ? 4096 : 0);
 template <int N, typename P>
-constexpr long kZPlanRows = N == 320 ? (kF32<P> ? 8192 : 4096) : (N == 160 && std::is_same<P, cpx<double>>::value ? 8192 : 0);
+constexpr long kZPlanRows = N == 320 ? (kF32<P> ? 12288 : 4096) : (N == 160 && std::is_same<P, cpx<double>>::value ? 8192 : 0);
 
 // half the lines per workgroup in the fused inverse z pass: where whole tiles
 // leave a CU 6-8 wavefronts (complex FP64 at 512: 153 -> 140 us, 128x256x512)

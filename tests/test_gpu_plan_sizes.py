@@ -12,9 +12,9 @@ from test_gpu_plane import field
 pytestmark = pytest.mark.gpu
 
 # x convolution: Ny (Nz/2 + 1) lines, 320 at 4096 (FP64) and 8192 (FP32), 512 at
-# 4096 (FP32); inverse z: Nx Ny rows, 320 at 4096 and 8192, complex 160 at 8192 (FP64)
+# 4096 (FP32); inverse z: Nx Ny rows, 320 at 4096 and 12288, complex 160 at 8192 (FP64)
 GRIDS = [(320, 16, 160), (320, 64, 160), (320, 128, 160), (512, 16, 160), (512, 48, 192),
-         (16, 160, 160), (64, 160, 160), (16, 160, 320), (32, 160, 320), (64, 160, 320)]
+         (16, 160, 160), (64, 160, 160), (16, 160, 320), (32, 160, 320), (80, 160, 320)]
 
 
 @pytest.mark.parametrize("n", GRIDS, ids=lambda n: "x".join(map(str, n)))
