@@ -224,11 +224,13 @@ FftArgs xconv_args(const dbec_ctx *c, const Solves &v, bool planes, bool phi = f
     FftArgs a = fft_args(c, 0, v);
     a.yq = planes ? (int)(c->Ny / 8) : 0;
     a.phi_plans = phi;
+    if (phi && c->prec == DBEC_MIXED) a.tune.lm[2] = c->tune.lm_phi[1];
     return a;
 }
 FftArgs phi_yargs(const dbec_ctx *c, const Solves &v) {
     FftArgs a = fft_args(c, 1, v);
     a.phi_plans = true;
+    if (c->prec == DBEC_MIXED) a.tune.lm[1] = c->tune.lm_phi[0];
     return a;
 }
 
@@ -712,10 +714,11 @@ void describe_tuning(const dbec_ctx *c, char *buf, size_t len) {
     const Tuning &t = c->tune;
     std::snprintf(buf, len,
                   "%ldx%ldx%ld %s %s: lm zfwd %d ypass %d xconv %d fused %d; sweep x rowb %d peel %d, "
-                  "y rowb %d peel %d, z direct %d; fused layout %d (0 / -1 = built-in rule)",
+                  "y rowb %d peel %d, z direct %d; fused layout %d; potential ypass %d xconv %d "
+                  "(0 / -1 = built-in rule)",
                   c->Nx, c->Ny, c->Nz, c->mode == DBEC_IMAG ? "imag" : "real",
                   c->prec == DBEC_MIXED ? "mixed" : "fp64", t.lm[0], t.lm[1], t.lm[2], t.lm[3], t.xy_rowb[0],
-                  t.xy_peel[0], t.xy_rowb[1], t.xy_peel[1], t.z_direct, t.zinv_swz);
+                  t.xy_peel[0], t.xy_rowb[1], t.xy_peel[1], t.z_direct, t.zinv_swz, t.lm_phi[0], t.lm_phi[1]);
 }
 
 int autotune(dbec_ctx *c) {
@@ -740,11 +743,13 @@ int autotune(dbec_ctx *c) {
     };
     Tuning &t = c->tune;
     const bool planes = c->planes;  // the plane kernels take the z and y passes' place
-    if (!phi_planes(c)) {
-        CHK(choose(&t.lm[0], {0, 1, 2}, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }));
-        CHK(choose(&t.lm[1], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }));
-    }
+    if (!phi_planes(c)) CHK(choose(&t.lm[0], {0, 1, 2}, [&] { return launch_zfwd(c->Nz, fft_args(c, 2, v)); }));
+    if (!planes) CHK(choose(&t.lm[1], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, fft_args(c, 1, v)); }));
     CHK(choose(&t.lm[2], {0, 1, 2}, [&] { return launch_xconv(c->Nx, xconv_args(c, v, planes)); }));
+    if (c->prec == DBEC_MIXED) {
+        CHK(choose(&t.lm_phi[0], {0, 1, 2}, [&] { return launch_ypass(c->Ny, -1, phi_yargs(c, v)); }));
+        CHK(choose(&t.lm_phi[1], {0, 1, 2}, [&] { return launch_xconv(c->Nx, xconv_args(c, v, false, true)); }));
+    }
     if (planes) {
         // no fused inverse z pass
     } else if (c->prec != DBEC_MIXED) {
@@ -769,7 +774,7 @@ int autotune(dbec_ctx *c) {
     CHK(choose(&t.z_direct, {-1, 0, 1}, [&] { return launch_sweep(c->stream, c, 2, v, c->mode == DBEC_IMAG); }));
     // the candidates ran on zero data; psi and the spectrum stay zero
     if (const char *lg = getenv("DBEC_AUTOTUNE_LOG"); lg && std::strcmp(lg, "0") != 0) {
-        char buf[256];
+        char buf[512];
         describe_tuning(c, buf, sizeof buf);
         std::fprintf(stderr, "[dbec autotune] %s\n", buf);
     }

@@ -54,6 +54,8 @@ enum { SC_NORM = 0, SC_SCALE = 1, SC_ONE = 2, SC_MU = 3, SC_EN = 4, SC_R0 = 5, S
 // per context by timing (autotune at creation); 0 / -1: the built-in rule.
 struct Tuning {
     int lm[4] = {0, 0, 0, 0};   // FFT tile multiplier (1, 2): zfwd, ypass, xconv, fused inverse z
+    int lm_phi[2] = {0, 0};     // the same of the mixed form's standalone potential, where the step runs
+                                // other kernels (plans, planes): ypass, xconv
     int xy_rowb[2] = {0, 0};    // x / y sweeps: bytes of z per row load (128, 256)
     int xy_peel[2] = {-1, -1};  // x / y sweeps: boundary iterations peeled (1) or tested (0)
     int z_direct = -1;          // z sweep: segments loaded straight from HBM (1) or staged through LDS (0)

@@ -90,3 +90,7 @@ def test_whole_and_half_tiles(program):
 
 def test_small_densities_in_one_slab(program):
     run(program, "one_slab")
+
+
+def test_tuner_times_the_kernels_that_run(program):
+    run(program, "tuned", DBEC_AUTOTUNE="1")
