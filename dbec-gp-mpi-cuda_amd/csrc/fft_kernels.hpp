@@ -341,30 +341,30 @@ k_sweepz_zfwd(Solves v, int Nx, int Ny, SweepTab<typename Arith<S>::T> tab, Swee
             }
         } else {
 #pragma unroll
-        for (int h = 0; h < NH; ++h) {
-            if (h) __syncthreads();  // the last pass's rows are in registers
+            for (int h = 0; h < NH; ++h) {
+                if (h) __syncthreads();  // the last pass's rows are in registers
 #pragma unroll
-            for (int q = h * (KV / NH); q < (h + 1) * (KV / NH); ++q) {
-                const int iv = tid + q * WG;
-                if (iv < npk) {
-                    const int e = (iv * VE) % N, row = (iv * VE) / N;
-                    st_pk(tile + at(row - h * LH, e), r[q]);
+                for (int q = h * (KV / NH); q < (h + 1) * (KV / NH); ++q) {
+                    const int iv = tid + q * WG;
+                    if (iv < npk) {
+                        const int e = (iv * VE) % N, row = (iv * VE) / N;
+                        st_pk(tile + at(row - h * LH, e), r[q]);
+                    }
+                }
+                __syncthreads();
+                if (hh == h) {
+                    const int row = l - h * LH;
+                    hl = hr = zero;
+#pragma unroll
+                    for (int m = 0; m < KV; ++m) {
+                        const typename Pk<S>::type pk = ld_pk(tile + at(row, e0 + m * VE));
+#pragma unroll
+                        for (int j = 0; j < VE; ++j) vv[m * VE + j] = act ? to_a(pk.e[j]) : zero;
+                    }
+                    if (act && e0 > 0) hl = to_a(tile[at(row, e0 - 1)]);
+                    if (act && e0 + M < N) hr = to_a(tile[at(row, e0 + M)]);
                 }
             }
-            __syncthreads();
-            if (NH == 1 || hh == h) {
-                const int row = l - h * LH;
-                hl = hr = zero;
-#pragma unroll
-                for (int m = 0; m < KV; ++m) {
-                    const typename Pk<S>::type pk = ld_pk(tile + at(row, e0 + m * VE));
-#pragma unroll
-                    for (int j = 0; j < VE; ++j) vv[m * VE + j] = act ? to_a(pk.e[j]) : zero;
-                }
-                if (act && e0 > 0) hl = to_a(tile[at(row, e0 - 1)]);
-                if (act && e0 + M < N) hr = to_a(tile[at(row, e0 + M)]);
-            }
-        }
         }
     }
     if constexpr (NH == 1) {

@@ -53,7 +53,7 @@ __device__ __forceinline__ double plane_mod2(cpx<double> v, double) { return fma
 __device__ __forceinline__ double plane_mod2(cpx<float> v, double) { return v.x * v.x + v.y * v.y; }
 
 struct PlaneDims {
-    int Nx, Ny, Nz, Nkz, qy, qz, nt;
+    int Nx, Ny, Nz, qy, qz, nt;
     FastDiv dNy, dNyh, dNz, dNzh, dqy;
     // inverse kernel: workgroups per plane, their share of the rows (qy / parts
     // butterflies), and as divisors
@@ -564,7 +564,6 @@ PlaneDims dims(const dbec_ctx *c, int parts, int extra = 0) {
     g.Nx = (int)c->Nx;
     g.Ny = (int)c->Ny;
     g.Nz = (int)c->Nz;
-    g.Nkz = (int)c->Nkz;
     g.qy = g.Ny / 8;
     g.qz = g.Nz / 8;
     g.nt = g.Ny * g.Nz / 16;

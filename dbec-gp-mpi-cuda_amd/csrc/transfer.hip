@@ -183,7 +183,6 @@ public:
         cv_.notify_all();
         for (auto &t : th) t.join();
     }
-    ~Workers() { stop(); }
 
 private:
     // born: generation_ when the thread was made.  It may get the lock for the
